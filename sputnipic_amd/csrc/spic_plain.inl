@@ -63,6 +63,12 @@ __device__ __forceinline__ bool clamp_index(int &ix, int n) {
 // One particle's predictor-corrector push and particle BC
 // (src/Mover.cpp:33-157).  Returns true if an iterate left the grid by
 // more than one cell.
+// The gathers bound it: 48 field values per particle from L2, a cache line
+// per lane and load once the particles have mixed.  They stay in registers
+// while the iterate stays in its cell (nine in ten do), so most particles
+// gather once instead of once per iteration: 5.97M FP64 particles of a mixed
+// order in 1.70 ms against 3.62, three waves per SIMD in FP64 (168 VGPRs,
+// the limit; unlimited it takes 176 and two).
 template <typename T>
 __device__ __forceinline__ bool push_particle_once(const KGrid<T> &g,
                                               const KField<T> &f,
@@ -74,6 +80,10 @@ __device__ __forceinline__ bool push_particle_once(const KGrid<T> &g,
   T upt = T(0), vpt = T(0), wpt = T(0);
   T xc = x, yc = y, zc = z;
   bool bad = false;
+  // the stencil of the last cell: nodes ix - a, iy - b, iz - c
+  int cix = -1, ciy = -1, ciz = -1;
+  T F[2][2][2][6];
+  T X0 = T(0), X1 = T(0), Y0 = T(0), Y1 = T(0), Z0 = T(0), Z1 = T(0);
   for (int it = 0; it < k.niter; ++it) {
     int ix = cell_trunc<T>(xc, g.xStart, g.invdx, g.nxn);
     int iy = cell_trunc<T>(yc, g.yStart, g.invdy, g.nyn);
@@ -81,10 +91,26 @@ __device__ __forceinline__ bool push_particle_once(const KGrid<T> &g,
     bad |= clamp_index(ix, g.nxn);
     bad |= clamp_index(iy, g.nyn);
     bad |= clamp_index(iz, g.nzn);
-    const T xi[2] = {xc - g.xn[ix - 1], g.xn[ix] - xc};
-    const T eta[2] = {yc - g.yn[iy - 1], g.yn[iy] - yc};
-    const T zeta[2] = {zc - g.zn[iz - 1], g.zn[iz] - zc};
-    const int base = (ix * nyn + iy) * nzn + iz;
+    if (ix != cix || iy != ciy || iz != ciz) {
+      cix = ix; ciy = iy; ciz = iz;
+      X0 = g.xn[ix - 1]; X1 = g.xn[ix];
+      Y0 = g.yn[iy - 1]; Y1 = g.yn[iy];
+      Z0 = g.zn[iz - 1]; Z1 = g.zn[iz];
+      const int base = (ix * nyn + iy) * nzn + iz;
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const int n = base - a * sx - b * sy - c;
+            F[a][b][c][0] = f.Ex[n]; F[a][b][c][1] = f.Ey[n]; F[a][b][c][2] = f.Ez[n];
+            F[a][b][c][3] = f.Bx[n]; F[a][b][c][4] = f.By[n]; F[a][b][c][5] = f.Bz[n];
+          }
+    }
+    const T xi[2] = {xc - X0, X1 - xc};
+    const T eta[2] = {yc - Y0, Y1 - yc};
+    const T zeta[2] = {zc - Z0, Z1 - zc};
     T Exl = T(0), Eyl = T(0), Ezl = T(0), Bxl = T(0), Byl = T(0), Bzl = T(0);
 #pragma unroll
     for (int a = 0; a < 2; ++a)
@@ -93,13 +119,12 @@ __device__ __forceinline__ bool push_particle_once(const KGrid<T> &g,
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           const T wgt = xi[a] * eta[b] * zeta[c] * g.invVOL;
-          const int n = base - a * sx - b * sy - c;
-          Exl += wgt * f.Ex[n];
-          Eyl += wgt * f.Ey[n];
-          Ezl += wgt * f.Ez[n];
-          Bxl += wgt * f.Bx[n];
-          Byl += wgt * f.By[n];
-          Bzl += wgt * f.Bz[n];
+          Exl += wgt * F[a][b][c][0];
+          Eyl += wgt * F[a][b][c][1];
+          Ezl += wgt * F[a][b][c][2];
+          Bxl += wgt * F[a][b][c][3];
+          Byl += wgt * F[a][b][c][4];
+          Bzl += wgt * F[a][b][c][5];
         }
     const T q2 = k.qomdt2;
     const T omdtsq = q2 * q2 * (Bxl * Bxl + Byl * Byl + Bzl * Bzl);
@@ -222,7 +247,9 @@ __device__ __forceinline__ bool deposit_particle(const KGrid<T> &g,
 constexpr int kBlock = 256;
 
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_mover(KGrid<T> g, KField<T> f,
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 4)))
+void k_mover(KGrid<T> g, KField<T> f,
                                                   KPart<T> p, KPush<T> k,
                                                   unsigned int *status) {
   bool bad = false;
@@ -249,7 +276,9 @@ __global__ __launch_bounds__(kBlock) void k_deposit(KGrid<T> g, KPart<T> p,
 }
 
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_mover_deposit(
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 4)))
+void k_mover_deposit(
     KGrid<T> g, KField<T> f, KPart<T> p, KPush<T> k, KMom m,
     unsigned int *status) {
   bool bad = false, bad_dep = false;
