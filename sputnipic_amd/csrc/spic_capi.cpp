@@ -120,6 +120,47 @@ hipError_t workspace(size_t bytes, void **out) {
 }  // namespace
 
 namespace spic {
+namespace {
+// One memory pool per device, made at its first use.
+struct ScratchPool {
+  int device;
+  hipMemPool_t pool;
+};
+std::mutex g_pool_mutex;
+std::vector<ScratchPool> g_pools;
+}  // namespace
+
+hipError_t stream_alloc(void **p, size_t bytes, hipStream_t s) {
+  *p = nullptr;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  hipMemPool_t pool = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_pool_mutex);
+    for (const auto &sp : g_pools)
+      if (sp.device == dev) pool = sp.pool;
+    if (!pool) {
+      hipMemPoolProps props;
+      std::memset(&props, 0, sizeof(props));
+      props.allocType = hipMemAllocationTypePinned;
+      props.location.type = hipMemLocationTypeDevice;
+      props.location.id = dev;
+      if ((e = hipMemPoolCreate(&pool, &props)) != hipSuccess) return e;
+      uint64_t keep = kScratchKeep;
+      if ((e = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep)) !=
+          hipSuccess) {
+        (void)hipMemPoolDestroy(pool);
+        return e;
+      }
+      g_pools.push_back(ScratchPool{dev, pool});
+    }
+  }
+  return hipMallocFromPoolAsync(p, bytes ? bytes : 1, pool, s);
+}
+
+hipError_t stream_free(void *p, hipStream_t s) { return hipFreeAsync(p, s); }
+
 int check_grid(const spic_grid *g) {
   if (!g) return fail(SPIC_EINVAL, "grid is NULL");
   if (g->prec != SPIC_F64 && g->prec != SPIC_F32)

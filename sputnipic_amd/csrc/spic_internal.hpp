@@ -78,6 +78,14 @@ hipError_t sort_reference_order(const spic_grid &g, int64_t sort_cps,
                                 size_t workspace_bytes, size_t *needed,
                                 hipStream_t s);
 
+// Scratch memory of one call, ordered on its stream: from a pool of the
+// current device that keeps at most kScratchKeep bytes between calls and
+// returns the rest (safe for any number of threads and streams).  Not for a
+// stream under capture.
+constexpr size_t kScratchKeep = size_t(512) << 20;
+hipError_t stream_alloc(void **p, size_t bytes, hipStream_t s);
+hipError_t stream_free(void *p, hipStream_t s);
+
 hipError_t zero_f64(double *p, size_t n, hipStream_t s);
 hipError_t zero_u32(unsigned int *p, size_t n, hipStream_t s);
 

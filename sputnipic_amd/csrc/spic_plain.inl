@@ -301,6 +301,417 @@ static inline unsigned grid_for(int n) {
   return (unsigned)blocks;
 }
 
+// ---- deposit through tiles -------------------------------------------------
+//
+// 80 global FP64 atomics per particle bound the direct deposit: 0.4 G
+// particles/s, 14.4 ms for 5.97M FP64 particles in bin order.  Here the
+// particles of a species are first counted into tiles of 4x4x4 cells (each
+// gets its rank in its tile), their indices are placed tile by tile, and one
+// workgroup per run of a tile's particles gathers them, sums their moments
+// per cell in registers and adds 5x5x5 nodes to the arrays: about 1250 atomics
+// per run instead of 80 per particle.  The particles themselves do not move.
+// Tiles cover the deposit cells ix - 1 = 0 .. nxn - 2, guard cells included.
+constexpr int kDepMinParticles = 12288, kDepMinPerTile = 4;
+constexpr int kDepTile = 4;
+constexpr int kDepCells = kDepTile * kDepTile * kDepTile;
+constexpr int kDepBatch = 512;         // particles staged in LDS at a time
+constexpr int kDepMaxRun = 4096;       // particles per workgroup at most
+constexpr int kDepSlice = 1 << 24;     // particles binned at a time (24-bit indices)
+constexpr uint32_t kDepIndexMask = (1u << 24) - 1u;
+constexpr int kDepLdsTiles = 6144;     // tile counters a workgroup keeps in LDS
+
+struct DepBins {
+  int nty, ntz, ntiles;
+  int run;                // particles per work item
+  int per;                // particles per thread of the count
+  int in_lds;             // the tiles' counters fit in LDS (kDepLdsTiles)
+  unsigned int *cnt;      // [ntiles + 2]: particles per tile, total, items
+  unsigned int *next;     // [ntiles]: next free place of each tile
+  uint4 *items;           // tile, first place, particles
+  unsigned int *where;    // [n]: cell in the tile | tile << 6
+  unsigned int *perm;     // [n] by place: index | cell in the tile << 24
+};
+
+// Tile and cell within the tile of a (clamped) deposit cell.
+__device__ __forceinline__ void dep_tile(const DepBins &b, int ix, int iy, int iz,
+                                         unsigned int &tile, unsigned int &cell) {
+  const int cx = ix - 1, cy = iy - 1, cz = iz - 1;
+  tile = ((cx / kDepTile) * b.nty + cy / kDepTile) * b.ntz + cz / kDepTile;
+  cell = ((cx % kDepTile) * kDepTile + cy % kDepTile) * kDepTile + cz % kDepTile;
+}
+
+// Adds this lane's particle to its tile's counter and returns its rank there.
+// Lanes of one wave that share a tile take one atomic together (particles of
+// a run are near each other in most orders); after four distinct tiles the
+// remaining lanes take one each.
+__device__ __forceinline__ unsigned int dep_rank(unsigned int *cnt, unsigned int tile,
+                                                 bool active) {
+  const int lane = threadIdx.x & 63;
+  unsigned long long todo = __ballot(active);
+  int leader = lane;
+  unsigned int off = 0, group = 1;
+  for (int round = 0; round < 4 && todo; ++round) {
+    const int first = __ffsll((long long)todo) - 1;
+    const unsigned int t0 = (unsigned int)__builtin_amdgcn_readlane((int)tile, first);
+    const bool mine = ((todo >> lane) & 1ull) && tile == t0;
+    const unsigned long long same = __ballot(mine);
+    if (mine) {
+      leader = first;
+      off = (unsigned int)__popcll(same & ((1ull << lane) - 1ull));
+      group = (unsigned int)__popcll(same);
+    }
+    todo &= ~same;
+  }
+  unsigned int r = 0;
+  if (active && lane == leader) r = atomicAdd(cnt + tile, group);
+  return (unsigned int)__shfl((int)r, leader) + off;
+}
+
+template <typename T>
+__device__ __forceinline__ bool dep_cell(const KGrid<T> &g, T x, T y, T z, int &ix, int &iy,
+                                         int &iz) {
+  ix = cell_floor<T>(x, g.xStart, g.invdx, g.nxn);
+  iy = cell_floor<T>(y, g.yStart, g.invdy, g.nyn);
+  iz = cell_floor<T>(z, g.zStart, g.invdz, g.nzn);
+  bool bad = clamp_index(ix, g.nxn);
+  bad |= clamp_index(iy, g.nyn);
+  bad |= clamp_index(iz, g.nzn);
+  return bad;
+}
+
+// Counts the particles into tiles; with PUSH, pushes them first.  Up to
+// kDepLdsTiles tiles a workgroup counts its particles in LDS and adds each
+// tile it met once: with counters in global memory alone, a million
+// particles in random order on 45 tiles took 1.3 ms in contended atomics.
+template <typename T, bool PUSH>
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && PUSH ? 3 : 4)))
+void k_dep_count(KGrid<T> g, KField<T> f, KPart<T> p, KPush<T> k, DepBins b,
+                 unsigned int *status) {
+  __shared__ unsigned int s_cnt[kDepLdsTiles];
+  const int tid = threadIdx.x;
+  if (b.in_lds) {
+    for (int t = tid; t < b.ntiles; t += kBlock) s_cnt[t] = 0u;
+    __syncthreads();
+  }
+  const int first = blockIdx.x * kBlock * b.per;
+  bool bad = false, bad_dep = false;
+  for (int e = 0; e < b.per; ++e) {
+    const int i = first + e * kBlock + tid;
+    const bool active = i < p.n;
+    unsigned int tile = 0, cell = 0;
+    if (active) {
+      T x = p.x[i], y = p.y[i], z = p.z[i];
+      if constexpr (PUSH) {
+        T u = p.u[i], v = p.v[i], w = p.w[i];
+        bad |= push_particle<T>(g, f, k, x, y, z, u, v, w);
+        p.x[i] = x; p.y[i] = y; p.z[i] = z;
+        p.u[i] = u; p.v[i] = v; p.w[i] = w;
+      }
+      int ix, iy, iz;
+      bad_dep |= dep_cell<T>(g, x, y, z, ix, iy, iz);
+      dep_tile(b, ix, iy, iz, tile, cell);
+      b.where[i] = cell | (tile << 6);
+    }
+    if (b.in_lds) dep_rank(s_cnt, tile, active);
+    else dep_rank(b.cnt, tile, active);
+  }
+  if (bad) atomicAdd(status, 1u);
+  if (bad_dep) atomicAdd(status + 1, 1u);
+  if (b.in_lds) {
+    __syncthreads();
+    for (int t = tid; t < b.ntiles; t += kBlock)
+      if (s_cnt[t]) atomicAdd(b.cnt + t, s_cnt[t]);
+  }
+}
+
+// Places of the tiles (in no particular order) and their work items.
+static __global__ __launch_bounds__(kBlock) void k_dep_bounds(DepBins b) {
+  const int t = blockIdx.x * kBlock + threadIdx.x, lane = threadIdx.x & 63;
+  const unsigned int c = t < b.ntiles ? b.cnt[t] : 0u;
+  const unsigned int ni = (c + b.run - 1) / b.run;
+  unsigned int sc = c, si = ni;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned int vc = __shfl_up(sc, d), vi = __shfl_up(si, d);
+    if (lane >= d) { sc += vc; si += vi; }
+  }
+  unsigned int bc = 0, bi = 0;
+  if (lane == 63 && sc) {
+    bc = atomicAdd(b.cnt + b.ntiles, sc);
+    bi = atomicAdd(b.cnt + b.ntiles + 1, si);
+  }
+  const unsigned int first = __shfl(bc, 63) + sc - c, item = __shfl(bi, 63) + si - ni;
+  if (c) b.next[t] = first;
+  for (unsigned int j = 0; j < ni; ++j)
+    b.items[item + j] = make_uint4((unsigned int)t, first + j * b.run,
+                                   min((unsigned int)b.run, c - j * b.run), 0u);
+}
+
+// Places each particle's index in its tile, the places taken as the count
+// took its counters: each tile's places at once per workgroup (IN_LDS), PER
+// particles per thread, or per wave.
+template <int PER, bool IN_LDS>
+static __global__ __launch_bounds__(kBlock) void k_dep_place(DepBins b, int n) {
+  __shared__ unsigned int s_cnt[IN_LDS ? kDepLdsTiles : 1];
+  const int tid = threadIdx.x;
+  const int first = blockIdx.x * kBlock * PER;
+  unsigned int w[PER], r[PER];
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    const int i = first + e * kBlock + tid;
+    w[e] = i < n ? b.where[i] : 0u;
+  }
+  if constexpr (IN_LDS) {
+    for (int t = tid; t < b.ntiles; t += kBlock) s_cnt[t] = 0u;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int e = 0; e < PER; ++e)
+    r[e] = dep_rank(IN_LDS ? s_cnt : b.next, w[e] >> 6, first + e * kBlock + tid < n);
+  if constexpr (IN_LDS) {
+    __syncthreads();
+    for (int t = tid; t < b.ntiles; t += kBlock)
+      if (s_cnt[t]) s_cnt[t] = atomicAdd(b.next + t, s_cnt[t]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    const int i = first + e * kBlock + tid;
+    if (i < n)
+      b.perm[(IN_LDS ? s_cnt[w[e] >> 6] : 0u) + r[e]] = (unsigned int)i | ((w[e] & 63u) << 24);
+  }
+}
+
+// One work item per workgroup: batches of kDepBatch particles are gathered
+// into LDS sorted by cell (a count, a wave scan and a placement; every
+// batch's particles fit, unlike fixed buckets), then the four threads of a
+// cell, two of its eight nodes each, sum them in FP64 registers that live
+// until the item's end.  39 KB of LDS and 126 VGPRs in FP64: four workgroups
+// per CU cover each other's gathers.  5.97M FP64 particles in bin order: 231 us
+// (64 B each, 1.65 TB/s); loading the next batch ahead needs 140 VGPRs, three
+// workgroups, and takes 250 us.
+template <typename T>
+__global__ __launch_bounds__(4 * kDepCells)
+__attribute__((amdgpu_waves_per_eu(4)))
+void k_tile_deposit(KGrid<T> g, KPart<T> p, KMom m,
+                                                                 DepBins b) {
+  constexpr int NT = 4 * kDepCells, PER = kDepBatch / NT, NB = kDepTile + 1;
+  // strict arithmetic, and FP32 particles as the direct kernel adds them:
+  // every term rounded in T before it is added in FP64
+  constexpr bool kTerms = kStrict || sizeof(T) == 4;
+  __shared__ T s_p[7][kDepBatch];
+  __shared__ double s_mom[10][NB * NB * NB];
+  __shared__ unsigned int s_cnt[kDepCells], s_off[kDepCells + 1];
+  if (blockIdx.x >= b.cnt[b.ntiles + 1]) return;
+  const uint4 item = b.items[blockIdx.x];
+  const int tid = threadIdx.x;
+  const int c0z = (int)(item.x % b.ntz) * kDepTile;
+  const int c0y = (int)((item.x / b.ntz) % b.nty) * kDepTile;
+  const int c0x = (int)(item.x / (b.ntz * b.nty)) * kDepTile;
+  for (int i = tid; i < 10 * NB * NB * NB; i += NT) (&s_mom[0][0])[i] = 0.0;
+  if (tid < kDepCells) s_cnt[tid] = 0u;
+  // this thread's cell and its node pair, corners (a, b, 0) and (a, b, 1)
+  const int my = tid >> 2, ma = (tid >> 1) & 1, mb = tid & 1;
+  const int lx = my / (kDepTile * kDepTile), ly = (my / kDepTile) % kDepTile,
+            lz = my % kDepTile;
+  // nodes of cells beyond the grid are never used; their index is bounded
+  const int nx1 = min(c0x + lx + 1, g.nxn - 1), ny1 = min(c0y + ly + 1, g.nyn - 1),
+            nz1 = min(c0z + lz + 1, g.nzn - 1);
+  const T X0 = g.xn[nx1 - 1], X1 = g.xn[nx1];
+  const T Y0 = g.yn[ny1 - 1], Y1 = g.yn[ny1];
+  const T Z0 = g.zn[nz1 - 1], Z1 = g.zn[nz1];
+  const T iv = g.invVOL;
+  double acc[20];
+#pragma unroll
+  for (int j = 0; j < 20; ++j) acc[j] = 0.0;
+  __syncthreads();
+  for (unsigned int o = 0; o < item.z; o += kDepBatch) {
+    T val[PER][7];
+    unsigned int cell[PER], rank[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const unsigned int j = o + e * NT + tid;
+      cell[e] = kDepCells;
+      if (j < item.z) {
+        const unsigned int w = b.perm[item.y + j];
+        const unsigned int i = w & kDepIndexMask;
+        cell[e] = w >> 24;
+        val[e][0] = p.x[i]; val[e][1] = p.y[i]; val[e][2] = p.z[i];
+        val[e][3] = p.q[i];
+        val[e][4] = p.u[i]; val[e][5] = p.v[i]; val[e][6] = p.w[i];
+        rank[e] = atomicAdd(&s_cnt[cell[e]], 1u);
+      }
+    }
+    __syncthreads();
+    if (tid < 64) {
+      const unsigned int c = s_cnt[tid];
+      unsigned int sum = c;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const unsigned int v = __shfl_up(sum, d);
+        if (tid >= d) sum += v;
+      }
+      s_off[tid] = sum - c;
+      if (tid == 63) s_off[64] = sum;
+      s_cnt[tid] = 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < PER; ++e)
+      if (cell[e] < (unsigned int)kDepCells) {
+        const unsigned int at = s_off[cell[e]] + rank[e];
+#pragma unroll
+        for (int c = 0; c < 7; ++c) s_p[c][at] = val[e][c];
+      }
+    __syncthreads();
+    const unsigned int end = s_off[my + 1];
+    for (unsigned int j = s_off[my]; j < end; ++j) {
+      const T x = s_p[0][j], y = s_p[1][j], z = s_p[2][j], q = s_p[3][j];
+      const T u = s_p[4][j], v = s_p[5][j], w = s_p[6][j];
+      const T xi = ma ? X1 - x : x - X0, eta = mb ? Y1 - y : y - Y0;
+      if constexpr (kTerms) {
+        // the reference's terms, each rounded in T (src/Mover.cpp:430-568)
+        const T wg[2] = {q * xi * eta * (z - Z0) * iv, q * xi * eta * (Z1 - z) * iv};
+        const T uu = u * u, uv = u * v, uw = u * w, vv = v * v, vw = v * w, ww = w * w;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          double *a = acc + 10 * c;
+          const T wgt = wg[c];
+          a[0] += (double)(wgt * iv);
+          a[1] += (double)((u * wgt) * iv);
+          a[2] += (double)((v * wgt) * iv);
+          a[3] += (double)((w * wgt) * iv);
+          a[4] += (double)((uu * wgt) * iv);
+          a[5] += (double)((uv * wgt) * iv);
+          a[6] += (double)((uw * wgt) * iv);
+          a[7] += (double)((vv * wgt) * iv);
+          a[8] += (double)((vw * wgt) * iv);
+          a[9] += (double)((ww * wgt) * iv);
+        }
+      } else {
+        // sums of p_m (q xi eta zeta); invVOL^2 enters once at the end
+        const double qxy = q * xi * eta;
+        const double w0 = qxy * (z - Z0), w1 = qxy * (Z1 - z);
+        const double pm[10] = {1.0, u, v, w, u * u, u * v, u * w, v * v, v * w, w * w};
+#pragma unroll
+        for (int j2 = 0; j2 < 10; ++j2) {
+          acc[j2] += pm[j2] * w0;
+          acc[10 + j2] += pm[j2] * w1;
+        }
+      }
+    }
+  }
+  // corner (a, b, c) of cell (lx, ly, lz) is block node (lx + 1 - a, ...)
+  const double scale = kTerms ? 1.0 : (double)iv * (double)iv;
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int nb = ((lx + 1 - ma) * NB + (ly + 1 - mb)) * NB + (lz + 1 - c);
+#pragma unroll
+    for (int j = 0; j < 10; ++j)
+      if (acc[10 * c + j] != 0.0) atomicAdd(&s_mom[j][nb], acc[10 * c + j] * scale);
+  }
+  __syncthreads();
+  for (int i = tid; i < 10 * NB * NB * NB; i += NT) {
+    const int j = i / (NB * NB * NB), nb = i % (NB * NB * NB);
+    const double v = s_mom[j][nb];
+    const int nx = c0x + nb / (NB * NB), ny = c0y + (nb / NB) % NB, nz = c0z + nb % NB;
+    if (v != 0.0 && nx < g.nxn && ny < g.nyn && nz < g.nzn)
+      unsafeAtomicAdd(m.m[j] + (size_t)((nx * g.nyn + ny) * g.nzn + nz), v);
+  }
+}
+
+// Whether a species' deposit goes through tiles: enough particles to fill the
+// workgroups' batches, and a stream that may allocate (a capture keeps the
+// direct kernels).
+inline bool dep_through_tiles(long ntiles, int n, hipStream_t s) {
+  if (n < kDepMinParticles || (long)n < ntiles * kDepMinPerTile || ntiles > (1 << 26))
+    return false;
+  if (s == nullptr) return true;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return cs == hipStreamCaptureStatusNone;
+}
+
+// Deposit through tiles, with the push before it when `f` is given.  `taken`
+// stays false when nothing has run: the caller then has the direct kernels.
+template <typename T>
+hipError_t tile_deposit(const KGrid<T> &g, const KField<T> *f, const KPart<T> &p,
+                        const KPush<T> *k, const KMom &m, unsigned int *status,
+                        hipStream_t s, bool &taken) {
+  taken = false;
+  DepBins b;
+  const long ntx = (g.nxn - 2) / kDepTile + 1;
+  b.nty = (g.nyn - 2) / kDepTile + 1;
+  b.ntz = (g.nzn - 2) / kDepTile + 1;
+  const long ntiles = ntx * b.nty * b.ntz;
+  if (!dep_through_tiles(ntiles, p.n, s)) return hipSuccess;
+  b.ntiles = (int)ntiles;
+  const int slice = p.n < kDepSlice ? p.n : kDepSlice;
+  // about a thousand items at least, so that small species fill the device
+  int run = (slice / 1024 + kDepBatch - 1) / kDepBatch * kDepBatch;
+  b.run = run < kDepBatch ? kDepBatch : run > kDepMaxRun ? kDepMaxRun : run;
+  const size_t max_items = (size_t)slice / b.run + (size_t)(ntiles < slice ? ntiles : slice);
+  auto up = [](size_t v) { return (v + 255) & ~size_t(255); };
+  // the count's particles per thread: enough workgroups first, then few
+  // enough that reading out their counters stays cheap
+  b.per = slice / (kBlock * 2048);
+  b.per = b.per < 1 ? 1 : b.per > 16 ? 16 : b.per;
+  b.in_lds = ntiles <= kDepLdsTiles && ntiles <= 8 * kBlock * b.per ? 1 : 0;
+  const size_t a_cnt = up(4 * (size_t)(ntiles + 2)), a_next = up(4 * (size_t)ntiles),
+               a_items = up(sizeof(uint4) * max_items), a_n = up(4 * (size_t)slice);
+  char *w = nullptr;
+  hipError_t e = stream_alloc((void **)&w, a_cnt + a_next + a_items + 2 * a_n, s);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // the direct kernels need no scratch
+    return hipSuccess;
+  }
+  taken = true;
+  b.cnt = (unsigned int *)w;
+  b.next = (unsigned int *)(w + a_cnt);
+  b.items = (uint4 *)(w + a_cnt + a_next);
+  b.where = (unsigned int *)(w + a_cnt + a_next + a_items);
+  b.perm = (unsigned int *)(w + a_cnt + a_next + a_items + a_n);
+  for (int first = 0; first < p.n && e == hipSuccess; first += slice) {
+    KPart<T> q = p;
+    q.x += first; q.y += first; q.z += first;
+    q.u += first; q.v += first; q.w += first;
+    q.q += first;
+    q.n = p.n - first < slice ? p.n - first : slice;
+    if ((e = zero_u32(b.cnt, (size_t)ntiles + 2, s)) != hipSuccess) break;
+    const unsigned counts = (unsigned)((q.n + kBlock * b.per - 1) / (kBlock * b.per));
+    if (f)
+      hipLaunchKernelGGL((k_dep_count<T, true>), dim3(counts), dim3(kBlock), 0, s, g, *f, q,
+                         *k, b, status);
+    else
+      hipLaunchKernelGGL((k_dep_count<T, false>), dim3(counts), dim3(kBlock), 0, s, g,
+                         KField<T>{}, q, KPush<T>{}, b, status);
+    hipLaunchKernelGGL(k_dep_bounds, dim3(grid_for(b.ntiles)), dim3(kBlock), 0, s, b);
+    // Places by workgroup: 4096 particles each where that leaves 128 of them,
+    // 1024 where few tiles make one atomic per wave contend (131072 particles
+    // on 45 tiles: 73 us per call against 291), else by wave (a million on 1377
+    // tiles that a short workgroup would read out: 239 us against 511).
+    if (ntiles <= kDepLdsTiles && q.n >= 128 * kBlock * 16)
+      hipLaunchKernelGGL((k_dep_place<16, true>), dim3(grid_for((q.n + 15) / 16)), dim3(kBlock),
+                         0, s, b, q.n);
+    else if (ntiles <= 4 * kBlock)
+      hipLaunchKernelGGL((k_dep_place<4, true>), dim3(grid_for((q.n + 3) / 4)), dim3(kBlock), 0,
+                         s, b, q.n);
+    else
+      hipLaunchKernelGGL((k_dep_place<1, false>), dim3(grid_for(q.n)), dim3(kBlock), 0, s, b,
+                         q.n);
+    const size_t items = (size_t)q.n / b.run + (size_t)(ntiles < q.n ? ntiles : q.n);
+    hipLaunchKernelGGL(k_tile_deposit<T>, dim3((unsigned)items), dim3(4 * kDepCells), 0, s, g,
+                       q, m, b);
+    e = hipGetLastError();
+  }
+  const hipError_t ef = stream_free(w, s);
+  return e != hipSuccess ? e : ef;
+}
+
 template <typename T>
 hipError_t launch_mover(const KGrid<T> &g, const KField<T> &f,
                         const KPart<T> &p, const KPush<T> &k,
@@ -315,6 +726,9 @@ template <typename T>
 hipError_t launch_deposit(const KGrid<T> &g, const KPart<T> &p, const KMom &m,
                           unsigned int *status, hipStream_t s) {
   if (p.n <= 0) return hipSuccess;
+  bool taken;
+  const hipError_t e = tile_deposit<T>(g, nullptr, p, nullptr, m, status, s, taken);
+  if (taken) return e;
   hipLaunchKernelGGL(k_deposit<T>, dim3(grid_for(p.n)), dim3(kBlock), 0, s, g,
                      p, m, status);
   return hipGetLastError();
@@ -326,6 +740,9 @@ hipError_t launch_mover_deposit(const KGrid<T> &g, const KField<T> &f,
                                 const KMom &m, unsigned int *status,
                                 hipStream_t s) {
   if (p.n <= 0) return hipSuccess;
+  bool taken;
+  const hipError_t e = tile_deposit<T>(g, &f, p, &k, m, status, s, taken);
+  if (taken) return e;
   hipLaunchKernelGGL(k_mover_deposit<T>, dim3(grid_for(p.n)), dim3(kBlock), 0,
                      s, g, f, p, k, m, status);
   return hipGetLastError();
