@@ -26,7 +26,6 @@
 namespace spic {
 
 constexpr int kMaxSpecies = 8;
-constexpr int kBucketCap = 7;  // LDS bucket slots per cell and batch
 constexpr int kListCap = 128;  // LDS list ring entries
 constexpr int kMaxInstances = 16;  // engines in one batched launch
 constexpr int kMaxTileCells = 128;  // cells of the largest tile shape (8x4x4)
@@ -141,7 +140,7 @@ struct BinnedArgs {
   unsigned int *status;
   // cumulative counters: [0] stencil gathers from global memory, [1]
   // deposits with global atomics, [2] stencil gathers from LDS, [3]
-  // deposits through LDS (bucket or LDS atomics)
+  // deposits through LDS (cell sums or LDS atomics)
   unsigned long long *counters;
   // per-tile moment partials [tile][species][block node][moment] in the
   // particle precision (PartialT<T>), written for every tile-species whose

@@ -17,13 +17,13 @@
 //        tile (it is in the list ring, below) is written when the ring is
 //        flushed, at the next slot of its destination segment's counter;
 //        the overflow region takes particles whose segment is full;
-//      - deposits it (src/Mover.cpp:399-570): a particle in one of the tile's
-//        cells goes into that cell's LDS bucket; one in a halo cell adds its
+//      - deposits it (src/Mover.cpp:399-570): the particles in the tile's
+//        cells are placed in LDS sorted by cell (a count per cell, a scan, a
+//        place per particle), and the four threads of each cell take the
+//        cell's run, each thread two of the cell's eight nodes, and accumulate
+//        their ten moments in registers; a particle in a halo cell adds its
 //        80 contributions to the LDS moment block; one outside the block adds
 //        them to global memory;
-//      - after a barrier the four threads of each cell take the cell's
-//        bucket, each thread two of the cell's eight nodes, and accumulate
-//        their ten moments in registers;
 //   3. adds the register sums into the LDS moment block and stores the block
 //      to the tile-partial scratch, summed per node by k_binned_reduce.
 // k_binned_overflow: the particles of the input overflow regions, one per
@@ -516,6 +516,29 @@ __device__ __forceinline__ int tile_of(const BinnedArgs<T> &a, int ix, int iy, i
 // base plus one per-lane offset.  kNoSlot marks "no slot".
 constexpr uint32_t kNoSlot = 0xffffffffu;
 
+// A value that is the same in every lane, as a scalar: loaded from memory it
+// would sit in a vector register across the batch loop, and the FP64 phase has
+// none to spare (a spilled one is reloaded from scratch memory behind every
+// load and store in flight).
+__device__ __forceinline__ uint32_t uniform(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+
+// Inclusive sum over the lanes of a wave (six DPP adds; ds_bpermute shuffles
+// would put six LDS round trips into every batch).
+__device__ __forceinline__ unsigned int wave_scan(unsigned int v) {
+#define SPIC_DPP_ADD(ctrl, rows) \
+  v += (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false)
+  SPIC_DPP_ADD(0x111, 0xf);  // row_shr 1, 2, 4, 8: within rows of 16
+  SPIC_DPP_ADD(0x112, 0xf);
+  SPIC_DPP_ADD(0x114, 0xf);
+  SPIC_DPP_ADD(0x118, 0xf);
+  SPIC_DPP_ADD(0x142, 0xa);  // row_bcast 15 into rows 1 and 3
+  SPIC_DPP_ADD(0x143, 0xc);  // row_bcast 31 into rows 2 and 3
+#undef SPIC_DPP_ADD
+  return v;
+}
+
 // The particles of range t (see RangeView) with 32-bit slots.
 struct SlotRange {
   uint32_t first, count, gap_lo, gap_len;
@@ -526,7 +549,8 @@ template <typename T>
 __device__ __forceinline__ SlotRange slot_range(const BinnedArgs<T> &a,
                                                 const BinnedSpecies<T> &sp, int t) {
   const RangeView v = range_view(gmem(sp.seg), gmem(sp.cnt_in), a.ntiles, sp.ovf_cap, t);
-  return SlotRange{(uint32_t)v.first, (uint32_t)v.count, v.gap_lo, v.gap_len};
+  return SlotRange{uniform((uint32_t)v.first), uniform((uint32_t)v.count), uniform(v.gap_lo),
+                   uniform(v.gap_len)};
 }
 
 // Component c (x y z u v w q) of the slot at byte offset `off`.
@@ -783,7 +807,16 @@ __device__ __forceinline__ int fx_deposit_cell(int X, int k, int n, bool &bad) {
 // ask for three waves per SIMD (at most 168 VGPRs).  FX: fixed-point
 // positions (FP32, production arithmetic): the x y z words of the particle
 // storage, the output buffer and the list ring hold the int32 coordinates,
-// the buckets the particle's offsets within its deposit cell.
+// the cell-sorted batch the particle's offsets within its deposit cell.
+//
+// Bound by issue and latency at the two (FP64: 256 VGPRs) or three (FP32)
+// waves per SIMD that registers and LDS leave; the particles' traffic is 9% of
+// it (timed without).  The batch is sorted by cell exactly: with buckets of
+// seven slots per cell the particles that met a full one (2% of a mixed plasma)
+// went through the list, 80 LDS atomics each, and the 262M-particle sheet took
+// 16.2 instead of 14.5 ms per FP64 phase, 9.67 instead of 8.94 in FP32 (after
+// 75 phases; 14.0 / 13.3 and 8.29 / 8.08 over the first five).  Carrying
+// them to the next batch instead was slower still.
 template <typename T, typename A, int TX, int TY, int TZ, bool PUSH = true, bool FX = false,
           int PPT = 1>
 __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const int tile) {
@@ -793,21 +826,19 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
   constexpr int NC = TX * TY * TZ;  // cells per tile
   constexpr int NT = 4 * NC;        // threads: four per cell
   constexpr int BX = Blk::BX, BY = Blk::BY, BZ = Blk::BZ, NB = Blk::NB;
-  // PPT: particles each thread pushes and bins per batch before the bucket
-  // step, which then sums PPT x NT particles; the buckets grow with it
-  constexpr int CAP = kBucketCap * PPT;
-  // bucket stride per cell: odd, so that the 16 cells a wave reads in the
-  // bucket step fall on distinct LDS banks
-  constexpr int CS = CAP | 1;
+  // particles per batch; PPT: particles each thread pushes before the cell
+  // step
+  constexpr int NP = NT * PPT;
   constexpr int NL = kListCap;  // list ring entries
   __shared__ T s_fld[NB * 6];
   __shared__ A s_mom[10 * NB];
   __shared__ T s_xn[BX], s_yn[BY], s_zn[BZ];
-  __shared__ T s_bkt[7][NC * CS];  // x y z q u v w of the bucketed particles
+  __shared__ T s_prt[7][NP];       // x y z q u v w of the batch, sorted by cell
   __shared__ T s_lst[7][NL];       // x y z q u v w of the listed particles
   __shared__ unsigned int s_lcell[NL];  // their deposit cells, packed
   __shared__ uint32_t s_lid[NL];        // and their ids
-  __shared__ unsigned int s_cnt[2][NC];
+  __shared__ unsigned int s_cnt[2][NC];   // particles per cell, batches alternating
+  __shared__ unsigned int s_off[NC + 1];  // first place of each cell in s_prt
   __shared__ unsigned int s_nl;    // entries appended to the ring this species
   __shared__ unsigned int s_stay;  // particles written that stay in the tile
   __shared__ unsigned int s_base;  // start of the block reserved for them
@@ -856,7 +887,7 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
     for (int c = 0; c < 6; ++c) s_fld[b * 6 + c] = v[c];
   }
 
-  // this thread's cell and node pair in the bucket step: corners (a, b, 0)
+  // this thread's cell and node pair in the cell step: corners (a, b, 0)
   // and (a, b, 1) of cell (mlx, mly, mlz)
   const int my_cell = tid >> 2;
   const int my_a = (tid >> 1) & 1, my_b = tid & 1;
@@ -883,19 +914,19 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
       // segment in one block
       s_base = gatomic_add(sp.cnt_out + tile, (unsigned int)nin);
     }
-    // entries [0, lst_done) of the ring have been deposited; the same value
-    // in every thread
-    unsigned int lst_done = 0u;
+    // entries [0, lst_done) of the ring have been deposited, and every thread
+    // is done with those of [0, lst_free): uniform
+    unsigned int lst_done = 0u, lst_free = 0u;
     __syncthreads();
-    const unsigned int stay_base = s_base;
+    const unsigned int stay_base = uniform(s_base);
     // this tile's output segment
-    const uint32_t own_lo = (uint32_t)gmem(sp.seg)[tile];
-    const uint32_t own_cap = (uint32_t)gmem(sp.seg)[tile + 1] - own_lo;
+    const uint32_t own_lo = uniform((uint32_t)gmem(sp.seg)[tile]);
+    const uint32_t own_cap = uniform((uint32_t)gmem(sp.seg)[tile + 1]) - own_lo;
     T acc[20];  // register sums, particle precision
 #pragma unroll
     for (int k = 0; k < 20; ++k) acc[k] = T(0);
 
-    const uint32_t nbatches = (nin + NT * PPT - 1) / (NT * PPT);
+    const uint32_t nbatches = (nin + NP - 1) / NP;
     // this thread's particle of batch j (x y z u v w q and its id), loaded
     // one batch ahead.  PREFETCH: batch j + 1 is loaded while batch j is
     // processed -- FP32, which has the registers for it at three waves per
@@ -905,7 +936,7 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
     // batch j is pushed and binned, before its particles are stored, so that
     // the loads cannot take the registers those stores still read (a load
     // into a register a pending store reads waits for the store) and are in
-    // flight over the stores, the bucket and the list steps: 2% faster than
+    // flight over the stores, the cell and the list steps: 2% faster than
     // loading at the start of each batch, and than loading after the stores.
     constexpr bool PREFETCH = sizeof(T) == 4 || !PUSH;
     constexpr bool LATE = !PREFETCH;
@@ -929,7 +960,13 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
     for (uint32_t j = 0; j < nbatches; ++j) {
       const int buf = (int)(j & 1);
       int bad_move = 0, bad_dep = 0, bad_store = 0;  // this batch's
-#pragma unroll 1
+      // this thread's particles of the batch: values, id, cell in the tile
+      // (negative: none, or it has left) and rank within the cell
+      T X[PPT], Y[PPT], Z[PPT], U[PPT], V[PPT], W[PPT], Q[PPT];
+      uint32_t PID[PPT];
+      int CELL[PPT];
+      unsigned int RANK[PPT];
+#pragma unroll
       for (int pp = 0; pp < PPT; ++pp) {
       // this thread's particle pp of batch j, and whether one follows
       const uint32_t step = j * (uint32_t)PPT + (uint32_t)pp;
@@ -981,36 +1018,24 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
         dest = in_tile ? tile : tile_of<TX, TY, TZ>(a, ix, iy, iz);
       }
 
-      // deposit: bucket (tile cell), else the list ring (halo cell,
-      // outside the block, full bucket), else directly
-      bool bucketed = false;
+      // deposit: with its cell's particles (tile cell), else through the list
+      // ring (halo cell, outside the block), else directly
+      X[pp] = x; Y[pp] = y; Z[pp] = z; U[pp] = u; V[pp] = v; W[pp] = w; Q[pp] = q;
+      PID[pp] = pid;
+      CELL[pp] = -1;
+      RANK[pp] = 0u;
       if (active) {
         bool done = false;
         if (in_tile) {
-          const int cell = ((ix - 2 - blk.c0x) * TY + (iy - 2 - blk.c0y)) * TZ + (iz - 2 - blk.c0z);
-          const unsigned int sl = atomicAdd(&s_cnt[buf][cell], 1u);
-          if (sl < (unsigned int)CAP) {
-            const int e = cell * CS + (int)sl;
-            if constexpr (FX) {
-              // offsets within the (unclamped) cell: the fixed-point
-              // coordinate's low bits
-              s_bkt[0][e] = (float)(__float_as_int(x) & ((1 << a.fx.k[0]) - 1)) * a.fx.unit[0];
-              s_bkt[1][e] = (float)(__float_as_int(y) & ((1 << a.fx.k[1]) - 1)) * a.fx.unit[1];
-              s_bkt[2][e] = (float)(__float_as_int(z) & ((1 << a.fx.k[2]) - 1)) * a.fx.unit[2];
-            } else {
-              s_bkt[0][e] = x; s_bkt[1][e] = y; s_bkt[2][e] = z;
-            }
-            s_bkt[3][e] = q;
-            s_bkt[4][e] = u; s_bkt[5][e] = v; s_bkt[6][e] = w;
-            done = true;
-            bucketed = true;
-            ++n_ld;
-          }
-        }
-        if (!done) {
-          // halo cell, outside the block or full bucket: to the list
+          CELL[pp] =
+              ((ix - 2 - blk.c0x) * TY + (iy - 2 - blk.c0y)) * TZ + (iz - 2 - blk.c0z);
+          RANK[pp] = atomicAdd(&s_cnt[buf][CELL[pp]], 1u);
+          done = true;
+          ++n_ld;
+        } else {
+          // halo cell or outside the block: to the list
           const unsigned int k = atomicAdd(&s_nl, 1u);
-          if (k - lst_done < (unsigned int)NL) {
+          if (k - lst_free < (unsigned int)NL) {
             const unsigned int e = k % NL;
             s_lst[0][e] = x; s_lst[1][e] = y; s_lst[2][e] = z; s_lst[3][e] = q;
             s_lst[4][e] = u; s_lst[5][e] = v; s_lst[6][e] = w;
@@ -1045,29 +1070,71 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
       }
 
       if (LATE && step + 1 < nbatches * (uint32_t)PPT) load_particle(r + NT);
-      // the bucketed particles stay in the tile: their slots come from the
-      // workgroup's reserved block, one LDS counter atomic per wave
+      }  // particle pp of the batch
+
+      __syncthreads();  // counts and list entries are complete
+      const unsigned int nl = uniform(s_nl);
+      // every wave scans the cells' counts for itself and writes the same
+      // offsets, so that its own reads of them need no barrier
       {
-        const unsigned long long m = __ballot(bucketed);
+        constexpr int CPL = NC / 64;  // cells per lane
+        unsigned int c[CPL], sum = 0;
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+          c[i] = s_cnt[buf][lane * CPL + i];
+          sum += c[i];
+        }
+        unsigned int at = wave_scan(sum);
+        if (lane == 63) s_off[NC] = at;
+        at -= sum;
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+          s_off[lane * CPL + i] = at;
+          at += c[i];
+        }
+        if (tid < NC) s_cnt[buf ^ 1][tid] = 0u;  // for the next batch
+      }
+#pragma unroll
+      for (int pp = 0; pp < PPT; ++pp) {
+        const bool stays = CELL[pp] >= 0;
+        if (stays) {
+          const unsigned int e = s_off[CELL[pp]] + RANK[pp];
+          if constexpr (FX) {
+            // offsets within the (unclamped) cell: the fixed-point
+            // coordinate's low bits
+            s_prt[0][e] = (float)(__float_as_int(X[pp]) & ((1 << a.fx.k[0]) - 1)) * a.fx.unit[0];
+            s_prt[1][e] = (float)(__float_as_int(Y[pp]) & ((1 << a.fx.k[1]) - 1)) * a.fx.unit[1];
+            s_prt[2][e] = (float)(__float_as_int(Z[pp]) & ((1 << a.fx.k[2]) - 1)) * a.fx.unit[2];
+          } else {
+            s_prt[0][e] = X[pp]; s_prt[1][e] = Y[pp]; s_prt[2][e] = Z[pp];
+          }
+          s_prt[3][e] = Q[pp];
+          s_prt[4][e] = U[pp]; s_prt[5][e] = V[pp]; s_prt[6][e] = W[pp];
+        }
+        // the particles that stay in the tile take their slots from the
+        // workgroup's reserved block, one LDS counter atomic per wave
+        const unsigned long long m = __ballot(stays);
         if (m) {
           const int leader = __ffsll((long long)m) - 1;
           unsigned int jb = 0;
           if (lane == leader) jb = atomicAdd(&s_stay, (unsigned int)__popcll(m));
           jb = __shfl(jb, leader);
-          if (bucketed) {
-            const unsigned int jj = jb + (unsigned int)__popcll(m & ((1ull << lane) - 1ull));
-            bad_store |= !put_particle(a, sp, own_lo, own_cap, stay_base, true, jj, tile, x,
-                                       y, z, u, v, w, q, pid);
+          if (stays) {
+            const unsigned int jj =
+                jb + __builtin_amdgcn_mbcnt_hi((unsigned int)(m >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((unsigned int)m, 0u));
+            bad_store |= !put_particle(a, sp, own_lo, own_cap, stay_base, true, jj, tile, X[pp],
+                                       Y[pp], Z[pp], U[pp], V[pp], W[pp], Q[pp], PID[pp]);
           }
         }
       }
-      }  // particle pp of the batch
 
-      // bucket step: each cell's four threads sum the cell's bucket
+      // cell step: each cell's four threads sum its particles.  No barrier
+      // follows: the next batch writes s_prt and s_off only behind its first
+      // one, counts in the other s_cnt, and leaves the list entries that
+      // this batch may still be reading (lst_free)
       __syncthreads();
       {
-        const unsigned int nb_c = min(s_cnt[buf][my_cell], (unsigned int)CAP);
-        if ((tid & 3) == 0) s_cnt[buf ^ 1][my_cell] = 0u;  // for the next batch
         const T X0 = s_xn[mlx + 1], X1 = s_xn[mlx + 2];
         const T Y0 = s_yn[mly + 1], Y1 = s_yn[mly + 2];
         const T Z0 = s_zn[mlz + 1], Z1 = s_zn[mlz + 2];
@@ -1078,10 +1145,10 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
         const T sa = my_a ? T(-1) : T(1), sb = my_b ? T(-1) : T(1);
         const T ca = FX ? (my_a ? T(1) : T(0)) : (my_a ? X1 : -X0);
         const T cb = FX ? (my_b ? T(1) : T(0)) : (my_b ? Y1 : -Y0);
-        for (unsigned int k = 0; k < nb_c; ++k) {
-          const int e = my_cell * CS + (int)k;
-          const T px = s_bkt[0][e], py = s_bkt[1][e], pz = s_bkt[2][e];
-          const T pq = s_bkt[3][e], pu = s_bkt[4][e], pv = s_bkt[5][e], pw = s_bkt[6][e];
+        const unsigned int end = s_off[my_cell + 1];
+        for (unsigned int e = s_off[my_cell]; e < end; ++e) {
+          const T px = s_prt[0][e], py = s_prt[1][e], pz = s_prt[2][e];
+          const T pq = s_prt[3][e], pu = s_prt[4][e], pv = s_prt[5][e], pw = s_prt[6][e];
           // px py pz: the particle's position, or with FX its offsets
           // within the cell (the distances from nodes X0 Y0 Z0 in cells)
           const T xa = fma(sa, px, ca);
@@ -1112,13 +1179,28 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
       }
       // list step: once the ring is half full (and after the species' last
       // batch), all threads deposit its pending entries, eight threads per
-      // entry, one node each.  s_nl is not written again before the next
-      // barrier, so every thread reads the same value and takes the same
-      // decision.
+      // entry, one node each.  Entry tid's slot is asked for first and its
+      // particle stored last: the counter atomic returns only behind every
+      // load and store in flight, and that wait overlaps the deposit.  The
+      // decision is uniform: nl was read between the barriers, where no
+      // thread appends.
       {
-        const unsigned int nl = s_nl;
-        const unsigned int pend = min(nl - lst_done, (unsigned int)NL);
-        if (pend >= (unsigned int)(NL / 2) || (j == nbatches - 1 && pend > 0u)) {
+        // entries from lst_free + NL on were refused (deposited directly); a
+        // ring that refused some is flushed, so that its entries stay a run
+        const bool full = nl - lst_free > (unsigned int)NL;
+        const unsigned int kept = full ? lst_free + (unsigned int)NL : nl;
+        const unsigned int pend = (int)(kept - lst_done) > 0 ? kept - lst_done : 0u;
+        lst_free = lst_done;
+        if (pend >= (unsigned int)(NL / 2) || full || (j == nbatches - 1 && pend > 0u)) {
+          static_assert(NL <= NT, "one entry per thread");
+          const unsigned int mine = (lst_done + (unsigned int)tid) % NL;
+          unsigned int slot_k = 0;
+          if ((unsigned int)tid < pend) {
+            const unsigned int c = s_lcell[mine];
+            const int dest = tile_of<TX, TY, TZ>(a, (int)(c >> 20), (int)((c >> 10) & 1023u),
+                                                 (int)(c & 1023u));
+            slot_k = dest == tile ? atomicAdd(&s_stay, 1u) : gatomic_add(sp.cnt_out + dest, 1u);
+          }
           const int nd = tid & 7;
           for (unsigned int k = (unsigned int)(tid >> 3); k < pend; k += NT / 8) {
             const unsigned int e = (lst_done + k) % NL;
@@ -1139,19 +1221,25 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
             if (nd == 0) {
               if (lds) ++n_ld;
               else ++n_gd;
-              // and the entry's particle to the output buffer
-              const int pdest = tile_of<TX, TY, TZ>(a, jx, jy, jz);
-              const bool stay = pdest == tile;
-              const unsigned int jj = stay ? atomicAdd(&s_stay, 1u) : 0u;
-              bad_store |= !put_particle(a, sp, own_lo, own_cap, stay_base, stay, jj, pdest,
-                                         px, py, pz, pu, pv, pw, pq, s_lid[e]);
             }
+          }
+          if ((unsigned int)tid < pend) {
+            const unsigned int c = s_lcell[mine];
+            const int dest = tile_of<TX, TY, TZ>(a, (int)(c >> 20), (int)((c >> 10) & 1023u),
+                                                 (int)(c & 1023u));
+            const uint32_t o =
+                seg_slot(a, sp, dest, dest == tile ? stay_base + slot_k : slot_k);
+            if (o == kNoSlot)
+              bad_store = 1;
+            else
+              write_particle(sp, o, s_lst[0][mine], s_lst[1][mine], s_lst[2][mine],
+                             s_lst[4][mine], s_lst[5][mine], s_lst[6][mine], s_lst[3][mine],
+                             s_lid[mine]);
           }
           lst_done = nl;
         }
       }
       bad_bits |= (bad_move ? 1 : 0) | (bad_dep ? 2 : 0) | (bad_store ? 4 : 0);
-      __syncthreads();
     }
 
     // 3. register sums into the LDS block: corner (a, b, c) of cell
@@ -1202,7 +1290,7 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
 
 // PUSH false: the deposit alone (spic_engine_deposit), in its own
 // instances so that the phase kernels carry no test for it.  PPT 2 (two
-// particles per thread and batch, FP32 fixed point only): its buckets take
+// particles per thread and batch, FP32 fixed point only): its batch takes
 // the LDS of a third workgroup, so it asks for two waves per SIMD.
 template <typename T, typename A, int TX, int TY, int TZ, bool PUSH = true, bool FX = false,
           int PPT = 1>

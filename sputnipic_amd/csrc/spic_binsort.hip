@@ -9,7 +9,7 @@
 // orders each tile's particles round-robin over its cells (every cell's
 // first particle, then every cell's second, ...), so that any run of
 // 4 * cells-per-tile consecutive particles holds about four per cell: the
-// phase kernel takes one such run per batch into its per-cell buckets, and
+// phase kernel sums one such run per batch cell by cell, and
 // particles that stay in their tile keep this order from phase to phase.
 // A stable LSD radix sort (rocPRIM) of (key, source slot) pairs gives the
 // permutation; the seven arrays and the particle id are gathered to sorted
