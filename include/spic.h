@@ -253,8 +253,10 @@ int spic_maxwell_image(const spic_grid *grd, const spic_field *field,
 /* slots) and an overflow region, and a particle id per slot, so particles */
 /* can be copied out in the order they were loaded.  Each phase writes     */
 /* every particle into its destination tile's segment of the other buffer, */
-/* so the binning stays current without a separate sort.  A sort (on load, */
-/* every `sort_every` phases, or on request) rebuilds the segments.        */
+/* so the binning stays current without a separate sort; a phase that      */
+/* finds more than 256 particles in the overflow region first fits the     */
+/* other buffer's segments to the tiles' present particles.  A sort (on    */
+/* load, every `sort_every` phases, or on request) rebuilds the segments.  */
 /* Neither changes a particle's trajectory, only the summation order of    */
 /* the moments.                                                            */
 /* ---------------------------------------------------------------------- */

@@ -5,17 +5,23 @@
 //   slots [seg[t], seg[t+1])      tile t's segment;
 //   slots [seg[ntiles], +ovf_cap)  overflow region, for particles whose
 //                                  destination segment was full.
-// Per buffer, one array of 3 * (ntiles + 1) counters:
+// Per buffer its segment bounds seg[ntiles + 1] and one array of
+// kCntArrays * (ntiles + 1) counters (NT1 = ntiles + 1):
 //   cnt[t]                 slots of range t taken (t == ntiles: the overflow
 //                          region); may exceed the range's capacity, the
 //                          excess went to the overflow region;
-//   cnt[NT1 + t], cnt[2 * NT1 + t]   (NT1 = ntiles + 1) the start and length
-//                          of one unused run inside the taken slots: the
-//                          rest of the block a tile's workgroup reserved for
-//                          the particles that stayed in it.
+//   cnt[NT1 + t], cnt[2 * NT1 + t]   the start and length of one unused run
+//                          inside the taken slots: the rest of the block a
+//                          tile's workgroup reserved for the particles that
+//                          stayed in it;
+//   cnt[3 * NT1 + t]       the slots of that block that no particle took,
+//                          inside the segment or beyond its end.
 // Range t holds min(cnt[t], capacity) - length particles, at the taken slots
-// outside the unused run.  Both buffers of a pair share seg; a phase reads
-// one and writes the other.
+// outside the unused run; cnt[t] - cnt[3 * NT1 + t] particles lie in tile t,
+// those in the overflow region included.  A phase reads one buffer and writes
+// the other, whose segments are the read buffer's (phase_layout) or, when its
+// overflow region holds more than kRelayoutOverflow particles, fitted anew to
+// the particles of each tile.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,8 +32,16 @@
 namespace spic {
 
 constexpr int kMaxSpecies = 8;
+constexpr int kCntArrays = 4;  // counter arrays of a buffer, see above
 constexpr int kListCap = 128;  // LDS list ring entries
 constexpr int kMaxInstances = 16;  // engines in one batched launch
+// Particles in an overflow region from which the next phase fits the segments
+// anew.  Up to one workgroup's worth costs the overflow pass nothing beyond its
+// launch; without a new fit a run whose density changes by more than the slack
+// keeps a growing part of its particles there, pushed and deposited through
+// global memory (262M-particle FP32 sheet without re-sorts: 8.6 ms per phase
+// after 50 phases, 26 after 200, 110 after 800).
+constexpr unsigned int kRelayoutOverflow = 256;
 constexpr int kMaxTileCells = 128;  // cells of the largest tile shape (8x4x4)
 
 // Blocks of a batched launch: instance i owns blocks [start[i], start[i+1]),
@@ -111,10 +125,13 @@ struct BinnedSpecies {
   int64_t stride;
   const uint32_t *id_in;  // load index per slot; both null when the engine
   uint32_t *id_out;       // keeps no load order
-  const int64_t *seg;          // [ntiles + 1]
-  const unsigned int *cnt_in;  // [3 * (ntiles + 1)], see above
-  unsigned int *cnt_out;       // [3 * (ntiles + 1)], zero on entry
+  const int64_t *seg_in;       // [ntiles + 1] of the buffer read
+  int64_t *seg_out;            // and of the one written (phase_layout)
+  const unsigned int *cnt_in;  // [kCntArrays * (ntiles + 1)], see above
+  unsigned int *cnt_out;       // [kCntArrays * (ntiles + 1)], zero on entry
   unsigned int ovf_cap;
+  int64_t slack;               // free slots per segment, on average
+  int64_t n;                   // the species' particles
   KPush<T> k;
   KMom m;
 };
@@ -161,10 +178,21 @@ struct BinnedReduceArgs {
   KMom mom[kMaxSpecies];
 };
 
+// The segments of the buffer a phase writes, from those and the counters of
+// the buffer it reads.
+struct LayoutArgs {
+  const int64_t *seg_in;
+  int64_t *seg_out;
+  const unsigned int *cnt_in;
+  int64_t slack, n;
+};
+
 struct CountArrays {
   unsigned int *p[kMaxSpecies];
   int n;  // entries per array
   int ns;
+  LayoutArgs lay[kMaxSpecies];  // seg_out null: no layout to write
+  int ntiles;
   // nn > 0: also zero the ten moment arrays of nn nodes of each species
   KMom mom[kMaxSpecies];
   int64_t nn;
@@ -238,20 +266,22 @@ inline FixedParams fixed_params(int ncx, int ncy, int ncz, double dx, double dy,
 // Sums the tile partials of every species into its node moments (+=).
 hipError_t launch_binned_reduce(const BinnedReduceArgs &a, int tx, int ty, int tz,
                                 int nn, hipStream_t s);
-// Zeroes ns count arrays of n entries each (and the moments, c.nn > 0).
-hipError_t zero_counts(const CountArrays &c, hipStream_t s);
+// The first launch of a phase: zeroes ns count arrays of n entries each (and
+// the moments, c.nn > 0) and writes the segments of the output buffers.
+hipError_t phase_start(const CountArrays &c, hipStream_t s);
 
 // The reduce and the count reset of a batch, from the device-resident
 // argument blocks tab[i] of its instances: per instance, the node blocks
-// nodes.start[i].. of 256 nodes each (reduce) and the reset blocks
-// counts.start[i].. of 256 threads each, thread j resetting counter j of
-// every species' cnt_out (3 * (ntiles + 1) entries) and, with `moments`,
-// node j of its ten moment arrays; max_ns species per launch row.
+// nodes.start[i].. of 256 nodes each (reduce) and the blocks
+// counts.start[i].. of 256 threads each: the first writes the segments of
+// every species' output buffer, thread j of the others resets counter j of its
+// cnt_out (kCntArrays * (ntiles + 1) entries) and, with `moments`, node j of
+// its ten moment arrays; max_ns species per launch row.
 template <typename T>
 hipError_t launch_batch_reduce(const BinnedArgs<T> *tab, const BatchMap &nodes,
                                int max_ns, int tx, int ty, int tz, hipStream_t s);
 template <typename T>
-hipError_t launch_batch_zero_counts(const BinnedArgs<T> *tab, const BatchMap &counts,
+hipError_t launch_batch_start(const BinnedArgs<T> *tab, const BatchMap &counts,
                                     int max_ns, int moments, hipStream_t s);
 
 // Sort of n particles of one species into binned storage (spic_binsort.hip).

@@ -548,7 +548,7 @@ struct SlotRange {
 template <typename T>
 __device__ __forceinline__ SlotRange slot_range(const BinnedArgs<T> &a,
                                                 const BinnedSpecies<T> &sp, int t) {
-  const RangeView v = range_view(gmem(sp.seg), gmem(sp.cnt_in), a.ntiles, sp.ovf_cap, t);
+  const RangeView v = range_view(gmem(sp.seg_in), gmem(sp.cnt_in), a.ntiles, sp.ovf_cap, t);
   return SlotRange{uniform((uint32_t)v.first), uniform((uint32_t)v.count), uniform(v.gap_lo),
                    uniform(v.gap_len)};
 }
@@ -587,11 +587,11 @@ template <typename T>
 __device__ __forceinline__ uint32_t seg_slot(const BinnedArgs<T> &a,
                                              const BinnedSpecies<T> &sp, int dest,
                                              unsigned int k) {
-  const uint32_t lo = (uint32_t)gmem(sp.seg)[dest];
-  const uint32_t cap = (uint32_t)gmem(sp.seg)[dest + 1] - lo;
+  const uint32_t lo = (uint32_t)gmem(sp.seg_out)[dest];
+  const uint32_t cap = (uint32_t)gmem(sp.seg_out)[dest + 1] - lo;
   if (k < cap) return lo + k;
   const unsigned int o = gatomic_add(sp.cnt_out + a.ntiles, 1u);
-  return o < sp.ovf_cap ? (uint32_t)gmem(sp.seg)[a.ntiles] + o : kNoSlot;
+  return o < sp.ovf_cap ? (uint32_t)gmem(sp.seg_out)[a.ntiles] + o : kNoSlot;
 }
 
 template <typename T>
@@ -626,7 +626,7 @@ __device__ __forceinline__ bool put_particle(const BinnedArgs<T> &a,
       o = own_lo + k;
     } else {
       const unsigned int e = gatomic_add(sp.cnt_out + a.ntiles, 1u);
-      o = e < sp.ovf_cap ? (uint32_t)gmem(sp.seg)[a.ntiles] + e : kNoSlot;
+      o = e < sp.ovf_cap ? (uint32_t)gmem(sp.seg_out)[a.ntiles] + e : kNoSlot;
     }
   } else {
     o = seg_slot(a, sp, dest, gatomic_add(sp.cnt_out + dest, 1u));
@@ -920,8 +920,8 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
     __syncthreads();
     const unsigned int stay_base = uniform(s_base);
     // this tile's output segment
-    const uint32_t own_lo = uniform((uint32_t)gmem(sp.seg)[tile]);
-    const uint32_t own_cap = uniform((uint32_t)gmem(sp.seg)[tile + 1]) - own_lo;
+    const uint32_t own_lo = uniform((uint32_t)gmem(sp.seg_out)[tile]);
+    const uint32_t own_cap = uniform((uint32_t)gmem(sp.seg_out)[tile + 1]) - own_lo;
     T acc[20];  // register sums, particle precision
 #pragma unroll
     for (int k = 0; k < 20; ++k) acc[k] = T(0);
@@ -1265,7 +1265,7 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
     if (tid == 0) {
       // the reserved block [stay_base, stay_base + nin) holds s_stay
       // particles; its remainder inside the segment stays unused
-      const int64_t cap = gmem(sp.seg)[tile + 1] - gmem(sp.seg)[tile];
+      const int64_t cap = gmem(sp.seg_out)[tile + 1] - gmem(sp.seg_out)[tile];
       const int64_t room = cap > (int64_t)stay_base ? cap - (int64_t)stay_base : 0;
       const int64_t lo = (int64_t)stay_base + min((int64_t)s_stay, room);
       const int64_t hi = min((int64_t)stay_base + nin, cap);
@@ -1273,6 +1273,7 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
         gmem(sp.cnt_out)[(a.ntiles + 1) + tile] = (unsigned int)lo;
         gmem(sp.cnt_out)[2 * (a.ntiles + 1) + tile] = (unsigned int)(hi - lo);
       }
+      gmem(sp.cnt_out)[3 * (a.ntiles + 1) + tile] = nin - s_stay;
     }
     __syncthreads();
   }

@@ -240,6 +240,7 @@ __global__ void k_bin_bounds(const uint32_t *__restrict__ keys, int shift, int64
     cnt[t] = t < ntiles ? (unsigned int)(b[1] - b[0]) : 0u;
     cnt[(ntiles + 1) + t] = 0u;
     cnt[2 * (ntiles + 1) + t] = 0u;
+    cnt[3 * (ntiles + 1) + t] = 0u;
   }
 }
 
@@ -300,14 +301,65 @@ __global__ void k_bin_store_be32(Arrays7<T> src, const uint32_t *__restrict__ id
   }
 }
 
-// Per species (blockIdx.y): thread i zeroes counter i (i < n) and, with
-// c.nn > 0, node i of the ten moment arrays (i < nn).
-__global__ void k_zero_counts(CountArrays c) {
+// One workgroup of 256 threads writes the output buffer's segments of a
+// species: the input buffer's, or, when its overflow region holds more than
+// kRelayoutOverflow particles, segments of each tile's particles plus its
+// share of the slack, half of it even and half in proportion to the particles
+// (arrivals grow with them).  Both halves are rounded down, so the segments
+// take at most n + ntiles * slack slots and the overflow region after them
+// stays inside the buffer.
+__device__ __forceinline__ void phase_layout(const LayoutArgs &l, int ntiles) {
+  __shared__ unsigned long long s_sum[4];
+  const SPIC_GLOBAL int64_t *in = gmem(l.seg_in);
+  SPIC_GLOBAL int64_t *out = gmem(l.seg_out);
+  const SPIC_GLOBAL unsigned int *cnt = gmem(l.cnt_in);
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (cnt[ntiles] <= kRelayoutOverflow) {
+    for (int t = tid; t <= ntiles; t += 256) out[t] = in[t];
+    return;
+  }
+  const int64_t even = l.slack / 2;
+  const double share = l.n > 0 ? 0.5 * (double)l.slack * (double)ntiles / (double)l.n : 0.0;
+  auto slots = [&](int t) -> unsigned long long {
+    const unsigned int held = cnt[t] - cnt[3 * (ntiles + 1) + t];
+    return (unsigned long long)held + (unsigned long long)even +
+           (unsigned long long)((double)held * share);
+  };
+  // thread t sums a run of tiles, the workgroup scans the sums
+  const int per = (ntiles + 255) / 256;
+  const int t0 = min(tid * per, ntiles), t1 = min(t0 + per, ntiles);
+  unsigned long long sum = 0;
+  for (int t = t0; t < t1; ++t) sum += slots(t);
+  unsigned long long at = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned long long v = __shfl_up(at, d);
+    if (lane >= d) at += v;
+  }
+  if (lane == 63) s_sum[tid >> 6] = at;
+  __syncthreads();
+  at -= sum;
+  for (int w = 0; w < (tid >> 6); ++w) at += s_sum[w];
+  for (int t = t0; t < t1; ++t) {
+    out[t] = (int64_t)at;
+    at += slots(t);
+  }
+  if (tid == 255) out[ntiles] = (int64_t)at;
+}
+
+// Per species (blockIdx.y): the first workgroup writes the output segments;
+// thread i of the others zeroes counter i (i < n) and, with c.nn > 0, node i
+// of the ten moment arrays (i < nn).
+__global__ __launch_bounds__(256) void k_phase_start(CountArrays c) {
   const int s = blockIdx.y;
   if (s >= c.ns) return;
+  if (blockIdx.x == 0) {
+    if (c.lay[s].seg_out) phase_layout(c.lay[s], c.ntiles);
+    return;
+  }
   const int64_t total = c.n > c.nn ? c.n : c.nn;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i = (blockIdx.x - 1) * (int64_t)blockDim.x + threadIdx.x; i < total;
+       i += (int64_t)(gridDim.x - 1) * blockDim.x) {
     if (i < c.n) gmem(c.p[s])[i] = 0u;
     if (i < c.nn) {
 #pragma unroll
@@ -385,19 +437,23 @@ __global__ __launch_bounds__(256) void k_binned_reduce_batch(
                                        a.sp[s].m.m);
 }
 
-// The count reset of a batch (blockIdx.y is the species): thread j of
-// instance i zeroes counter j and, when `moments` is set, node j of the ten
-// moment arrays.
+// The same for a batch: the blocks of instance i are map.start[i] and up.
 template <typename T>
-__global__ __launch_bounds__(256) void k_zero_counts_batch(
+__global__ __launch_bounds__(256) void k_phase_start_batch(
     const BinnedArgs<T> *__restrict__ tab, BatchMap map, int moments) {
   int i = 0;
   for (int k = 1; k < map.n; ++k) i += (int)blockIdx.x >= map.start[k] ? 1 : 0;
   const BinnedArgs<T> &a = tab[i];
   const int s = blockIdx.y;
   if (s >= a.ns) return;
-  const int64_t j = (int64_t)(blockIdx.x - map.start[i]) * 256 + threadIdx.x;
-  if (j < 3 * (int64_t)(a.ntiles + 1)) gmem(a.sp[s].cnt_out)[j] = 0u;
+  const int block = blockIdx.x - map.start[i];
+  if (block == 0) {
+    const BinnedSpecies<T> &sp = a.sp[s];
+    phase_layout(LayoutArgs{sp.seg_in, sp.seg_out, sp.cnt_in, sp.slack, sp.n}, a.ntiles);
+    return;
+  }
+  const int64_t j = (int64_t)(block - 1) * 256 + threadIdx.x;
+  if (j < kCntArrays * (int64_t)(a.ntiles + 1)) gmem(a.sp[s].cnt_out)[j] = 0u;
   if (moments && j < (int64_t)a.g.nxn * a.g.nyn * a.g.nzn) {
 #pragma unroll
     for (int m = 0; m < 10; ++m) gmem(a.sp[s].m.m[m])[j] = 0.0;
@@ -440,10 +496,10 @@ hipError_t launch_batch_reduce(const BinnedArgs<T> *tab, const BatchMap &nodes,
 }
 
 template <typename T>
-hipError_t launch_batch_zero_counts(const BinnedArgs<T> *tab, const BatchMap &counts,
+hipError_t launch_batch_start(const BinnedArgs<T> *tab, const BatchMap &counts,
                                     int max_ns, int moments, hipStream_t s) {
   if (counts.n <= 0 || counts.start[counts.n] <= 0 || max_ns <= 0) return hipSuccess;
-  hipLaunchKernelGGL((k_zero_counts_batch<T>), dim3(counts.start[counts.n], max_ns),
+  hipLaunchKernelGGL((k_phase_start_batch<T>), dim3(counts.start[counts.n], max_ns),
                      dim3(256), 0, s, tab, counts, moments);
   return hipGetLastError();
 }
@@ -453,10 +509,10 @@ template hipError_t launch_batch_reduce<double>(const BinnedArgs<double> *,
                                                 hipStream_t);
 template hipError_t launch_batch_reduce<float>(const BinnedArgs<float> *, const BatchMap &,
                                                int, int, int, int, hipStream_t);
-template hipError_t launch_batch_zero_counts<double>(const BinnedArgs<double> *,
+template hipError_t launch_batch_start<double>(const BinnedArgs<double> *,
                                                      const BatchMap &, int, int,
                                                      hipStream_t);
-template hipError_t launch_batch_zero_counts<float>(const BinnedArgs<float> *,
+template hipError_t launch_batch_start<float>(const BinnedArgs<float> *,
                                                     const BatchMap &, int, int, hipStream_t);
 
 // Copy particle j of the source to slot o of the destination.
@@ -614,6 +670,7 @@ __device__ __forceinline__ void tile_bounds_body(const TileSortJob<T> &J) {
       gmem(J.dst_cnt)[t] = c;
       gmem(J.dst_cnt)[(nt + 1) + t] = 0u;
       gmem(J.dst_cnt)[2 * (nt + 1) + t] = 0u;
+      gmem(J.dst_cnt)[3 * (nt + 1) + t] = 0u;
     }
     __syncthreads();
     if (tid == 0) s_carry = carry + s_wsum[NW - 1];
@@ -936,9 +993,9 @@ template hipError_t tile_sort_batch<float>(const TileSortJob<float> *, const Til
                                            int, int, int, unsigned int *, size_t,
                                            hipStream_t);
 
-hipError_t zero_counts(const CountArrays &c, hipStream_t s) {
+hipError_t phase_start(const CountArrays &c, hipStream_t s) {
   if (c.ns <= 0 || c.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_zero_counts, dim3(nblocks(c.n > c.nn ? c.n : c.nn), c.ns), dim3(256),
+  hipLaunchKernelGGL(k_phase_start, dim3(1 + nblocks(c.n > c.nn ? c.n : c.nn), c.ns), dim3(256),
                      0, s, c);
   return hipGetLastError();
 }

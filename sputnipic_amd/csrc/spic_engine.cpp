@@ -46,10 +46,11 @@ struct spic_engine {
     void *block[2] = {};           // two buffers of x y z u v w q, one block each
     void *buf[2][7] = {};          // the components: block[b] + c * cap
     uint32_t *id[2] = {nullptr, nullptr};
-    unsigned int *cnt[2] = {nullptr, nullptr};  // [3 * (ntiles + 1)] per buffer
-    int64_t *seg[2] = {nullptr, nullptr};       // [ntiles + 1] per layout
+    unsigned int *cnt[2] = {nullptr, nullptr};  // [kCntArrays * (ntiles + 1)] per buffer
+    int64_t *seg[2] = {nullptr, nullptr};       // [ntiles + 1] per buffer
     int cur = 0;                   // buffer holding the particles
-    int segi = 0;                  // layout in use
+    int parity = 0;                // of the re-sorts since the load: a batch's members
+                                   // are sorted in step
   } sp[spic::kMaxSpecies];
   unsigned long long *counters = nullptr;  // see BinnedArgs::counters
   void *partials = nullptr;        // see BinnedArgs::partials
@@ -98,7 +99,7 @@ void free_species(spic_engine *e, spic_engine::Species &s) {
     }
     if (s.cnt[b]) {
       (void)hipFree(s.cnt[b]);
-      e->bytes -= sizeof(unsigned int) * 3 * nt1;
+      e->bytes -= sizeof(unsigned int) * spic::kCntArrays * nt1;
     }
     if (s.seg[b]) {
       (void)hipFree(s.seg[b]);
@@ -123,14 +124,13 @@ hipError_t ensure_workspace(spic_engine *e, size_t need, hipStream_t s) {
   return hipSuccess;
 }
 
-// Sort species `is` into the other buffer and the other layout.  With
+// Sort species `is` into the other buffer.  With
 // `src` given, the particles come densely from the caller's arrays instead.
 // A re-sort in SPIC_SORT_TILE mode is a tile sort.
-// The tile-sort job of species `is` from buffer `cur` in layout `segi` into
-// the other ones; count / own / fill at ws.
+// The tile-sort job of species `is` from buffer `cur` into the other one;
+// count / own / fill at ws.
 template <typename T>
-spic::TileSortJob<T> tile_sort_job(const spic_engine *e, int is, int cur, int segi,
-                                   unsigned int *ws) {
+spic::TileSortJob<T> tile_sort_job(const spic_engine *e, int is, int cur, unsigned int *ws) {
   const auto &sp = e->sp[is];
   spic::TileSortJob<T> J;
   std::memset(&J, 0, sizeof(J));
@@ -143,8 +143,8 @@ spic::TileSortJob<T> tile_sort_job(const spic_engine *e, int is, int cur, int se
   J.stride = sp.cap;
   J.src_id = sp.id[from];
   J.dst_id = sp.id[to];
-  J.src_seg = sp.seg[segi];
-  J.dst_seg = sp.seg[1 - segi];
+  J.src_seg = sp.seg[from];
+  J.dst_seg = sp.seg[to];
   J.src_cnt = sp.cnt[from];
   J.dst_cnt = sp.cnt[to];
   J.ovf_cap = sp.ovf_cap;
@@ -161,10 +161,10 @@ hipError_t tile_sort_species(spic_engine *e, int is, hipStream_t s) {
   hipError_t err =
       ensure_workspace(e, 3 * ((size_t)e->L.ntiles + 1) * sizeof(unsigned int), s);
   if (err != hipSuccess) return err;
-  err = spic::tile_sort<T>(tile_sort_job<T>(e, is, sp.cur, sp.segi, (unsigned int *)e->ws), s);
+  err = spic::tile_sort<T>(tile_sort_job<T>(e, is, sp.cur, (unsigned int *)e->ws), s);
   if (err != hipSuccess) return err;
   sp.cur = 1 - sp.cur;
-  sp.segi = 1 - sp.segi;
+  sp.parity ^= 1;
   e->sorts++;
   return hipSuccess;
 }
@@ -179,7 +179,6 @@ hipError_t sort_species(spic_engine *e, int is, void *const *src, int src_f64,
   spic::BinLayout L = e->L;
   L.slack = sp.slack;
   const int from = sp.cur, to = src ? 0 : 1 - sp.cur;
-  const int lay_from = sp.segi, lay_to = src ? 0 : 1 - sp.segi;
   const void *in[7];
   T *out[7];
   for (int a = 0; a < 7; ++a) {
@@ -188,20 +187,20 @@ hipError_t sort_species(spic_engine *e, int is, void *const *src, int src_f64,
   }
   const int in_f64 = src ? src_f64 : (sizeof(T) == 8 ? 1 : 0);
   const uint32_t *in_id = src ? nullptr : sp.id[from];
-  const int64_t *in_seg = src ? nullptr : sp.seg[lay_from];
+  const int64_t *in_seg = src ? nullptr : sp.seg[from];
   const unsigned int *in_cnt = src ? nullptr : sp.cnt[from];
   size_t need = 0;
   hipError_t err = spic::bin_sort<T>(g, L, sp.n, in, in_f64, in_id, in_seg, in_cnt,
-                                     sp.ovf_cap, out, sp.id[to], sp.seg[lay_to], sp.cnt[to],
+                                     sp.ovf_cap, out, sp.id[to], sp.seg[to], sp.cnt[to],
                                      nullptr, 0, &need, s);
   if (err != hipSuccess) return err;
   if ((err = ensure_workspace(e, need, s)) != hipSuccess) return err;
   err = spic::bin_sort<T>(g, L, sp.n, in, in_f64, in_id, in_seg, in_cnt, sp.ovf_cap, out,
-                          sp.id[to], sp.seg[lay_to], sp.cnt[to], e->ws, e->ws_bytes,
+                          sp.id[to], sp.seg[to], sp.cnt[to], e->ws, e->ws_bytes,
                           nullptr, s);
   if (err != hipSuccess) return err;
   sp.cur = to;
-  sp.segi = lay_to;
+  sp.parity = src ? 0 : sp.parity ^ 1;
   e->sorts++;
   return hipSuccess;
 }
@@ -213,11 +212,11 @@ hipError_t sort_any(spic_engine *e, int is, void *const *src, hipStream_t s,
 }
 
 // The phase kernel's argument block for the loaded species of `e`, read
-// from buffer `cur` in layout `segi` (the species' own when negative).
+// from buffer `cur` (the species' own when negative).
 // idx[k] is the engine species of argument species k; returns the count.
 template <typename T>
 int fill_args(const spic_engine *e, const spic_field *field, const spic_moments *mom,
-              const spic_push *push, unsigned int *status, int cur, int segi,
+              const spic_push *push, unsigned int *status, int cur,
               spic::BinnedArgs<T> &a, int *idx) {
   std::memset(&a, 0, sizeof(a));
   a.g = spic::kgrid<T>(&e->grd);
@@ -247,7 +246,10 @@ int fill_args(const spic_engine *e, const spic_field *field, const spic_moments 
     t.stride = sp.cap;
     t.id_in = sp.id[in];
     t.id_out = sp.id[out];
-    t.seg = sp.seg[segi < 0 ? sp.segi : segi];
+    t.seg_in = sp.seg[in];
+    t.seg_out = sp.seg[out];
+    t.slack = sp.slack;
+    t.n = sp.n;
     t.cnt_in = sp.cnt[in];
     t.cnt_out = sp.cnt[out];
     t.ovf_cap = sp.ovf_cap;
@@ -272,7 +274,7 @@ hipError_t launch_phase(spic_engine *e, const spic_field *field,
                         unsigned int *status, hipStream_t s, int push_off = 0) {
   spic::BinnedArgs<T> a;
   int idx[spic::kMaxSpecies];
-  const int k = fill_args<T>(e, field, mom, push, status, -1, -1, a, idx);
+  const int k = fill_args<T>(e, field, mom, push, status, -1, a, idx);
   spic::BinnedReduceArgs r;
   std::memset(&r, 0, sizeof(r));
   spic::CountArrays zc;
@@ -281,6 +283,8 @@ hipError_t launch_phase(spic_engine *e, const spic_field *field,
     r.mom[j] = a.sp[j].m;
     zc.p[j] = a.sp[j].cnt_out;
     zc.mom[j] = a.sp[j].m;
+    zc.lay[j] = spic::LayoutArgs{a.sp[j].seg_in, a.sp[j].seg_out, a.sp[j].cnt_in, a.sp[j].slack,
+                                 a.sp[j].n};
   }
   r.ns = zc.ns = k;
   // writing the moments: zero them in the same launch; the deposits (LDS
@@ -298,9 +302,10 @@ hipError_t launch_phase(spic_engine *e, const spic_field *field,
   }
   if (zc.ns == 0) return hipSuccess;
   a.push_off = push_off;
-  zc.n = 3 * (e->L.ntiles + 1);
+  zc.ntiles = e->L.ntiles;
+  zc.n = spic::kCntArrays * (e->L.ntiles + 1);
   zc.nn = e->set_moments ? (int64_t)e->grd.nxn * e->grd.nyn * e->grd.nzn : 0;
-  hipError_t err = spic::zero_counts(zc, s);
+  hipError_t err = spic::phase_start(zc, s);
   if (err != hipSuccess || k == 0) return err;
   err = spic::strict_mode() ? spic::spic_strict::launch_binned_phase<T>(a, s)
                             : spic::spic_fast::launch_binned_phase<T>(a, s);
@@ -326,11 +331,11 @@ hipError_t store_bases(spic_engine *e, int is, const uint32_t **bases, hipStream
   const auto &sp = e->sp[is];
   if (sp.id[sp.cur]) return hipSuccess;
   size_t need = 0;
-  hipError_t err = spic::range_bases(sp.seg[sp.segi], sp.cnt[sp.cur], sp.ovf_cap, e->L.ntiles,
+  hipError_t err = spic::range_bases(sp.seg[sp.cur], sp.cnt[sp.cur], sp.ovf_cap, e->L.ntiles,
                                      nullptr, 0, &need, bases, s);
   if (err != hipSuccess) return err;
   if ((err = ensure_workspace(e, need, s)) != hipSuccess) return err;
-  return spic::range_bases(sp.seg[sp.segi], sp.cnt[sp.cur], sp.ovf_cap, e->L.ntiles, e->ws,
+  return spic::range_bases(sp.seg[sp.cur], sp.cnt[sp.cur], sp.ovf_cap, e->L.ntiles, e->ws,
                            e->ws_bytes, nullptr, bases, s);
 }
 
@@ -554,7 +559,8 @@ int spic_engine_load_as(spic_engine *e, int is, const spic_species *src, int pre
                (err = dmalloc(e, (void **)&sp.id[b], sizeof(uint32_t) * cap)) != hipSuccess)
         what = "engine id storage";
       else if ((err = dmalloc(e, (void **)&sp.cnt[b],
-                              sizeof(unsigned int) * 3 * (nt + 1))) != hipSuccess ||
+                              sizeof(unsigned int) * spic::kCntArrays * (nt + 1))) !=
+                   hipSuccess ||
                (err = dmalloc(e, (void **)&sp.seg[b], sizeof(int64_t) * (nt + 1))) !=
                    hipSuccess)
         what = "engine tile tables";
@@ -575,7 +581,7 @@ int spic_engine_load_as(spic_engine *e, int is, const spic_species *src, int pre
   sp.niter = src->NiterMover;
   sp.nsub = src->n_sub_cycles;
   sp.cur = 0;
-  sp.segi = 0;
+  sp.parity = 0;
   sp.loaded = true;
   e->gen++;
   void *srcs[7] = {src->x, src->y, src->z, src->u, src->v, src->w, src->q};
@@ -617,10 +623,10 @@ int spic_engine_store_as(spic_engine *e, int is, spic_species *dst, int prec,
   if (err == hipSuccess)
     err = e->esz == 8
               ? spic::bin_store<double>(e->L, (double *const *)sp.buf[sp.cur], sp.id[sp.cur],
-                                        bases, sp.seg[sp.segi], sp.cnt[sp.cur], sp.ovf_cap,
+                                        bases, sp.seg[sp.cur], sp.cnt[sp.cur], sp.ovf_cap,
                                         dsts, f64, s)
               : spic::bin_store<float>(e->L, (float *const *)sp.buf[sp.cur], sp.id[sp.cur],
-                                       bases, sp.seg[sp.segi], sp.cnt[sp.cur], sp.ovf_cap,
+                                       bases, sp.seg[sp.cur], sp.cnt[sp.cur], sp.ovf_cap,
                                        dsts, f64, s);
   if (err == hipSuccess && !spic::async_mode()) err = hipStreamSynchronize(s);
   return err == hipSuccess ? SPIC_OK : hip_fail(err, "engine store");
@@ -647,10 +653,10 @@ int spic_engine_snapshot_be32(spic_engine *e, int is, void *const dst[6], void *
   if (err == hipSuccess)
     err = e->esz == 8
               ? spic::bin_store_be32<double>(e->L, (double *const *)sp.buf[sp.cur],
-                                             sp.id[sp.cur], bases, sp.seg[sp.segi],
+                                             sp.id[sp.cur], bases, sp.seg[sp.cur],
                                              sp.cnt[sp.cur], sp.ovf_cap, d, s)
               : spic::bin_store_be32<float>(e->L, (float *const *)sp.buf[sp.cur],
-                                            sp.id[sp.cur], bases, sp.seg[sp.segi],
+                                            sp.id[sp.cur], bases, sp.seg[sp.cur],
                                             sp.cnt[sp.cur], sp.ovf_cap, d, s);
   if (err == hipSuccess && !spic::async_mode()) err = hipStreamSynchronize(s);
   return err == hipSuccess ? SPIC_OK : hip_fail(err, "engine snapshot");
@@ -781,15 +787,15 @@ struct spic_batch {
   // status buffer
   uint64_t gen[spic::kMaxInstances] = {};
   unsigned int *status = nullptr;
-  // device: four tables of n argument blocks, one per (layout, buffer)
-  // state: table (segi * 2 + cur)
+  // device: two tables of n argument blocks, one per buffer the particles
+  // are in
   void *tab = nullptr;
   size_t arg_bytes = 0;
   spic::BatchMap nodes{}, counts{};
   int max_ns = 0;
   // re-sorts of the whole batch in four launches when every member sorts
   // by tile sort: device tables of the jobs (member species with
-  // particles) per (layout, buffer) state, their block map, and the jobs'
+  // particles) per buffer they are in, their block map, and the jobs'
   // count / own / fill words
   bool tile_sorts = false;
   void *sort_tab = nullptr;
@@ -828,7 +834,7 @@ hipError_t build_items(spic_batch *b) {
       if (!sp.loaded || sp.n == 0) continue;
       any = true;
       seg.resize((size_t)nt + 1);
-      hipError_t err = hipMemcpy(seg.data(), sp.seg[sp.segi], sizeof(int64_t) * (nt + 1),
+      hipError_t err = hipMemcpy(seg.data(), sp.seg[sp.cur], sizeof(int64_t) * (nt + 1),
                                  hipMemcpyDeviceToHost);
       if (err != hipSuccess) return err;
       for (int t = 0; t < nt; ++t) load[t] += seg[t + 1] - seg[t];
@@ -870,19 +876,19 @@ hipError_t build_items(spic_batch *b) {
 template <typename T>
 hipError_t build_tables(spic_batch *b, unsigned int *status) {
   const size_t nb = sizeof(spic::BinnedArgs<T>);
-  std::vector<spic::BinnedArgs<T>> host(4 * (size_t)b->n);
+  std::vector<spic::BinnedArgs<T>> host(2 * (size_t)b->n);
   b->max_ns = 0;
-  for (int st = 0; st < 4; ++st)
+  for (int st = 0; st < 2; ++st)
     for (int i = 0; i < b->n; ++i) {
       const int k = fill_args<T>(b->e[i], &b->field[i], b->mom[i], &b->push[i], status,
-                                 st & 1, st >> 1, host[(size_t)st * b->n + i], nullptr);
+                                 st, host[(size_t)st * b->n + i], nullptr);
       if (k > b->max_ns) b->max_ns = k;
     }
   hipError_t err;
   if (!b->tab) {
-    if ((err = hipMalloc(&b->tab, 4 * nb * b->n)) != hipSuccess) return err;
+    if ((err = hipMalloc(&b->tab, 2 * nb * b->n)) != hipSuccess) return err;
   }
-  if ((err = hipMemcpy(b->tab, host.data(), 4 * nb * b->n, hipMemcpyHostToDevice)) !=
+  if ((err = hipMemcpy(b->tab, host.data(), 2 * nb * b->n, hipMemcpyHostToDevice)) !=
       hipSuccess)
     return err;
   b->arg_bytes = nb;
@@ -894,10 +900,10 @@ hipError_t build_tables(spic_batch *b, unsigned int *status) {
     const bool any = host[i].ns > 0;
     const int64_t nn = (int64_t)e->grd.nxn * e->grd.nyn * e->grd.nzn;
     b->nodes.start[i + 1] = b->nodes.start[i] + (any ? blocks(nn, 256) : 0);
-    const int64_t ncnt = 3 * (int64_t)(e->L.ntiles + 1);
+    const int64_t ncnt = spic::kCntArrays * (int64_t)(e->L.ntiles + 1);
     const int64_t zeroed =
         (b->flags & SPIC_BATCH_SET_MOMENTS) && nn > ncnt ? nn : ncnt;
-    b->counts.start[i + 1] = b->counts.start[i] + (any ? blocks(zeroed, 256) : 0);
+    b->counts.start[i + 1] = b->counts.start[i] + (any ? 1 + blocks(zeroed, 256) : 0);
     b->gen[i] = e->gen;
   }
   b->status = status;
@@ -931,10 +937,10 @@ hipError_t build_tables(spic_batch *b, unsigned int *status) {
   }
   b->sort_ws_words = words;
   if (!b->sort_tab) {
-    if ((err = hipMalloc(&b->sort_tab, 4 * kMaxJobs * jb)) != hipSuccess) return err;
+    if ((err = hipMalloc(&b->sort_tab, 2 * kMaxJobs * jb)) != hipSuccess) return err;
   }
-  std::vector<spic::TileSortJob<T>> jobs(4 * (size_t)kMaxJobs);
-  for (int st = 0; st < 4; ++st) {
+  std::vector<spic::TileSortJob<T>> jobs(2 * (size_t)kMaxJobs);
+  for (int st = 0; st < 2; ++st) {
     size_t off = 0;
     int j = 0;
     for (int i = 0; i < b->n; ++i) {
@@ -942,13 +948,13 @@ hipError_t build_tables(spic_batch *b, unsigned int *status) {
       for (int is = 0; is < e->ns; ++is) {
         if (!e->sp[is].loaded || e->sp[is].n == 0) continue;
         jobs[(size_t)st * kMaxJobs + j] =
-            tile_sort_job<T>(e, is, st & 1, st >> 1, b->sort_ws + off);
+            tile_sort_job<T>(e, is, st, b->sort_ws + off);
         off += 3 * ((size_t)e->L.ntiles + 1);
         ++j;
       }
     }
   }
-  if ((err = hipMemcpy(b->sort_tab, jobs.data(), 4 * kMaxJobs * jb,
+  if ((err = hipMemcpy(b->sort_tab, jobs.data(), 2 * kMaxJobs * jb,
                        hipMemcpyHostToDevice)) != hipSuccess)
     return err;
   b->job_bytes = jb;
@@ -962,7 +968,7 @@ hipError_t launch_batch_tile_sort(spic_batch *b, int state, hipStream_t s) {
   constexpr int kMaxJobs = spic::kMaxInstances * spic::kMaxSpecies;
   const spic::TileSortJob<T> *jobs =
       (const spic::TileSortJob<T> *)((char *)b->sort_tab +
-                                     (size_t)state * kMaxJobs * b->job_bytes);
+                                     (size_t)(state & 1) * kMaxJobs * b->job_bytes);
   const spic::BinLayout &L = b->e[0]->L;
   return spic::tile_sort_batch<T>(jobs, b->sort_map, L.tx, L.ty, L.tz, b->sort_ws,
                                   b->sort_ws_words, s);
@@ -990,10 +996,10 @@ hipError_t zero_empty_batch_moments(const spic_batch *b, hipStream_t s) {
 template <typename T>
 hipError_t launch_batch(spic_batch *b, int state, hipStream_t s) {
   const spic::BinnedArgs<T> *tab =
-      (const spic::BinnedArgs<T> *)((char *)b->tab + (size_t)state * b->n * b->arg_bytes);
+      (const spic::BinnedArgs<T> *)((char *)b->tab + (size_t)(state & 1) * b->n * b->arg_bytes);
   const spic::BinLayout &L = b->e[0]->L;
   const int set = (b->flags & SPIC_BATCH_SET_MOMENTS) ? 1 : 0;
-  hipError_t err = spic::launch_batch_zero_counts<T>(tab, b->counts, b->max_ns, set, s);
+  hipError_t err = spic::launch_batch_start<T>(tab, b->counts, b->max_ns, set, s);
   if (err == hipSuccess && set) err = zero_empty_batch_moments(b, s);
   if (err != hipSuccess) return err;
   // every instance's tiles and overflow parts in one persistent launch
@@ -1079,7 +1085,8 @@ int spic_batch_phase(spic_batch *b, void *stream) {
   if (int prc = check_positions(b->e[0])) return prc;
   hipStream_t s = (hipStream_t)stream;
   hipError_t err;
-  // every loaded species of the batch must be in one (layout, buffer) state
+  // every loaded species of the batch must be in the same one of its buffers,
+  // after as many re-sorts
   int state = -1;
   bool stale = false;
   for (int i = 0; i < b->n; ++i) {
@@ -1091,7 +1098,7 @@ int spic_batch_phase(spic_batch *b, void *stream) {
       if (!b->mom[i][is].rhon)
         return fail(SPIC_EINVAL, "batch member %d: species %d loaded after the batch "
                                  "was created without moments", i, is);
-      const int st = sp.segi * 2 + sp.cur;
+      const int st = sp.parity * 2 + sp.cur;
       if (state < 0) state = st;
       else if (st != state)
         return fail(SPIC_EINVAL,
@@ -1131,14 +1138,14 @@ int spic_batch_phase(spic_batch *b, void *stream) {
         auto &sp = e->sp[is];
         if (!sp.loaded || sp.n == 0) continue;
         sp.cur = 1 - sp.cur;
-        sp.segi = 1 - sp.segi;
+        sp.parity ^= 1;
         e->sorts++;
       }
     }
     state ^= 3;
   } else if (sort_now) {
-    // A sort moves each species to the other buffer and the other layout;
-    // members in step stay in one state.
+    // A sort moves each species to the other buffer; members in step stay
+    // in step.
     int after = -1;
     for (int i = 0; i < b->n; ++i) {
       spic_engine *e = b->e[i];
@@ -1148,7 +1155,7 @@ int spic_batch_phase(spic_batch *b, void *stream) {
         if (!sp.loaded || sp.n == 0) continue;
         if ((err = sort_any(e, is, nullptr, s)) != hipSuccess)
           return hip_fail(err, "batch sort");
-        const int st2 = sp.segi * 2 + sp.cur;
+        const int st2 = sp.parity * 2 + sp.cur;
         if (after < 0) after = st2;
         else if (st2 != after)
           return fail(SPIC_EINVAL,
