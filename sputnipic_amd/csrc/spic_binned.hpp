@@ -308,7 +308,7 @@ hipError_t bin_sort(const KGrid<T> &g, const BinLayout &L, int64_t n,
 // particles are written densely in storage order, range t from base[t]
 // (range_bases).
 template <typename T>
-hipError_t bin_store(const BinLayout &L, T *const src[7], const uint32_t *id,
+hipError_t bin_store(const BinLayout &L, int64_t n, T *const src[7], const uint32_t *id,
                      const uint32_t *base, const int64_t *seg, const unsigned int *cnt,
                      unsigned int ovf_cap, void *const dst[7], int dst_f64, hipStream_t s);
 
@@ -373,7 +373,7 @@ hipError_t tile_sort_batch(const TileSortJob<T> *jobs, const TileSortMap &map, i
 // bin_store of x y z u v w only, as big-endian IEEE float32 words (values
 // rounded to float): the particle datasets of a snapshot.
 template <typename T>
-hipError_t bin_store_be32(const BinLayout &L, T *const src[7], const uint32_t *id,
+hipError_t bin_store_be32(const BinLayout &L, int64_t n, T *const src[7], const uint32_t *id,
                           const uint32_t *base, const int64_t *seg, const unsigned int *cnt,
                           unsigned int ovf_cap, uint32_t *const dst[6], hipStream_t s);
 

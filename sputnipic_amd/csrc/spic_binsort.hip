@@ -11,7 +11,9 @@
 // 4 * cells-per-tile consecutive particles holds about four per cell: the
 // phase kernel sums one such run per batch cell by cell, and
 // particles that stay in their tile keep this order from phase to phase.
-// A stable LSD radix sort (rocPRIM) of (key, source slot) pairs gives the
+// A load from the caller's arrays gets there by tiles (counts, places and one
+// workgroup per tile); its largest tiles, and a binned source, by a stable LSD
+// radix sort (rocPRIM) of (key, source slot) pairs, whose result is the
 // permutation; the seven arrays and the particle id are gathered to sorted
 // position i + tile * slack, so that every segment gets `slack` free slots
 // after its particles.  A binned source is enumerated densely through an
@@ -22,6 +24,7 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include "spic_binned.hpp"
+#include "spic_wave.hpp"
 
 namespace spic {
 namespace {
@@ -186,10 +189,6 @@ struct Arrays7 {
   T *p[7];
 };
 
-struct Words6 {
-  uint32_t *p[6];
-};
-
 // The sorted gather into binned storage.  A dense source (src_id null)
 // holds the caller's values in TS: with fixed-point storage (to_fixed) its
 // positions are converted, the rest rounded to T; a binned source is the
@@ -215,6 +214,232 @@ __global__ void k_bin_gather(Arrays7<TS> src, const uint32_t *__restrict__ src_i
       dst.p[a][o] = (T)src.p[a][j];
     }
     if (dst_id) dst_id[o] = src_id ? src_id[j] : j;
+  }
+}
+
+// ---- load through tiles ----------------------------------------------------
+//
+// A dense source is counted into tiles, its indices are placed tile by tile,
+// and one workgroup per tile ranks its particles per cell and gathers them in
+// round-robin order.  4.0M FP64 particles that have drifted two cells from
+// their cell order: 262 us (gather 193, the rest counts and places) against
+// 735 us for keys, radix sort and gather.  Most of a line's particles then lie
+// in different tiles: 490 MB are fetched for 232 MB of particles, 3.7 TB/s in
+// all.  Gathering component by component over all tiles instead fetches 797 MB
+// (281 us).  Tiles of more than kLoadHeld particles on average keep the radix
+// sort, whose work does not depend on the number of tiles.
+constexpr int kLoadThreads = 1024;
+constexpr int kLoadPer = 8;      // particles per thread that a tile's workgroup holds
+constexpr int kLoadHeld = kLoadThreads * kLoadPer;
+constexpr int kLoadStage = 4096;  // values staged in LDS at a time
+constexpr int kLoadRanks = 128;   // ranks in the slot tables
+constexpr int kStoreThreads = 512;
+constexpr int kStorePer = 8;
+constexpr int kStoreHeld = kStoreThreads * kStorePer;
+constexpr int kStoreLines = 512;  // line counters of a store
+// Particles per tile from which a store groups them by line: with 128 a
+// workgroup is mostly idle (230k FP64 particles: 25 us grouped, 19 direct), 512
+// take 13.0 against 14.6, 1728 237 against 534 (3.1M).
+constexpr int kStoreMinTile = 512;
+
+struct LoadBins {
+  int64_t n;
+  int per;                 // particles per thread of the count
+  unsigned int *count;     // [ntiles] particles per tile
+  unsigned int *next;      // [ntiles] places taken in each tile
+  const int64_t *seg;      // the segments: tile t's places begin at seg[t] - t * slack
+  uint32_t *where;         // [n] tile | cell in the tile (cell_bits)
+  uint32_t *perm;          // [n] by place: index of the particle
+};
+
+// Counts the particles into tiles: up to kLdsTiles tiles (IN_LDS) a workgroup
+// counts in LDS and adds each tile it met once.
+template <typename TS, typename T, bool IN_LDS>
+__global__ __launch_bounds__(256) void k_load_count(KGrid<T> g, BinLayout L, LoadBins b,
+                                                    const TS *__restrict__ x,
+                                                    const TS *__restrict__ y,
+                                                    const TS *__restrict__ z) {
+  __shared__ unsigned int s_cnt[IN_LDS ? kLdsTiles : 1];
+  const int tid = threadIdx.x;
+  if constexpr (IN_LDS) {
+    for (int t = tid; t < L.ntiles; t += 256) s_cnt[t] = 0u;
+    __syncthreads();
+  }
+  const int64_t first = blockIdx.x * (int64_t)(256 * b.per);
+  for (int e = 0; e < b.per; ++e) {
+    const int64_t i = first + e * 256 + tid;
+    const bool active = i < b.n;
+    uint32_t tile = 0, cit = 0;
+    if (active) {
+      int cx, cy, cz;
+      cell_of(g, L, x[i], y[i], z[i], cx, cy, cz, tile, cit, false);
+      b.where[i] = (tile << L.cell_bits) | cit;
+    }
+    key_rank(IN_LDS ? s_cnt : b.count, tile, active);
+  }
+  if constexpr (IN_LDS) {
+    __syncthreads();
+    for (int t = tid; t < L.ntiles; t += 256)
+      if (s_cnt[t]) atomicAdd(b.count + t, s_cnt[t]);
+  }
+}
+
+// Places each particle's index in its tile: each tile's places at once per
+// workgroup (IN_LDS), PER particles per thread, or per wave.
+template <int PER, bool IN_LDS>
+__global__ __launch_bounds__(256) void k_load_place(BinLayout L, LoadBins b) {
+  __shared__ unsigned int s_cnt[IN_LDS ? kLdsTiles : 1];
+  const int tid = threadIdx.x;
+  const int64_t first = blockIdx.x * (int64_t)(256 * PER);
+  unsigned int t[PER], r[PER];
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    const int64_t i = first + e * 256 + tid;
+    t[e] = i < b.n ? b.where[i] >> L.cell_bits : 0u;
+  }
+  if constexpr (IN_LDS) {
+    for (int k = tid; k < L.ntiles; k += 256) s_cnt[k] = 0u;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int e = 0; e < PER; ++e)
+    r[e] = key_rank(IN_LDS ? s_cnt : b.next, t[e], first + e * 256 + tid < b.n);
+  if constexpr (IN_LDS) {
+    __syncthreads();
+    for (int k = tid; k < L.ntiles; k += 256)
+      if (s_cnt[k]) s_cnt[k] = atomicAdd(b.next + k, s_cnt[k]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    const int64_t i = first + e * 256 + tid;
+    if (i < b.n)
+      b.perm[b.seg[t[e]] - (int64_t)t[e] * L.slack + (IN_LDS ? s_cnt[t[e]] : 0u) + r[e]] =
+          (uint32_t)i;
+  }
+}
+
+// A caller's value into binned storage: with fixed-point storage positions
+// are converted, everything else is rounded to T.
+template <typename TS, typename T>
+__device__ __forceinline__ T load_value(TS v, int a, int fixed, const FixedParams &fx) {
+  if constexpr (sizeof(T) == 4) {
+    if (a < 3 && fixed) return __int_as_float(to_fixed_pos((double)v, fx, a));
+  }
+  return (T)v;
+}
+
+// One workgroup per tile, tiles in runs per XCD: counts its cells, turns each
+// particle's rank within its cell into its slot in round-robin order (slot of
+// the k-th particle of cell c: particles of rank < k over all cells, plus the
+// cells before c that hold more than k; tables up to kLoadRanks ranks, a loop
+// over the cells beyond), then takes the components one after another: read in
+// the order of the places, where neighbours of the caller's arrays are mostly
+// neighbours, put at their slots in LDS and written in order.  A tile of more
+// than kLoadHeld particles ranks them in a second sweep and writes each at its
+// slot.
+template <typename TS, typename T, int NC>
+__global__ __launch_bounds__(kLoadThreads) __attribute__((amdgpu_waves_per_eu(8)))
+void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint32_t *dst_id) {
+  __shared__ unsigned int s_count[NC], s_rank[NC], s_A[kLoadRanks];
+  __shared__ unsigned char s_T[NC][kLoadRanks];
+  __shared__ T s_stage[kLoadStage];
+  const int t = (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
+  if (t >= L.ntiles) return;
+  const int tid = threadIdx.x;
+  const int64_t n64 = b.count[t], out0 = b.seg[t];
+  if (n64 == 0) return;
+  const uint32_t *perm = b.perm + (out0 - (int64_t)t * L.slack);
+  const uint32_t mask = (1u << L.cell_bits) - 1u;
+  const bool held = n64 <= kLoadHeld;
+  const int n = held ? (int)n64 : 0;
+  for (int c = tid; c < NC; c += kLoadThreads) s_count[c] = s_rank[c] = 0u;
+  __syncthreads();
+  uint32_t j[kLoadPer], pos[kLoadPer];  // index; rank and cell, then slot
+  if (held) {
+#pragma unroll
+    for (int e = 0; e < kLoadPer; ++e) {
+      const int r = e * kLoadThreads + tid;
+      if (r < n) j[e] = perm[r];
+    }
+#pragma unroll
+    for (int e = 0; e < kLoadPer; ++e)
+      if (e * kLoadThreads + tid < n) pos[e] = b.where[j[e]] & mask;
+#pragma unroll
+    for (int e = 0; e < kLoadPer; ++e)
+      if (e * kLoadThreads + tid < n) pos[e] |= atomicAdd(&s_count[pos[e]], 1u) << 8;
+  } else {
+    for (int64_t r = tid; r < n64; r += kLoadThreads)
+      atomicAdd(&s_count[b.where[perm[r]] & mask], 1u);
+  }
+  __syncthreads();
+  if (tid < kLoadRanks) {
+    unsigned int a = 0, before = 0;
+#pragma unroll 8
+    for (int c = 0; c < NC; ++c) {
+      const unsigned int m = s_count[c];
+      a += m < (unsigned)tid ? m : (unsigned)tid;
+      s_T[c][tid] = (unsigned char)before;
+      before += m > (unsigned)tid ? 1u : 0u;
+    }
+    s_A[tid] = a;
+  }
+  __syncthreads();
+  auto slot = [&](unsigned int c, unsigned int k) -> unsigned int {
+    if (k < (unsigned)kLoadRanks) return s_A[k] + s_T[c][k];
+    unsigned int p = 0;
+#pragma unroll 4
+    for (int cc = 0; cc < NC; ++cc) {
+      const unsigned int m = s_count[cc];
+      p += m < k ? m : k;
+      if (cc < (int)c && m > k) ++p;
+    }
+    return p;
+  };
+  if (!held) {
+    for (int64_t r = tid; r < n64; r += kLoadThreads) {
+      const uint32_t i = perm[r], c = b.where[i] & mask;
+      const int64_t o = out0 + slot(c, atomicAdd(&s_rank[c], 1u));
+#pragma unroll
+      for (int a = 0; a < 7; ++a)
+        dst.p[a][o] = load_value<TS, T>(src.p[a][i], a, L.fixed, L.fx);
+      if (dst_id) dst_id[o] = i;
+    }
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < kLoadPer; ++e)
+    if (e * kLoadThreads + tid < n) pos[e] = slot(pos[e] & 0xffu, pos[e] >> 8);
+#pragma unroll
+  for (int a = 0; a < 7; ++a) {
+    T val[kLoadPer];
+#pragma unroll
+    for (int e = 0; e < kLoadPer; ++e)
+      if (e * kLoadThreads + tid < n)
+        val[e] = load_value<TS, T>(src.p[a][j[e]], a, L.fixed, L.fx);
+    T *__restrict__ to = dst.p[a] + out0;
+    for (int c0 = 0; c0 < n; c0 += kLoadStage) {
+#pragma unroll
+      for (int e = 0; e < kLoadPer; ++e)
+        if (e * kLoadThreads + tid < n && pos[e] - c0 < (unsigned)kLoadStage)
+          s_stage[pos[e] - c0] = val[e];
+      __syncthreads();
+      const int m = min(n - c0, kLoadStage);
+      for (int p = tid; p < m; p += kLoadThreads) to[c0 + p] = s_stage[p];
+      __syncthreads();
+    }
+  }
+  if (!dst_id) return;
+  uint32_t *s_id = reinterpret_cast<uint32_t *>(s_stage);
+  for (int c0 = 0; c0 < n; c0 += kLoadStage) {
+#pragma unroll
+    for (int e = 0; e < kLoadPer; ++e)
+      if (e * kLoadThreads + tid < n && pos[e] - c0 < (unsigned)kLoadStage)
+        s_id[pos[e] - c0] = j[e];
+    __syncthreads();
+    const int m = min(n - c0, kLoadStage);
+    for (int p = tid; p < m; p += kLoadThreads) dst_id[out0 + c0 + p] = s_id[p];
+    __syncthreads();
   }
 }
 
@@ -244,59 +469,140 @@ __global__ void k_bin_bounds(const uint32_t *__restrict__ keys, int shift, int64
   }
 }
 
-// One workgroup per segment (then the overflow region): dst[id] = src, in
-// the caller's element type TD; fixed-point positions converted back.
-template <typename T, typename TD>
-__global__ void k_bin_store(Arrays7<T> src, const uint32_t *__restrict__ id,
-                            const uint32_t *__restrict__ base,
-                            const int64_t *__restrict__ seg,
-                            const unsigned int *__restrict__ cnt,
-                            unsigned int ovf_cap, int ntiles, Arrays7<TD> dst, int fixed,
-                            FixedParams fx) {
-  const RangeView v = range_view(seg, cnt, ntiles, ovf_cap, (int)blockIdx.x);
-  for (int64_t r = threadIdx.x; r < v.count; r += blockDim.x) {
-    const int64_t i = v.slot(r);
-    const uint32_t k = id ? id[i] : base[blockIdx.x] + (uint32_t)r;
-#pragma unroll
-    for (int a = 0; a < 7; ++a) {
-      if constexpr (sizeof(T) == 4) {
-        if (a < 3 && fixed) {
-          dst.p[a][k] = (TD)from_fixed_pos(__float_as_int((float)src.p[a][i]), fx, a);
-          continue;
-        }
-      }
-      dst.p[a][k] = (TD)src.p[a][i];
-    }
-  }
-}
-
 // Big-endian IEEE float32 bits of v rounded to float (H5T_IEEE_F32BE).
 template <typename T>
 __device__ __forceinline__ uint32_t be32(T v) {
   return __builtin_bswap32(__float_as_uint((float)v));
 }
 
-// bin_store's scatter to load order, writing x y z u v w as big-endian
-// float32: the datasets of a particle snapshot.
-template <typename T>
-__global__ void k_bin_store_be32(Arrays7<T> src, const uint32_t *__restrict__ id,
-                                 const uint32_t *__restrict__ base,
-                                 const int64_t *__restrict__ seg,
-                                 const unsigned int *__restrict__ cnt, unsigned int ovf_cap,
-                                 int ntiles, Words6 dst, int fixed, FixedParams fx) {
+// A stored value out of binned storage in the caller's element type TD:
+// fixed-point positions converted back; with NA = 6 (a snapshot) as big-endian
+// float32 words.
+template <typename T, typename TD, int NA>
+__device__ __forceinline__ TD store_value(T v, int a, int fixed, const FixedParams &fx) {
+  if constexpr (sizeof(T) == 4) {
+    if (a < 3 && fixed) {
+      const double p = from_fixed_pos(__float_as_int((float)v), fx, a);
+      if constexpr (NA == 6) return be32(p);
+      else return (TD)p;
+    }
+  }
+  if constexpr (NA == 6) return be32(v);
+  else return (TD)v;
+}
+
+// Each particle of a segment (one workgroup each, then the overflow region)
+// straight to its place: dst[id] = src, or, in an engine without ids, densely
+// in storage order.
+template <typename T, typename TD, int NA>
+__global__ __launch_bounds__(256) void k_bin_store(
+    Arrays7<T> src, const uint32_t *__restrict__ id, const uint32_t *__restrict__ base,
+    const int64_t *__restrict__ seg, const unsigned int *__restrict__ cnt,
+    unsigned int ovf_cap, int ntiles, Arrays7<TD> dst, int fixed, FixedParams fx) {
   const RangeView v = range_view(seg, cnt, ntiles, ovf_cap, (int)blockIdx.x);
-  for (int64_t r = threadIdx.x; r < v.count; r += blockDim.x) {
+  for (int64_t r = threadIdx.x; r < v.count; r += 256) {
     const int64_t i = v.slot(r);
     const uint32_t k = id ? id[i] : base[blockIdx.x] + (uint32_t)r;
 #pragma unroll
-    for (int a = 0; a < 6; ++a) {
-      if constexpr (sizeof(T) == 4) {
-        if (a < 3 && fixed) {
-          dst.p[a][k] = be32(from_fixed_pos(__float_as_int((float)src.p[a][i]), fx, a));
-          continue;
-        }
+    for (int a = 0; a < NA; ++a)
+      dst.p[a][k] = store_value<T, TD, NA>(src.p[a][i], a, fixed, fx);
+  }
+}
+
+// One workgroup per segment (then the overflow region), in runs per XCD:
+// dst[id] = src.  Particles of one line of the caller's arrays lie all over
+// the segment (round-robin over the cells); written in storage order, a line
+// goes out in parts, one per particle.  Here up to kStoreHeld particles are
+// grouped by that line first (counts by line modulo kStoreLines, a scan, a
+// placement), then the components follow one another: read in storage order,
+// put at their places in LDS, written line by line.  4.0M FP64 particles, two
+// cells from their cell order: 300 us against 601 straight to their places
+// (particles of a line that lie in other tiles still make partial writes: 706
+// MB go out for 224 MB).  Not faster: slots inverted first and the particles
+// read at them in load order, 378 us; component by component over all tiles,
+// 469; 1024 threads for up to 8192 particles, 294 to 312 with spills.
+template <typename T, typename TD, int NA>
+__global__ __launch_bounds__(kStoreThreads) __attribute__((amdgpu_waves_per_eu(6)))
+void k_store_tile(Arrays7<T> src, const uint32_t *__restrict__ id,
+                  const int64_t *__restrict__ seg, const unsigned int *__restrict__ cnt,
+                  unsigned int ovf_cap, int ntiles, Arrays7<TD> dst, int fixed,
+                  FixedParams fx) {
+  constexpr unsigned int kLine = 128 / sizeof(TD);
+  __shared__ unsigned int s_line[kStoreLines];
+  __shared__ unsigned int s_wave[kStoreLines / 64];
+  __shared__ uint32_t s_id[kStoreHeld];
+  __shared__ T s_stage[kStoreHeld];
+  __shared__ const T *s_from[NA];
+  __shared__ TD *s_to[NA];
+  static_assert(kStoreLines == kStoreThreads, "a thread per counter");
+  const int t = (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
+  if (t > ntiles) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const RangeView v = range_view(seg, cnt, ntiles, ovf_cap, t);
+  if (tid < NA) {
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+      if (tid == a) {
+        s_from[a] = src.p[a] + v.first;
+        s_to[a] = dst.p[a];
       }
-      dst.p[a][k] = be32(src.p[a][i]);
+  }
+  // a slot's offset within the range fits 32 bits
+  auto at = [&v](uint32_t r) { return r < v.gap_lo ? r : r + v.gap_len; };
+  const uint32_t count = (uint32_t)v.count;
+  for (uint32_t first = 0; first < count; first += kStoreHeld) {
+    const int n = (int)min(count - first, (uint32_t)kStoreHeld);
+    s_line[tid] = 0u;
+    __syncthreads();
+    uint32_t k[kStorePer], pos[kStorePer];
+#pragma unroll
+    for (int e = 0; e < kStorePer; ++e) {
+      const int r = e * kStoreThreads + tid;
+      if (r < n) k[e] = (id + v.first)[at(first + r)];
+    }
+#pragma unroll
+    for (int e = 0; e < kStorePer; ++e)
+      if (e * kStoreThreads + tid < n)
+        pos[e] = atomicAdd(&s_line[k[e] / kLine % kStoreLines], 1u);
+    __syncthreads();
+    const unsigned int c = s_line[tid];
+    unsigned int sum = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned int u = __shfl_up(sum, d);
+      if (lane >= d) sum += u;
+    }
+    if (lane == 63) s_wave[tid >> 6] = sum;
+    __syncthreads();
+    sum -= c;
+    for (int w = 0; w < (tid >> 6); ++w) sum += s_wave[w];
+    s_line[tid] = sum;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kStorePer; ++e)
+      if (e * kStoreThreads + tid < n) {
+        pos[e] += s_line[k[e] / kLine % kStoreLines];
+        s_id[pos[e]] = k[e];
+      }
+    // a loop of its own per component: unrolled, the loads of the next ones
+    // are moved ahead and spill
+#pragma unroll 1
+    for (int a = 0; a < NA; ++a) {
+      const SPIC_GLOBAL T *from = gmem(s_from[a]);
+      SPIC_GLOBAL TD *to = gmem(s_to[a]);
+      T val[kStorePer];
+#pragma unroll
+      for (int e = 0; e < kStorePer; ++e) {
+        const int r = e * kStoreThreads + tid;
+        if (r < n) val[e] = from[at(first + r)];
+      }
+#pragma unroll
+      for (int e = 0; e < kStorePer; ++e)
+        if (e * kStoreThreads + tid < n) s_stage[pos[e]] = val[e];
+      __syncthreads();
+      for (int p = tid; p < n; p += kStoreThreads)
+        to[s_id[p]] = store_value<T, TD, NA>(s_stage[p], a, fixed, fx);
+      __syncthreads();
     }
   }
 }
@@ -1000,6 +1306,70 @@ hipError_t phase_start(const CountArrays &c, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The load of a dense source through tiles.  Workspace: three words per tile,
+// two per particle.
+template <typename TS, typename T>
+hipError_t load_tiles(const KGrid<T> &g, const BinLayout &L, int64_t n, const void *const src[7],
+                      T *const dst[7], uint32_t *dst_id, int64_t *dst_seg,
+                      unsigned int *dst_cnt, char *w, size_t a_t, size_t a_n, hipStream_t s) {
+  const int nc = L.tx * L.ty * L.tz;
+  if (nc != 64 && nc != 128) return hipErrorInvalidValue;
+  TileSortJob<T> J;
+  std::memset(&J, 0, sizeof(J));
+  J.L = L;
+  J.dst_seg = dst_seg;
+  J.dst_cnt = dst_cnt;
+  J.count = (unsigned int *)w;
+  LoadBins b;
+  b.n = n;
+  b.count = J.count;
+  b.next = J.count + L.ntiles + 1;
+  b.seg = dst_seg;
+  b.where = (uint32_t *)(w + a_t);
+  b.perm = (uint32_t *)(w + a_t + a_n);
+  const int64_t per = n / (256 * 2048);
+  b.per = per < 1 ? 1 : per > 16 ? 16 : (int)per;
+  Arrays7<TS> as;
+  Arrays7<T> ad;
+  for (int a = 0; a < 7; ++a) {
+    as.p[a] = (TS *)src[a];
+    ad.p[a] = dst[a];
+  }
+  const int64_t nzero = 2 * ((int64_t)L.ntiles + 1);
+  hipLaunchKernelGGL(k_zero_u32, dim3(nblocks(nzero)), dim3(256), 0, s, J.count, nzero);
+  hipError_t e;
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (n > 0) {
+    const dim3 grid((unsigned)((n + 256 * b.per - 1) / (256 * b.per)));
+    if (L.ntiles <= kLdsTiles && L.ntiles <= 8 * 256 * b.per)
+      hipLaunchKernelGGL((k_load_count<TS, T, true>), grid, dim3(256), 0, s, g, L, b, as.p[0],
+                         as.p[1], as.p[2]);
+    else
+      hipLaunchKernelGGL((k_load_count<TS, T, false>), grid, dim3(256), 0, s, g, L, b, as.p[0],
+                         as.p[1], as.p[2]);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k_tile_bounds<T>, dim3(1), dim3(kScanThreads), 0, s, J);
+  if ((e = hipGetLastError()) != hipSuccess || n == 0) return e;
+  // places by workgroup or by wave, as the deposit through tiles takes them
+  auto blocks = [n](int per) { return dim3((unsigned)((n + 256 * per - 1) / (256 * per))); };
+  if (L.ntiles <= kLdsTiles && n >= 128 * 256 * 16)
+    hipLaunchKernelGGL((k_load_place<16, true>), blocks(16), dim3(256), 0, s, L, b);
+  else if (L.ntiles <= 4 * 256)
+    hipLaunchKernelGGL((k_load_place<4, true>), blocks(4), dim3(256), 0, s, L, b);
+  else
+    hipLaunchKernelGGL((k_load_place<1, false>), blocks(1), dim3(256), 0, s, L, b);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  const dim3 tiles((unsigned)((L.ntiles + 7) / 8 * 8));
+  if (nc == 64)
+    hipLaunchKernelGGL((k_load_tile<TS, T, 64>), tiles, dim3(kLoadThreads), 0, s, L, b, as, ad,
+                       dst_id);
+  else
+    hipLaunchKernelGGL((k_load_tile<TS, T, 128>), tiles, dim3(kLoadThreads), 0, s, L, b, as, ad,
+                       dst_id);
+  return hipGetLastError();
+}
+
 template <typename T>
 hipError_t bin_sort(const KGrid<T> &g, const BinLayout &L, int64_t n,
                     const void *const src[7], int src_f64, const uint32_t *src_id,
@@ -1020,6 +1390,17 @@ hipError_t bin_sort(const KGrid<T> &g, const BinLayout &L, int64_t n,
   const size_t a_c = align_up(sizeof(uint32_t) * (size_t)ncell);
   const int shift = L.rank_bits + L.cell_bits;
   const int key_bits = L.tile_bits + shift;
+  if (!binned && n <= (int64_t)kLoadHeld * L.ntiles) {
+    const size_t a_w = align_up(2 * sizeof(uint32_t) * nt1);
+    const size_t total = a_w + 2 * a_n;
+    if (needed) *needed = total;
+    if (!workspace) return hipSuccess;
+    if (workspace_bytes < total) return hipErrorInvalidValue;
+    return widened ? load_tiles<double, T>(g, L, n, src, dst, dst_id, dst_seg, dst_cnt,
+                                           (char *)workspace, a_w, a_n, s)
+                   : load_tiles<T, T>(g, L, n, src, dst, dst_id, dst_seg, dst_cnt,
+                                      (char *)workspace, a_w, a_n, s);
+  }
   size_t sort_bytes = 0, scan_bytes = 0;
   hipError_t e = rocprim::radix_sort_pairs(
       nullptr, sort_bytes, (uint32_t *)nullptr, (uint32_t *)nullptr,
@@ -1112,54 +1493,59 @@ template hipError_t bin_sort<float>(const KGrid<float> &, const BinLayout &, int
                                     int64_t *, unsigned int *, void *, size_t,
                                     size_t *, hipStream_t);
 
+namespace {
+
+template <typename T, typename TD, int NA>
+hipError_t store_any(const BinLayout &L, int64_t n, T *const src[7], const uint32_t *id,
+                     const uint32_t *base, const int64_t *seg, const unsigned int *cnt,
+                     unsigned int ovf_cap, void *const *dst, hipStream_t s) {
+  Arrays7<T> as;
+  Arrays7<TD> ad;
+  for (int a = 0; a < 7; ++a) as.p[a] = src[a];
+  for (int a = 0; a < 7; ++a) ad.p[a] = a < NA ? (TD *)dst[a] : nullptr;
+  if (id && n >= kStoreMinTile * (int64_t)L.ntiles)
+    hipLaunchKernelGGL((k_store_tile<T, TD, NA>), dim3((unsigned)(L.ntiles / 8 + 1) * 8),
+                       dim3(kStoreThreads), 0, s, as, id, seg, cnt, ovf_cap, L.ntiles, ad,
+                       L.fixed, L.fx);
+  else
+    hipLaunchKernelGGL((k_bin_store<T, TD, NA>), dim3(L.ntiles + 1), dim3(256), 0, s, as, id, base,
+                       seg, cnt, ovf_cap, L.ntiles, ad, L.fixed, L.fx);
+  return hipGetLastError();
+}
+
+}  // namespace
+
 template <typename T>
-hipError_t bin_store(const BinLayout &L, T *const src[7], const uint32_t *id,
+hipError_t bin_store(const BinLayout &L, int64_t n, T *const src[7], const uint32_t *id,
                      const uint32_t *base, const int64_t *seg, const unsigned int *cnt,
                      unsigned int ovf_cap, void *const dst[7], int dst_f64, hipStream_t s) {
-  Arrays7<T> as;
-  for (int a = 0; a < 7; ++a) as.p[a] = src[a];
-  if (dst_f64) {
-    Arrays7<double> ad;
-    for (int a = 0; a < 7; ++a) ad.p[a] = (double *)dst[a];
-    hipLaunchKernelGGL((k_bin_store<T, double>), dim3(L.ntiles + 1), dim3(256), 0, s, as, id,
-                       base, seg, cnt, ovf_cap, L.ntiles, ad, L.fixed, L.fx);
-  } else {
-    if (sizeof(T) == 8) return hipErrorInvalidValue;  // no narrowing store
-    Arrays7<float> ad;
-    for (int a = 0; a < 7; ++a) ad.p[a] = (float *)dst[a];
-    hipLaunchKernelGGL((k_bin_store<T, float>), dim3(L.ntiles + 1), dim3(256), 0, s, as, id,
-                       base, seg, cnt, ovf_cap, L.ntiles, ad, L.fixed, L.fx);
-  }
-  return hipGetLastError();
+  if (dst_f64) return store_any<T, double, 7>(L, n, src, id, base, seg, cnt, ovf_cap, dst, s);
+  if constexpr (sizeof(T) == 8) return hipErrorInvalidValue;  // no narrowing store
+  else return store_any<T, float, 7>(L, n, src, id, base, seg, cnt, ovf_cap, dst, s);
 }
 
 template <typename T>
-hipError_t bin_store_be32(const BinLayout &L, T *const src[7], const uint32_t *id,
+hipError_t bin_store_be32(const BinLayout &L, int64_t n, T *const src[7], const uint32_t *id,
                           const uint32_t *base, const int64_t *seg, const unsigned int *cnt,
                           unsigned int ovf_cap, uint32_t *const dst[6], hipStream_t s) {
-  Arrays7<T> as;
-  Words6 ad;
-  for (int a = 0; a < 7; ++a) as.p[a] = src[a];
-  for (int a = 0; a < 6; ++a) ad.p[a] = dst[a];
-  hipLaunchKernelGGL(k_bin_store_be32<T>, dim3(L.ntiles + 1), dim3(256), 0, s, as, id, base,
-                     seg, cnt, ovf_cap, L.ntiles, ad, L.fixed, L.fx);
-  return hipGetLastError();
+  return store_any<T, uint32_t, 6>(L, n, src, id, base, seg, cnt, ovf_cap, (void *const *)dst,
+                                   s);
 }
 
-template hipError_t bin_store_be32<double>(const BinLayout &, double *const[7],
+template hipError_t bin_store_be32<double>(const BinLayout &, int64_t, double *const[7],
                                            const uint32_t *, const uint32_t *, const int64_t *,
                                            const unsigned int *, unsigned int,
                                            uint32_t *const[6], hipStream_t);
-template hipError_t bin_store_be32<float>(const BinLayout &, float *const[7],
+template hipError_t bin_store_be32<float>(const BinLayout &, int64_t, float *const[7],
                                           const uint32_t *, const uint32_t *, const int64_t *,
                                           const unsigned int *, unsigned int,
                                           uint32_t *const[6], hipStream_t);
 
-template hipError_t bin_store<double>(const BinLayout &, double *const[7],
+template hipError_t bin_store<double>(const BinLayout &, int64_t, double *const[7],
                                       const uint32_t *, const uint32_t *, const int64_t *,
                                       const unsigned int *, unsigned int,
                                       void *const[7], int, hipStream_t);
-template hipError_t bin_store<float>(const BinLayout &, float *const[7],
+template hipError_t bin_store<float>(const BinLayout &, int64_t, float *const[7],
                                      const uint32_t *, const uint32_t *, const int64_t *,
                                      const unsigned int *, unsigned int,
                                      void *const[7], int, hipStream_t);

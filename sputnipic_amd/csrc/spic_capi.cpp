@@ -161,6 +161,16 @@ hipError_t stream_alloc(void **p, size_t bytes, hipStream_t s) {
 
 hipError_t stream_free(void *p, hipStream_t s) { return hipFreeAsync(p, s); }
 
+bool stream_may_alloc(hipStream_t s) {
+  if (s == nullptr) return true;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return cs == hipStreamCaptureStatusNone;
+}
+
 int check_grid(const spic_grid *g) {
   if (!g) return fail(SPIC_EINVAL, "grid is NULL");
   if (g->prec != SPIC_F64 && g->prec != SPIC_F32)

@@ -622,10 +622,10 @@ int spic_engine_store_as(spic_engine *e, int is, spic_species *dst, int prec,
   hipError_t err = store_bases(e, is, &bases, s);
   if (err == hipSuccess)
     err = e->esz == 8
-              ? spic::bin_store<double>(e->L, (double *const *)sp.buf[sp.cur], sp.id[sp.cur],
+              ? spic::bin_store<double>(e->L, sp.n, (double *const *)sp.buf[sp.cur], sp.id[sp.cur],
                                         bases, sp.seg[sp.cur], sp.cnt[sp.cur], sp.ovf_cap,
                                         dsts, f64, s)
-              : spic::bin_store<float>(e->L, (float *const *)sp.buf[sp.cur], sp.id[sp.cur],
+              : spic::bin_store<float>(e->L, sp.n, (float *const *)sp.buf[sp.cur], sp.id[sp.cur],
                                        bases, sp.seg[sp.cur], sp.cnt[sp.cur], sp.ovf_cap,
                                        dsts, f64, s);
   if (err == hipSuccess && !spic::async_mode()) err = hipStreamSynchronize(s);
@@ -652,10 +652,10 @@ int spic_engine_snapshot_be32(spic_engine *e, int is, void *const dst[6], void *
   hipError_t err = store_bases(e, is, &bases, s);
   if (err == hipSuccess)
     err = e->esz == 8
-              ? spic::bin_store_be32<double>(e->L, (double *const *)sp.buf[sp.cur],
+              ? spic::bin_store_be32<double>(e->L, sp.n, (double *const *)sp.buf[sp.cur],
                                              sp.id[sp.cur], bases, sp.seg[sp.cur],
                                              sp.cnt[sp.cur], sp.ovf_cap, d, s)
-              : spic::bin_store_be32<float>(e->L, (float *const *)sp.buf[sp.cur],
+              : spic::bin_store_be32<float>(e->L, sp.n, (float *const *)sp.buf[sp.cur],
                                             sp.id[sp.cur], bases, sp.seg[sp.cur],
                                             sp.cnt[sp.cur], sp.ovf_cap, d, s);
   if (err == hipSuccess && !spic::async_mode()) err = hipStreamSynchronize(s);

@@ -85,6 +85,8 @@ hipError_t sort_reference_order(const spic_grid &g, int64_t sort_cps,
 constexpr size_t kScratchKeep = size_t(512) << 20;
 hipError_t stream_alloc(void **p, size_t bytes, hipStream_t s);
 hipError_t stream_free(void *p, hipStream_t s);
+// Whether work on the stream may take such scratch: not while it is captured.
+bool stream_may_alloc(hipStream_t s);
 
 hipError_t zero_f64(double *p, size_t n, hipStream_t s);
 hipError_t zero_u32(unsigned int *p, size_t n, hipStream_t s);

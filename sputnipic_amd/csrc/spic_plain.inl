@@ -9,6 +9,7 @@
 // reference's operand types and order (src/Mover.cpp:4-162, 385-572), so an
 // FP64 or FP32 particle state matches the CPU reference bit for bit.
 #include "spic_internal.hpp"
+#include "spic_wave.hpp"
 
 #ifndef SPIC_NS
 #error "define SPIC_NS and SPIC_STRICT before including spic_plain.inl"
@@ -318,13 +319,12 @@ constexpr int kDepBatch = 512;         // particles staged in LDS at a time
 constexpr int kDepMaxRun = 4096;       // particles per workgroup at most
 constexpr int kDepSlice = 1 << 24;     // particles binned at a time (24-bit indices)
 constexpr uint32_t kDepIndexMask = (1u << 24) - 1u;
-constexpr int kDepLdsTiles = 6144;     // tile counters a workgroup keeps in LDS
 
 struct DepBins {
   int nty, ntz, ntiles;
   int run;                // particles per work item
   int per;                // particles per thread of the count
-  int in_lds;             // the tiles' counters fit in LDS (kDepLdsTiles)
+  int in_lds;             // the tiles' counters fit in LDS (kLdsTiles)
   unsigned int *cnt;      // [ntiles + 2]: particles per tile, total, items
   unsigned int *next;     // [ntiles]: next free place of each tile
   uint4 *items;           // tile, first place, particles
@@ -340,33 +340,6 @@ __device__ __forceinline__ void dep_tile(const DepBins &b, int ix, int iy, int i
   cell = ((cx % kDepTile) * kDepTile + cy % kDepTile) * kDepTile + cz % kDepTile;
 }
 
-// Adds this lane's particle to its tile's counter and returns its rank there.
-// Lanes of one wave that share a tile take one atomic together (particles of
-// a run are near each other in most orders); after four distinct tiles the
-// remaining lanes take one each.
-__device__ __forceinline__ unsigned int dep_rank(unsigned int *cnt, unsigned int tile,
-                                                 bool active) {
-  const int lane = threadIdx.x & 63;
-  unsigned long long todo = __ballot(active);
-  int leader = lane;
-  unsigned int off = 0, group = 1;
-  for (int round = 0; round < 4 && todo; ++round) {
-    const int first = __ffsll((long long)todo) - 1;
-    const unsigned int t0 = (unsigned int)__builtin_amdgcn_readlane((int)tile, first);
-    const bool mine = ((todo >> lane) & 1ull) && tile == t0;
-    const unsigned long long same = __ballot(mine);
-    if (mine) {
-      leader = first;
-      off = (unsigned int)__popcll(same & ((1ull << lane) - 1ull));
-      group = (unsigned int)__popcll(same);
-    }
-    todo &= ~same;
-  }
-  unsigned int r = 0;
-  if (active && lane == leader) r = atomicAdd(cnt + tile, group);
-  return (unsigned int)__shfl((int)r, leader) + off;
-}
-
 template <typename T>
 __device__ __forceinline__ bool dep_cell(const KGrid<T> &g, T x, T y, T z, int &ix, int &iy,
                                          int &iz) {
@@ -380,7 +353,7 @@ __device__ __forceinline__ bool dep_cell(const KGrid<T> &g, T x, T y, T z, int &
 }
 
 // Counts the particles into tiles; with PUSH, pushes them first.  Up to
-// kDepLdsTiles tiles a workgroup counts its particles in LDS and adds each
+// kLdsTiles tiles a workgroup counts its particles in LDS and adds each
 // tile it met once: with counters in global memory alone, a million
 // particles in random order on 45 tiles took 1.3 ms in contended atomics.
 template <typename T, bool PUSH>
@@ -388,7 +361,7 @@ __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && PUSH ? 3 : 4)))
 void k_dep_count(KGrid<T> g, KField<T> f, KPart<T> p, KPush<T> k, DepBins b,
                  unsigned int *status) {
-  __shared__ unsigned int s_cnt[kDepLdsTiles];
+  __shared__ unsigned int s_cnt[kLdsTiles];
   const int tid = threadIdx.x;
   if (b.in_lds) {
     for (int t = tid; t < b.ntiles; t += kBlock) s_cnt[t] = 0u;
@@ -413,8 +386,8 @@ void k_dep_count(KGrid<T> g, KField<T> f, KPart<T> p, KPush<T> k, DepBins b,
       dep_tile(b, ix, iy, iz, tile, cell);
       b.where[i] = cell | (tile << 6);
     }
-    if (b.in_lds) dep_rank(s_cnt, tile, active);
-    else dep_rank(b.cnt, tile, active);
+    if (b.in_lds) key_rank(s_cnt, tile, active);
+    else key_rank(b.cnt, tile, active);
   }
   if (bad) atomicAdd(status, 1u);
   if (bad_dep) atomicAdd(status + 1, 1u);
@@ -453,7 +426,7 @@ static __global__ __launch_bounds__(kBlock) void k_dep_bounds(DepBins b) {
 // particles per thread, or per wave.
 template <int PER, bool IN_LDS>
 static __global__ __launch_bounds__(kBlock) void k_dep_place(DepBins b, int n) {
-  __shared__ unsigned int s_cnt[IN_LDS ? kDepLdsTiles : 1];
+  __shared__ unsigned int s_cnt[IN_LDS ? kLdsTiles : 1];
   const int tid = threadIdx.x;
   const int first = blockIdx.x * kBlock * PER;
   unsigned int w[PER], r[PER];
@@ -468,7 +441,7 @@ static __global__ __launch_bounds__(kBlock) void k_dep_place(DepBins b, int n) {
   }
 #pragma unroll
   for (int e = 0; e < PER; ++e)
-    r[e] = dep_rank(IN_LDS ? s_cnt : b.next, w[e] >> 6, first + e * kBlock + tid < n);
+    r[e] = key_rank(IN_LDS ? s_cnt : b.next, w[e] >> 6, first + e * kBlock + tid < n);
   if constexpr (IN_LDS) {
     __syncthreads();
     for (int t = tid; t < b.ntiles; t += kBlock)
@@ -625,15 +598,8 @@ void k_tile_deposit(KGrid<T> g, KPart<T> p, KMom m,
 // workgroups' batches, and a stream that may allocate (a capture keeps the
 // direct kernels).
 inline bool dep_through_tiles(long ntiles, int n, hipStream_t s) {
-  if (n < kDepMinParticles || (long)n < ntiles * kDepMinPerTile || ntiles > (1 << 26))
-    return false;
-  if (s == nullptr) return true;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return cs == hipStreamCaptureStatusNone;
+  return n >= kDepMinParticles && (long)n >= ntiles * kDepMinPerTile && ntiles <= (1 << 26) &&
+         stream_may_alloc(s);
 }
 
 // Deposit through tiles, with the push before it when `f` is given.  `taken`
@@ -660,7 +626,7 @@ hipError_t tile_deposit(const KGrid<T> &g, const KField<T> *f, const KPart<T> &p
   // enough that reading out their counters stays cheap
   b.per = slice / (kBlock * 2048);
   b.per = b.per < 1 ? 1 : b.per > 16 ? 16 : b.per;
-  b.in_lds = ntiles <= kDepLdsTiles && ntiles <= 8 * kBlock * b.per ? 1 : 0;
+  b.in_lds = ntiles <= kLdsTiles && ntiles <= 8 * kBlock * b.per ? 1 : 0;
   const size_t a_cnt = up(4 * (size_t)(ntiles + 2)), a_next = up(4 * (size_t)ntiles),
                a_items = up(sizeof(uint4) * max_items), a_n = up(4 * (size_t)slice);
   char *w = nullptr;
@@ -694,7 +660,7 @@ hipError_t tile_deposit(const KGrid<T> &g, const KField<T> *f, const KPart<T> &p
     // 1024 where few tiles make one atomic per wave contend (131072 particles
     // on 45 tiles: 73 us per call against 291), else by wave (a million on 1377
     // tiles that a short workgroup would read out: 239 us against 511).
-    if (ntiles <= kDepLdsTiles && q.n >= 128 * kBlock * 16)
+    if (ntiles <= kLdsTiles && q.n >= 128 * kBlock * 16)
       hipLaunchKernelGGL((k_dep_place<16, true>), dim3(grid_for((q.n + 15) / 16)), dim3(kBlock),
                          0, s, b, q.n);
     else if (ntiles <= 4 * kBlock)
