@@ -61,6 +61,64 @@ __device__ __forceinline__ bool clamp_index(int &ix, int n) {
   return bad;
 }
 
+// The six field components of every node together (kRec values each, FP32
+// padded to 16-byte alignment), as the mover's gather reads them: a node is
+// one line instead of six, and the two nodes of a z pair mostly share it.
+template <typename T>
+struct PackedField {
+  static constexpr int kRec = sizeof(T) == 8 ? 6 : 8;
+  const T *rec;
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_pack_fields(KField<T> f, T *__restrict__ rec, int nn) {
+  constexpr int kRec = PackedField<T>::kRec;
+  const int n = blockIdx.x * 256 + threadIdx.x;
+  if (n >= nn) return;
+  T *r = rec + (size_t)n * kRec;
+  r[0] = f.Ex[n]; r[1] = f.Ey[n]; r[2] = f.Ez[n];
+  r[3] = f.Bx[n]; r[4] = f.By[n]; r[5] = f.Bz[n];
+}
+
+// The stencil of the cell whose upper node is `base`: F[a][b][c] holds node
+// base - a * sx - b * sy - c.
+template <typename T>
+__device__ __forceinline__ void load_stencil(const KField<T> &f, int base, int sx, int sy,
+                                             T (&F)[2][2][2][6]) {
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int n = base - a * sx - b * sy - c;
+        F[a][b][c][0] = f.Ex[n]; F[a][b][c][1] = f.Ey[n]; F[a][b][c][2] = f.Ez[n];
+        F[a][b][c][3] = f.Bx[n]; F[a][b][c][4] = f.By[n]; F[a][b][c][5] = f.Bz[n];
+      }
+}
+
+template <typename T>
+__device__ __forceinline__ void load_stencil(const PackedField<T> &f, int base, int sx, int sy,
+                                             T (&F)[2][2][2][6]) {
+  constexpr int kVec = 16 / sizeof(T);  // 16-byte loads
+  typedef T Vec __attribute__((ext_vector_type(kVec)));
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const T *r = f.rec + (size_t)(base - a * sx - b * sy - c) * PackedField<T>::kRec;
+#pragma unroll
+        for (int i = 0; i < 6; i += kVec) {
+          const Vec v = *reinterpret_cast<const Vec *>(r + i);
+#pragma unroll
+          for (int j = 0; j < kVec; ++j)
+            if (i + j < 6) F[a][b][c][i + j] = v[j];
+        }
+      }
+}
+
 // One particle's predictor-corrector push and particle BC
 // (src/Mover.cpp:33-157).  Returns true if an iterate left the grid by
 // more than one cell.
@@ -69,10 +127,12 @@ __device__ __forceinline__ bool clamp_index(int &ix, int n) {
 // while the iterate stays in its cell (nine in ten do), so most particles
 // gather once instead of once per iteration: 5.97M FP64 particles of a mixed
 // order in 1.70 ms against 3.62, three waves per SIMD in FP64 (168 VGPRs,
-// the limit; unlimited it takes 176 and two).
-template <typename T>
+// the limit; unlimited it takes 176 and two).  From packed fields 24 loads of
+// 16 bytes on a sixth of the lines: a million in random order on 257499 nodes
+// 110 us against 419, in cell order 54 against 65.
+template <typename T, typename FV>
 __device__ __forceinline__ bool push_particle_once(const KGrid<T> &g,
-                                              const KField<T> &f,
+                                              const FV &f,
                                               const KPush<T> &k, T &x, T &y,
                                               T &z, T &u, T &v, T &w) {
   const int nyn = g.nyn, nzn = g.nzn;
@@ -97,17 +157,7 @@ __device__ __forceinline__ bool push_particle_once(const KGrid<T> &g,
       X0 = g.xn[ix - 1]; X1 = g.xn[ix];
       Y0 = g.yn[iy - 1]; Y1 = g.yn[iy];
       Z0 = g.zn[iz - 1]; Z1 = g.zn[iz];
-      const int base = (ix * nyn + iy) * nzn + iz;
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            const int n = base - a * sx - b * sy - c;
-            F[a][b][c][0] = f.Ex[n]; F[a][b][c][1] = f.Ey[n]; F[a][b][c][2] = f.Ez[n];
-            F[a][b][c][3] = f.Bx[n]; F[a][b][c][4] = f.By[n]; F[a][b][c][5] = f.Bz[n];
-          }
+      load_stencil(f, (ix * nyn + iy) * nzn + iz, sx, sy, F);
     }
     const T xi[2] = {xc - X0, X1 - xc};
     const T eta[2] = {yc - Y0, Y1 - yc};
@@ -190,14 +240,14 @@ __device__ __forceinline__ bool push_particle_once(const KGrid<T> &g,
 // The push of one particle: once, or k.nloop times with the particle BC
 // after each (the reference GPU mover's sub-cycle loop,
 // src/gpu/Particles_gpu.cu:336-437).
-template <typename T>
-__device__ __forceinline__ bool push_particle(const KGrid<T> &g, const KField<T> &f,
+template <typename T, typename FV>
+__device__ __forceinline__ bool push_particle(const KGrid<T> &g, const FV &f,
                                               const KPush<T> &k, T &x, T &y, T &z, T &u,
                                               T &v, T &w) {
   bool bad = false;
 #pragma unroll 1
   for (int isub = 0; isub < k.nloop; ++isub)
-    bad |= push_particle_once<T>(g, f, k, x, y, z, u, v, w);
+    bad |= push_particle_once<T, FV>(g, f, k, x, y, z, u, v, w);
   return bad;
 }
 
@@ -247,17 +297,15 @@ __device__ __forceinline__ bool deposit_particle(const KGrid<T> &g,
 
 constexpr int kBlock = 256;
 
-template <typename T>
+template <typename T, typename FV>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 4)))
-void k_mover(KGrid<T> g, KField<T> f,
-                                                  KPart<T> p, KPush<T> k,
-                                                  unsigned int *status) {
+void k_mover(KGrid<T> g, FV f, KPart<T> p, KPush<T> k, unsigned int *status) {
   bool bad = false;
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < p.n;
        i += gridDim.x * kBlock) {
     T x = p.x[i], y = p.y[i], z = p.z[i], u = p.u[i], v = p.v[i], w = p.w[i];
-    bad |= push_particle<T>(g, f, k, x, y, z, u, v, w);
+    bad |= push_particle(g, f, k, x, y, z, u, v, w);
     p.x[i] = x; p.y[i] = y; p.z[i] = z;
     p.u[i] = u; p.v[i] = v; p.w[i] = w;
   }
@@ -286,7 +334,7 @@ void k_mover_deposit(
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < p.n;
        i += gridDim.x * kBlock) {
     T x = p.x[i], y = p.y[i], z = p.z[i], u = p.u[i], v = p.v[i], w = p.w[i];
-    bad |= push_particle<T>(g, f, k, x, y, z, u, v, w);
+    bad |= push_particle(g, f, k, x, y, z, u, v, w);
     p.x[i] = x; p.y[i] = y; p.z[i] = z;
     p.u[i] = u; p.v[i] = v; p.w[i] = w;
     bad_dep |= deposit_particle<T>(g, m, x, y, z, u, v, w, p.q[i]);
@@ -356,10 +404,10 @@ __device__ __forceinline__ bool dep_cell(const KGrid<T> &g, T x, T y, T z, int &
 // kLdsTiles tiles a workgroup counts its particles in LDS and adds each
 // tile it met once: with counters in global memory alone, a million
 // particles in random order on 45 tiles took 1.3 ms in contended atomics.
-template <typename T, bool PUSH>
+template <typename T, bool PUSH, typename FV>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && PUSH ? 3 : 4)))
-void k_dep_count(KGrid<T> g, KField<T> f, KPart<T> p, KPush<T> k, DepBins b,
+void k_dep_count(KGrid<T> g, FV f, KPart<T> p, KPush<T> k, DepBins b,
                  unsigned int *status) {
   __shared__ unsigned int s_cnt[kLdsTiles];
   const int tid = threadIdx.x;
@@ -377,7 +425,7 @@ void k_dep_count(KGrid<T> g, KField<T> f, KPart<T> p, KPush<T> k, DepBins b,
       T x = p.x[i], y = p.y[i], z = p.z[i];
       if constexpr (PUSH) {
         T u = p.u[i], v = p.v[i], w = p.w[i];
-        bad |= push_particle<T>(g, f, k, x, y, z, u, v, w);
+        bad |= push_particle(g, f, k, x, y, z, u, v, w);
         p.x[i] = x; p.y[i] = y; p.z[i] = z;
         p.u[i] = u; p.v[i] = v; p.w[i] = w;
       }
@@ -602,6 +650,19 @@ inline bool dep_through_tiles(long ntiles, int n, hipStream_t s) {
          stream_may_alloc(s);
 }
 
+// Whether the push packs the fields first.  Packing costs a launch and the
+// scratch's allocation, 14 us per call, and 96 bytes per node: from 262144
+// particles (131072 in cell order on 2197 nodes: 11.4 us as they are, 21.2
+// packed; a million 59.7 / 48.9) and up to a node for two particles.
+constexpr int kPackMin = 1 << 18;
+inline bool pack_pays(int n, int nn) { return n >= kPackMin && nn <= n / 2; }
+
+template <typename T>
+void pack_fields(const KField<T> &f, const PackedField<T> &to, int nn, hipStream_t s) {
+  hipLaunchKernelGGL(k_pack_fields<T>, dim3((nn + 255) / 256), dim3(256), 0, s, f,
+                     const_cast<T *>(to.rec), nn);
+}
+
 // Deposit through tiles, with the push before it when `f` is given.  `taken`
 // stays false when nothing has run: the caller then has the direct kernels.
 template <typename T>
@@ -627,10 +688,13 @@ hipError_t tile_deposit(const KGrid<T> &g, const KField<T> *f, const KPart<T> &p
   b.per = slice / (kBlock * 2048);
   b.per = b.per < 1 ? 1 : b.per > 16 ? 16 : b.per;
   b.in_lds = ntiles <= kLdsTiles && ntiles <= 8 * kBlock * b.per ? 1 : 0;
+  const int nn = g.nxn * g.nyn * g.nzn;
+  const bool pack = f && pack_pays(p.n, nn);
+  const size_t a_fld = pack ? up(sizeof(T) * PackedField<T>::kRec * (size_t)nn) : 0;
   const size_t a_cnt = up(4 * (size_t)(ntiles + 2)), a_next = up(4 * (size_t)ntiles),
                a_items = up(sizeof(uint4) * max_items), a_n = up(4 * (size_t)slice);
   char *w = nullptr;
-  hipError_t e = stream_alloc((void **)&w, a_cnt + a_next + a_items + 2 * a_n, s);
+  hipError_t e = stream_alloc((void **)&w, a_cnt + a_next + a_items + 2 * a_n + a_fld, s);
   if (e != hipSuccess) {
     (void)hipGetLastError();  // the direct kernels need no scratch
     return hipSuccess;
@@ -641,6 +705,8 @@ hipError_t tile_deposit(const KGrid<T> &g, const KField<T> *f, const KPart<T> &p
   b.items = (uint4 *)(w + a_cnt + a_next);
   b.where = (unsigned int *)(w + a_cnt + a_next + a_items);
   b.perm = (unsigned int *)(w + a_cnt + a_next + a_items + a_n);
+  const PackedField<T> packed{(const T *)(w + a_cnt + a_next + a_items + 2 * a_n)};
+  if (pack) pack_fields(*f, packed, nn, s);
   for (int first = 0; first < p.n && e == hipSuccess; first += slice) {
     KPart<T> q = p;
     q.x += first; q.y += first; q.z += first;
@@ -649,12 +715,15 @@ hipError_t tile_deposit(const KGrid<T> &g, const KField<T> *f, const KPart<T> &p
     q.n = p.n - first < slice ? p.n - first : slice;
     if ((e = zero_u32(b.cnt, (size_t)ntiles + 2, s)) != hipSuccess) break;
     const unsigned counts = (unsigned)((q.n + kBlock * b.per - 1) / (kBlock * b.per));
-    if (f)
-      hipLaunchKernelGGL((k_dep_count<T, true>), dim3(counts), dim3(kBlock), 0, s, g, *f, q,
-                         *k, b, status);
+    if (pack)
+      hipLaunchKernelGGL((k_dep_count<T, true, PackedField<T>>), dim3(counts), dim3(kBlock), 0,
+                         s, g, packed, q, *k, b, status);
+    else if (f)
+      hipLaunchKernelGGL((k_dep_count<T, true, KField<T>>), dim3(counts), dim3(kBlock), 0, s, g,
+                         *f, q, *k, b, status);
     else
-      hipLaunchKernelGGL((k_dep_count<T, false>), dim3(counts), dim3(kBlock), 0, s, g,
-                         KField<T>{}, q, KPush<T>{}, b, status);
+      hipLaunchKernelGGL((k_dep_count<T, false, KField<T>>), dim3(counts), dim3(kBlock), 0, s,
+                         g, KField<T>{}, q, KPush<T>{}, b, status);
     hipLaunchKernelGGL(k_dep_bounds, dim3(grid_for(b.ntiles)), dim3(kBlock), 0, s, b);
     // Places by workgroup: 4096 particles each where that leaves 128 of them,
     // 1024 where few tiles make one atomic per wave contend (131072 particles
@@ -683,9 +752,25 @@ hipError_t launch_mover(const KGrid<T> &g, const KField<T> &f,
                         const KPart<T> &p, const KPush<T> &k,
                         unsigned int *status, hipStream_t s) {
   if (p.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_mover<T>, dim3(grid_for(p.n)), dim3(kBlock), 0, s, g,
-                     f, p, k, status);
-  return hipGetLastError();
+  const int nn = g.nxn * g.nyn * g.nzn;
+  T *rec = nullptr;
+  if (pack_pays(p.n, nn) && stream_may_alloc(s) &&
+      stream_alloc((void **)&rec, sizeof(T) * PackedField<T>::kRec * (size_t)nn, s) !=
+          hipSuccess) {
+    (void)hipGetLastError();  // the fields as they are need no scratch
+    rec = nullptr;
+  }
+  if (!rec) {
+    hipLaunchKernelGGL((k_mover<T, KField<T>>), dim3(grid_for(p.n)), dim3(kBlock), 0, s, g, f,
+                       p, k, status);
+    return hipGetLastError();
+  }
+  const PackedField<T> packed{rec};
+  pack_fields(f, packed, nn, s);
+  hipLaunchKernelGGL((k_mover<T, PackedField<T>>), dim3(grid_for(p.n)), dim3(kBlock), 0, s, g,
+                     packed, p, k, status);
+  const hipError_t e = hipGetLastError(), ef = stream_free(rec, s);
+  return e != hipSuccess ? e : ef;
 }
 
 template <typename T>
