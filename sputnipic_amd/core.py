@@ -207,6 +207,10 @@ class Particles:
                             self.qom, self.NiterMover, self.n_sub_cycles)
 
 
+# structs of pointers are filled through arrays of the same layout
+_P4, _P10 = C.c_void_p * 4, C.c_void_p * 10
+
+
 class InterpDensSpecies:
     """The ten node moments of one species, FP64 on the device."""
 
@@ -222,8 +226,8 @@ class InterpDensSpecies:
             self.d[n].upload(np.ascontiguousarray(arrays[n], np.float64))
 
     def c_struct(self) -> spic_moments:
-        D = C.POINTER(C.c_double)
-        return spic_moments(*[C.cast(self.d[n].ptr, D) for n in MOMENT_NAMES])
+        # ten addresses at once: 2.4 us, 9.9 with a cast for each
+        return spic_moments.from_buffer(_P10(*[self.d[n].ptr for n in MOMENT_NAMES]))
 
 
 class InterpDensNet(InterpDensSpecies):
@@ -254,9 +258,8 @@ class InterpDensAux:
 
     def c_struct(self):
         from ._capi import spic_hat
-        D = C.POINTER(C.c_double)
-        return spic_hat(C.cast(self.rhoh.ptr, D), *[C.cast(self.J[n].ptr, D)
-                                                    for n in ("Jxh", "Jyh", "Jzh")])
+        return spic_hat.from_buffer(
+            _P4(self.rhoh.ptr, *[self.J[n].ptr for n in ("Jxh", "Jyh", "Jzh")]))
 
 
 @dataclass

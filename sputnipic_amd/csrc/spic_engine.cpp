@@ -705,7 +705,7 @@ int spic_engine_phase(spic_engine *e, const spic_field *field,
   err = e->grd.prec == SPIC_F64 ? launch_phase<double>(e, field, mom, push, st, s)
                                 : launch_phase<float>(e, field, mom, push, st, s);
   e->phases++;
-  return spic::end_call(s, st, err);
+  return spic::end_call(s, err);
 }
 
 int spic_engine_deposit(spic_engine *e, const spic_moments *mom, void *stream) {
@@ -730,7 +730,7 @@ int spic_engine_deposit(spic_engine *e, const spic_moments *mom, void *stream) {
   hipError_t err = e->grd.prec == SPIC_F64
                        ? launch_phase<double>(e, &f0, mom, &p0, st, s, 1)
                        : launch_phase<float>(e, &f0, mom, &p0, st, s, 1);
-  return spic::end_call(s, st, err);
+  return spic::end_call(s, err);
 }
 
 int spic_test_fail_engine_alloc(int after) {
@@ -983,11 +983,8 @@ hipError_t zero_empty_batch_moments(const spic_batch *b, hipStream_t s) {
     const size_t nn = (size_t)e->grd.nxn * e->grd.nyn * e->grd.nzn;
     for (int is = 0; is < e->ns; ++is) {
       if (!e->sp[is].loaded || e->sp[is].n != 0 || !b->mom[i][is].rhon) continue;
-      const spic::KMom m = spic::kmom(&b->mom[i][is]);
-      for (int c = 0; c < 10; ++c) {
-        const hipError_t err = spic::zero_f64(m.m[c], nn, s);
-        if (err != hipSuccess) return err;
-      }
+      const hipError_t err = spic::zero_moment_arrays(b->mom[i][is], nn, s);
+      if (err != hipSuccess) return err;
     }
   }
   return hipSuccess;
@@ -1114,7 +1111,7 @@ int spic_batch_phase(spic_batch *b, void *stream) {
     // no member holds a particle: the written moments are all zero
     err = (b->flags & SPIC_BATCH_SET_MOMENTS) ? zero_empty_batch_moments(b, s) : hipSuccess;
     if (err == hipSuccess) b->phases++;
-    return spic::end_call(s, st, err);
+    return spic::end_call(s, err);
   }
   if (stale || st != b->status) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -1176,7 +1173,7 @@ int spic_batch_phase(spic_batch *b, void *stream) {
     }
     b->phases++;
   }
-  return spic::end_call(s, st, err);
+  return spic::end_call(s, err);
 }
 
 int spic_batch_destroy(spic_batch *b) {

@@ -88,8 +88,10 @@ hipError_t stream_free(void *p, hipStream_t s);
 // Whether work on the stream may take such scratch: not while it is captured.
 bool stream_may_alloc(hipStream_t s);
 
-hipError_t zero_f64(double *p, size_t n, hipStream_t s);
 hipError_t zero_u32(unsigned int *p, size_t n, hipStream_t s);
+hipError_t zero_moment_arrays(const spic_moments &m, size_t nn, hipStream_t s);
+// n words into pinned host memory, there once the stream has been waited for.
+hipError_t copy_u32(unsigned int *host, const unsigned int *p, size_t n, hipStream_t s);
 
 // Synthetic Harris-sheet input (spic_gem.hip).
 hipError_t gem_fields(const spic_grid &g, const spic_gem_params &p,
@@ -165,8 +167,7 @@ bool async_mode();
 bool strict_mode();
 unsigned int *status_buffer(hipError_t *err);
 int begin_call(hipStream_t s, unsigned int **st);
-int read_status(hipStream_t s, unsigned int *st, bool clear);
-int end_call(hipStream_t s, unsigned int *st, hipError_t launch);
+int end_call(hipStream_t s, hipError_t launch);
 int check_grid(const spic_grid *g);
 int check_species(const spic_species *sp, bool need_q, bool need_move);
 int check_field(const spic_field *f);

@@ -74,6 +74,14 @@ __global__ void k_sum_species(MomentSets net, MomentSets ids, int ns, long nn) {
   }
 }
 
+// The ten arrays of a set in one launch, a node of each per thread.
+__global__ __launch_bounds__(256) void k_zero_moments(MomentSets m, size_t nn) {
+  for (size_t n = blockIdx.x * (size_t)256 + threadIdx.x; n < nn; n += (size_t)gridDim.x * 256) {
+#pragma unroll
+    for (int k = 0; k < 10; ++k) m.a[k][n] = 0.0;
+  }
+}
+
 inline unsigned nblocks(long n) {
   long b = (n + 255) / 256;
   if (b < 1) b = 1;
@@ -88,6 +96,15 @@ int finish(hipStream_t s, const char *what) {
 }
 
 }  // namespace
+
+hipError_t zero_moment_arrays(const spic_moments &mom, size_t nn, hipStream_t s) {
+  if (nn == 0) return hipSuccess;
+  MomentSets m;
+  moment_arrays(mom, m.a);
+  hipLaunchKernelGGL(k_zero_moments, dim3(nblocks((long)nn)), dim3(256), 0, s, m, nn);
+  return hipGetLastError();
+}
+
 }  // namespace spic
 
 extern "C" {

@@ -53,10 +53,10 @@ __global__ void k_gather(const T *__restrict__ src, T *__restrict__ dst,
     dst[i] = src[perm[i]];
 }
 
-__global__ void k_fill_f64(double *p, size_t n) {
+__global__ void k_copy_u32(unsigned int *host, const unsigned int *p, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
-    p[i] = 0.0;
+    __hip_atomic_store(host + i, p[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void k_fill_u32(unsigned int *p, size_t n) {
@@ -76,17 +76,16 @@ inline size_t align_up(size_t v) { return (v + 255) & ~size_t(255); }
 
 }  // namespace
 
-hipError_t zero_f64(double *p, size_t n, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_f64, dim3(blocks_for(n, 256)), dim3(256), 0, s, p,
-                     n);
-  return hipGetLastError();
-}
-
 hipError_t zero_u32(unsigned int *p, size_t n, hipStream_t s) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(n, 256)), dim3(256), 0, s, p,
                      n);
+  return hipGetLastError();
+}
+
+hipError_t copy_u32(unsigned int *host, const unsigned int *p, size_t n, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(n, 256)), dim3(256), 0, s, host, p, n);
   return hipGetLastError();
 }
 
