@@ -832,7 +832,11 @@ __device__ __forceinline__ void copy_particle(PS src, PSI src_id, int64_t stride
 
 constexpr int kTileThreads = 512;
 constexpr unsigned int kTileStaged = 12288;  // particles a tile block stages in LDS
-constexpr int kTileStageBytes = 32768;       // one output chunk of one component
+// Values of one component that a tile block stages at a time.  In FP32 its 16 KB
+// (and slot tables of 256 ranks in them) leave room for a third workgroup per
+// CU: 6.3M particles on 3072 tiles in 145 us against 187 with 8192 (a fourth, at
+// 6144 staged slots, changes nothing).
+constexpr int kTileChunk = 4096;
 constexpr int kTileU = 4;                    // particles a thread loads at once
 constexpr int kScanThreads = 1024;
 
@@ -1011,11 +1015,12 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_sort(
     const int64_t *src_seg_a, const unsigned int *src_cnt_a, unsigned int ovf_cap, T *dst_a,
     uint32_t *dst_id_a, const int64_t *dst_seg_a, const unsigned int *own_a,
     unsigned int *fill_a, const TileSortJob<T> *__restrict__ jobs, TileSortMap map) {
+  constexpr int kTileStageBytes = kTileChunk * (int)sizeof(T);
   static_assert(KT * NC <= kTileStageBytes, "slot table exceeds the stage");
   static_assert(NC <= 256, "counts of the cells before a cell must fit a byte");
   constexpr uint16_t kForeign = 0xFFFF;  // also "no slot": foreign particles take none
   constexpr uint16_t kNoSlot = 0xFFFF;
-  constexpr int kChunk = kTileStageBytes / (int)sizeof(T);
+  constexpr int kChunk = kTileChunk;
   __shared__ unsigned int s_count[NC], s_rank[NC], s_kmax, s_own;
   __shared__ unsigned int s_A[KT];
   // each staged particle's cell (step 1), then its slot (step 2)
@@ -1241,12 +1246,12 @@ hipError_t tile_sort(const TileSortJob<T> &J, hipStream_t s) {
   hipLaunchKernelGGL(k_tile_bounds<T>, dim3(1), dim3(kScanThreads), 0, s, J);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (nc == 64)
-    hipLaunchKernelGGL((k_tile_sort<T, 64, 512, false>), grid, dim3(kTileThreads), 0, s, J.g, J.L,
+    hipLaunchKernelGGL((k_tile_sort<T, 64, 64 * sizeof(T), false>), grid, dim3(kTileThreads), 0, s, J.g, J.L,
                        J.src, J.stride, J.src_id, J.src_seg, J.src_cnt, J.ovf_cap, J.dst,
                        J.dst_id, (const int64_t *)J.dst_seg, (const unsigned int *)J.own,
                        J.fill, (const TileSortJob<T> *)nullptr, TileSortMap{});
   else
-    hipLaunchKernelGGL((k_tile_sort<T, 128, 256, false>), grid, dim3(kTileThreads), 0, s, J.g, J.L,
+    hipLaunchKernelGGL((k_tile_sort<T, 128, 32 * sizeof(T), false>), grid, dim3(kTileThreads), 0, s, J.g, J.L,
                        J.src, J.stride, J.src_id, J.src_seg, J.src_cnt, J.ovf_cap, J.dst,
                        J.dst_id, (const int64_t *)J.dst_seg, (const unsigned int *)J.own,
                        J.fill, (const TileSortJob<T> *)nullptr, TileSortMap{});
@@ -1276,13 +1281,13 @@ hipError_t tile_sort_batch(const TileSortJob<T> *jobs, const TileSortMap &map, i
   if ((e = hipGetLastError()) != hipSuccess) return e;
   // the batch instances take their arguments from the job table
   if (nc == 64)
-    hipLaunchKernelGGL((k_tile_sort<T, 64, 512, true>), grid, dim3(kTileThreads), 0, s, g0, L0,
+    hipLaunchKernelGGL((k_tile_sort<T, 64, 64 * sizeof(T), true>), grid, dim3(kTileThreads), 0, s, g0, L0,
                        (const T *)nullptr, (int64_t)0, (const uint32_t *)nullptr,
                        (const int64_t *)nullptr, (const unsigned int *)nullptr, 0u,
                        (T *)nullptr, (uint32_t *)nullptr, (const int64_t *)nullptr,
                        (const unsigned int *)nullptr, (unsigned int *)nullptr, jobs, map);
   else
-    hipLaunchKernelGGL((k_tile_sort<T, 128, 256, true>), grid, dim3(kTileThreads), 0, s, g0,
+    hipLaunchKernelGGL((k_tile_sort<T, 128, 32 * sizeof(T), true>), grid, dim3(kTileThreads), 0, s, g0,
                        L0, (const T *)nullptr, (int64_t)0, (const uint32_t *)nullptr,
                        (const int64_t *)nullptr, (const unsigned int *)nullptr, 0u,
                        (T *)nullptr, (uint32_t *)nullptr, (const int64_t *)nullptr,
