@@ -229,6 +229,7 @@ __global__ void k_bin_gather(Arrays7<TS> src, const uint32_t *__restrict__ src_i
 // (281 us).  Tiles of more than kLoadHeld particles on average keep the radix
 // sort, whose work does not depend on the number of tiles.
 constexpr int kLoadThreads = 1024;
+constexpr int kLoadManyTiles = 16384;
 constexpr int kLoadPer = 8;      // particles per thread that a tile's workgroup holds
 constexpr int kLoadHeld = kLoadThreads * kLoadPer;
 constexpr int kLoadStage = 4096;  // values staged in LDS at a time
@@ -252,22 +253,23 @@ struct LoadBins {
   uint32_t *perm;          // [n] by place: index of the particle
 };
 
-// Counts the particles into tiles: up to kLdsTiles tiles (IN_LDS) a workgroup
-// counts in LDS and adds each tile it met once.
-template <typename TS, typename T, bool IN_LDS>
-__global__ __launch_bounds__(256) void k_load_count(KGrid<T> g, BinLayout L, LoadBins b,
-                                                    const TS *__restrict__ x,
-                                                    const TS *__restrict__ y,
-                                                    const TS *__restrict__ z) {
-  __shared__ unsigned int s_cnt[IN_LDS ? kLdsTiles : 1];
+// Counts the particles into tiles, NT threads per workgroup, which counts up to
+// LT tiles in LDS and adds each tile it met once; LT = 0: one atomic per wave and
+// tile in global memory.
+template <typename TS, typename T, int NT, int LT>
+__global__ __launch_bounds__(NT) void k_load_count(KGrid<T> g, BinLayout L, LoadBins b,
+                                                   const TS *__restrict__ x,
+                                                   const TS *__restrict__ y,
+                                                   const TS *__restrict__ z) {
+  __shared__ unsigned int s_cnt[LT > 0 ? LT : 1];
   const int tid = threadIdx.x;
-  if constexpr (IN_LDS) {
-    for (int t = tid; t < L.ntiles; t += 256) s_cnt[t] = 0u;
+  if constexpr (LT > 0) {
+    for (int t = tid; t < L.ntiles; t += NT) s_cnt[t] = 0u;
     __syncthreads();
   }
-  const int64_t first = blockIdx.x * (int64_t)(256 * b.per);
+  const int64_t first = blockIdx.x * (int64_t)(NT * b.per);
   for (int e = 0; e < b.per; ++e) {
-    const int64_t i = first + e * 256 + tid;
+    const int64_t i = first + e * NT + tid;
     const bool active = i < b.n;
     uint32_t tile = 0, cit = 0;
     if (active) {
@@ -275,46 +277,46 @@ __global__ __launch_bounds__(256) void k_load_count(KGrid<T> g, BinLayout L, Loa
       cell_of(g, L, x[i], y[i], z[i], cx, cy, cz, tile, cit, false);
       b.where[i] = (tile << L.cell_bits) | cit;
     }
-    key_rank(IN_LDS ? s_cnt : b.count, tile, active);
+    key_rank(LT > 0 ? s_cnt : b.count, tile, active);
   }
-  if constexpr (IN_LDS) {
+  if constexpr (LT > 0) {
     __syncthreads();
-    for (int t = tid; t < L.ntiles; t += 256)
+    for (int t = tid; t < L.ntiles; t += NT)
       if (s_cnt[t]) atomicAdd(b.count + t, s_cnt[t]);
   }
 }
 
 // Places each particle's index in its tile: each tile's places at once per
-// workgroup (IN_LDS), PER particles per thread, or per wave.
-template <int PER, bool IN_LDS>
-__global__ __launch_bounds__(256) void k_load_place(BinLayout L, LoadBins b) {
-  __shared__ unsigned int s_cnt[IN_LDS ? kLdsTiles : 1];
+// workgroup (LT > 0), PER particles per thread, or per wave.
+template <int PER, int NT, int LT>
+__global__ __launch_bounds__(NT) void k_load_place(BinLayout L, LoadBins b) {
+  __shared__ unsigned int s_cnt[LT > 0 ? LT : 1];
   const int tid = threadIdx.x;
-  const int64_t first = blockIdx.x * (int64_t)(256 * PER);
+  const int64_t first = blockIdx.x * (int64_t)(NT * PER);
   unsigned int t[PER], r[PER];
 #pragma unroll
   for (int e = 0; e < PER; ++e) {
-    const int64_t i = first + e * 256 + tid;
+    const int64_t i = first + e * NT + tid;
     t[e] = i < b.n ? b.where[i] >> L.cell_bits : 0u;
   }
-  if constexpr (IN_LDS) {
-    for (int k = tid; k < L.ntiles; k += 256) s_cnt[k] = 0u;
+  if constexpr (LT > 0) {
+    for (int k = tid; k < L.ntiles; k += NT) s_cnt[k] = 0u;
     __syncthreads();
   }
 #pragma unroll
   for (int e = 0; e < PER; ++e)
-    r[e] = key_rank(IN_LDS ? s_cnt : b.next, t[e], first + e * 256 + tid < b.n);
-  if constexpr (IN_LDS) {
+    r[e] = key_rank(LT > 0 ? s_cnt : b.next, t[e], first + e * NT + tid < b.n);
+  if constexpr (LT > 0) {
     __syncthreads();
-    for (int k = tid; k < L.ntiles; k += 256)
+    for (int k = tid; k < L.ntiles; k += NT)
       if (s_cnt[k]) s_cnt[k] = atomicAdd(b.next + k, s_cnt[k]);
     __syncthreads();
   }
 #pragma unroll
   for (int e = 0; e < PER; ++e) {
-    const int64_t i = first + e * 256 + tid;
+    const int64_t i = first + e * NT + tid;
     if (i < b.n)
-      b.perm[b.seg[t[e]] - (int64_t)t[e] * L.slack + (IN_LDS ? s_cnt[t[e]] : 0u) + r[e]] =
+      b.perm[b.seg[t[e]] - (int64_t)t[e] * L.slack + (LT > 0 ? s_cnt[t[e]] : 0u) + r[e]] =
           (uint32_t)i;
   }
 }
@@ -1332,8 +1334,11 @@ hipError_t load_tiles(const KGrid<T> &g, const BinLayout &L, int64_t n, const vo
   b.seg = dst_seg;
   b.where = (uint32_t *)(w + a_t);
   b.perm = (uint32_t *)(w + a_t + a_n);
+  // many tiles: workgroups of 1024 threads and 64 KB of counters, 16384
+  // particles each, where that leaves one per CU
+  const bool many = L.ntiles > kLdsTiles && L.ntiles <= kLoadManyTiles && n >= 256 * 1024 * 16;
   const int64_t per = n / (256 * 2048);
-  b.per = per < 1 ? 1 : per > 16 ? 16 : (int)per;
+  b.per = many || per > 16 ? 16 : per < 1 ? 1 : (int)per;
   Arrays7<TS> as;
   Arrays7<T> ad;
   for (int a = 0; a < 7; ++a) {
@@ -1345,12 +1350,16 @@ hipError_t load_tiles(const KGrid<T> &g, const BinLayout &L, int64_t n, const vo
   hipError_t e;
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (n > 0) {
-    const dim3 grid((unsigned)((n + 256 * b.per - 1) / (256 * b.per)));
-    if (L.ntiles <= kLdsTiles && L.ntiles <= 8 * 256 * b.per)
-      hipLaunchKernelGGL((k_load_count<TS, T, true>), grid, dim3(256), 0, s, g, L, b, as.p[0],
-                         as.p[1], as.p[2]);
+    const int nt = many ? 1024 : 256;
+    const dim3 grid((unsigned)((n + nt * b.per - 1) / (nt * b.per)));
+    if (many)
+      hipLaunchKernelGGL((k_load_count<TS, T, 1024, kLoadManyTiles>), grid, dim3(1024), 0, s, g,
+                         L, b, as.p[0], as.p[1], as.p[2]);
+    else if (L.ntiles <= kLdsTiles && L.ntiles <= 8 * 256 * b.per)
+      hipLaunchKernelGGL((k_load_count<TS, T, 256, kLdsTiles>), grid, dim3(256), 0, s, g, L, b,
+                         as.p[0], as.p[1], as.p[2]);
     else
-      hipLaunchKernelGGL((k_load_count<TS, T, false>), grid, dim3(256), 0, s, g, L, b, as.p[0],
+      hipLaunchKernelGGL((k_load_count<TS, T, 256, 0>), grid, dim3(256), 0, s, g, L, b, as.p[0],
                          as.p[1], as.p[2]);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
@@ -1358,12 +1367,15 @@ hipError_t load_tiles(const KGrid<T> &g, const BinLayout &L, int64_t n, const vo
   if ((e = hipGetLastError()) != hipSuccess || n == 0) return e;
   // places by workgroup or by wave, as the deposit through tiles takes them
   auto blocks = [n](int per) { return dim3((unsigned)((n + 256 * per - 1) / (256 * per))); };
-  if (L.ntiles <= kLdsTiles && n >= 128 * 256 * 16)
-    hipLaunchKernelGGL((k_load_place<16, true>), blocks(16), dim3(256), 0, s, L, b);
+  if (many)
+    hipLaunchKernelGGL((k_load_place<16, 1024, kLoadManyTiles>), blocks(64), dim3(1024), 0, s, L,
+                       b);
+  else if (L.ntiles <= kLdsTiles && n >= 128 * 256 * 16)
+    hipLaunchKernelGGL((k_load_place<16, 256, kLdsTiles>), blocks(16), dim3(256), 0, s, L, b);
   else if (L.ntiles <= 4 * 256)
-    hipLaunchKernelGGL((k_load_place<4, true>), blocks(4), dim3(256), 0, s, L, b);
+    hipLaunchKernelGGL((k_load_place<4, 256, kLdsTiles>), blocks(4), dim3(256), 0, s, L, b);
   else
-    hipLaunchKernelGGL((k_load_place<1, false>), blocks(1), dim3(256), 0, s, L, b);
+    hipLaunchKernelGGL((k_load_place<1, 256, 0>), blocks(1), dim3(256), 0, s, L, b);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   const dim3 tiles((unsigned)((L.ntiles + 7) / 8 * 8));
   if (nc == 64)
