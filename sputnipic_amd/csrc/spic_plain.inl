@@ -1,7 +1,8 @@
 // spic_plain.inl -- caller-order ("plain") gfx950 kernels for mover_PC,
-// interpP2G and the fused mover_interp.  One lane per particle; SoA loads
-// and stores are coalesced; field and node-coordinate gathers go through
-// L2; the deposit adds FP64 with hardware global atomics.
+// interpP2G and the fused mover_interp.  The push takes one lane per particle;
+// SoA loads and stores are coalesced; field and node-coordinate gathers go
+// through L2.  The deposit sums per cell in registers, by tile or by wave, and
+// adds its sums in FP64 with hardware global atomics.
 //
 // Included by two translation units: spic_plain_fast.hip (SPIC_STRICT 0,
 // FMA contraction allowed) and spic_plain_strict.hip (SPIC_STRICT 1, built

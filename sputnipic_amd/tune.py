@@ -4,7 +4,7 @@ threads, per workgroup: 4x4x4 = 256 or 8x4x4 = 512) and the sort schedule
 candidate on the caller's own workload -- a batch of independent instances
 (tune_batch) or one engine (tune_engine) -- and, for an FP32 fixed-point
 engine, the particles each thread pushes per batch of the phase
-(tune_engine's ``ppt_choices``: one, or two with buckets twice as deep, which
+(tune_engine's ``ppt_choices``: one, or two with batches twice as large, which
 costs the third workgroup per compute unit).  Batches run one particle per
 thread.
 
