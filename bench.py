@@ -156,7 +156,7 @@ def run_form(prec: str, steps: int, warmup: int, engine: str, sort_every: int,
                   f"particle order: {order})")
     else:
         s_c = [p.c_struct() for p in parts]
-        kernel = "k_mover_deposit (plain fused, one launch per species)"
+        kernel = "mover_interp in caller order (push and count, deposit by tile)"
     S.set_async(True)
     marks = []  # (kind, start event, end event) of the timed cycles
     pool = [S.Event() for _ in range(2 * (steps + 1) * (NS + 1))]

@@ -329,9 +329,9 @@ typedef struct spic_engine_opts {
                                  load the species again) */
   int particles_per_thread;   /* particles each thread pushes and bins per
                                  batch of the phase kernel before the
-                                 batch's bucket step: 0 or 1 (default), or
+                                 batch's cell step: 0 or 1 (default), or
                                  2 (FP32 engines with fixed-point positions;
-                                 the buckets double, two workgroups per CU
+                                 the sorted batch doubles, two workgroups per CU
                                  instead of three).  Trajectories do not
                                  depend on it.  Batches (spic_batch_create)
                                  and spic_engine_deposit use one */
