@@ -66,21 +66,53 @@ struct StatusBuf {
   bool shared = false;
   bool maybe_set = false;  // a call since the last read may have set a word
 };
-thread_local std::vector<StatusBuf> t_status;
+// Words of threads that have ended, for the next ones: those that nothing can
+// write any more and that were last read as zeros.  Never destroyed, since
+// threads may end after static objects have.
+struct StatusFree {
+  std::mutex mutex;
+  std::vector<StatusBuf> bufs;
+};
+StatusFree &status_free() {
+  static StatusFree *f = new StatusFree();
+  return *f;
+}
+struct ThreadStatus {
+  std::vector<StatusBuf> bufs;
+  ~ThreadStatus() {
+    StatusFree &f = status_free();
+    std::lock_guard<std::mutex> lock(f.mutex);
+    for (const auto &sb : bufs)
+      if (!sb.shared && !sb.maybe_set) f.bufs.push_back(sb);
+  }
+};
+thread_local ThreadStatus t_thread_status;
 
 StatusBuf *status_words(hipError_t *err) {
   int dev = 0;
   *err = hipGetDevice(&dev);
   if (*err != hipSuccess) return nullptr;
+  std::vector<StatusBuf> &t_status = t_thread_status.bufs;
   for (auto &sb : t_status)
     if (sb.device == dev) return &sb;
+  {
+    StatusFree &f = status_free();
+    std::lock_guard<std::mutex> lock(f.mutex);
+    for (size_t i = 0; i < f.bufs.size(); ++i)
+      if (f.bufs[i].device == dev) {
+        t_status.push_back(f.bufs[i]);
+        f.bufs.erase(f.bufs.begin() + i);
+        return &t_status.back();
+      }
+  }
   StatusBuf sb;
   sb.device = dev;
   *err = hipMalloc((void **)&sb.d, 4 * sizeof(unsigned int));
   if (*err != hipSuccess) return nullptr;
   if ((*err = hipHostMalloc((void **)&sb.h, 4 * sizeof(unsigned int), hipHostMallocDefault)) !=
           hipSuccess ||
-      (*err = hipMemset(sb.d, 0, 4 * sizeof(unsigned int))) != hipSuccess) {
+      (*err = hipMemset(sb.d, 0, 4 * sizeof(unsigned int))) != hipSuccess ||
+      (*err = hipStreamSynchronize(nullptr)) != hipSuccess) {
     if (sb.h) (void)hipHostFree(sb.h);
     (void)hipFree(sb.d);
     return nullptr;
