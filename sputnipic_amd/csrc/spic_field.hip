@@ -314,20 +314,22 @@ __device__ __forceinline__ void div_symm(const A (&P)[6], int64_t o, int64_t si,
   out[2] = (c3X + c3Y + c3Z) * alfa;
 }
 
-// Workgroup tiles of the fused field kernels: 256 points, 16 along z.
-constexpr int kFX = 4, kFY = 4, kFZ = 16;
-constexpr int kFieldThreads = 448;  // one per node of the tile, in whole waves
+// Workgroup tiles of the image's first kernel: FX x 4 x 16 cells.
+constexpr int kFY = 4, kFZ = 16;
+// One thread per node of the tile, in whole waves.
+template <int FX>
+constexpr int kFieldThreads = ((FX + 1) * (kFY + 1) * (kFZ + 1) + 63) / 64 * 64;
 
 struct Tiles {
   int ny, nz;  // tiles per axis
   unsigned total;
 };
 
-inline Tiles tiles_of(int n0, int n1, int n2) {
+inline Tiles tiles_of(int fx, int n0, int n1, int n2) {
   Tiles t;
   t.ny = (n1 + kFY - 1) / kFY;
   t.nz = (n2 + kFZ - 1) / kFZ;
-  t.total = (unsigned)((n0 + kFX - 1) / kFX * t.ny * t.nz);
+  t.total = (unsigned)((n0 + fx - 1) / fx * t.ny * t.nz);
   return t;
 }
 
@@ -464,22 +466,23 @@ __device__ __forceinline__ int64_t vec_at(const Dims &d, int i, int j, int k) {
 // interior nodes, species in order from zero, and divN2C of D on the interior
 // cells (its stencil reads interior nodes only, so D's ghost update, which
 // the reference applies first, does not change it).  One workgroup per tile
-// of cells; D of the tile's 5x5x17 nodes passes through LDS, so the nodes of
-// the upper faces are computed twice (1.66 nodes per cell) and a launch and a
-// read of D are saved.  Latency bounds it: one node per thread (448 threads, 17.4
-// us on 128x64x64 cells) instead of two in turn (256 threads, 24 us).
-__global__ __launch_bounds__(kFieldThreads) void k_image_d(Dims d, ImageArgs a, Tiles tiles,
+// of cells; D of the tile's nodes passes through LDS, so the nodes of the upper
+// faces are computed twice (1.66 nodes per cell with FX 4, 1.49 with 8) and a
+// launch and a read of D are saved.  Latency bounds it: one node per thread
+// instead of two in turn (17.4 against 24 us on 128x64x64 cells, FX 4).
+template <int FX>
+__global__ __launch_bounds__(kFieldThreads<FX>) void k_image_d(Dims d, ImageArgs a, Tiles tiles,
                                                            double *divc, double invdx,
                                                            double invdy, double invdz) {
-  constexpr int NX = kFX + 1, NY = kFY + 1, NZ = kFZ + 1;
+  constexpr int NX = FX + 1, NY = kFY + 1, NZ = kFZ + 1;
   __shared__ double s_d[3][NX * NY * NZ];
   const int tid = threadIdx.x;
   const unsigned tile = xcd_block();
   if (tile >= tiles.total) return;
   const int bz = tile % tiles.nz, by = (tile / tiles.nz) % tiles.ny,
             bx = tile / (tiles.nz * tiles.ny);
-  const int i0 = 1 + bx * kFX, j0 = 1 + by * kFY, k0 = 1 + bz * kFZ;
-  for (int e = tid; e < NX * NY * NZ; e += kFieldThreads) {
+  const int i0 = 1 + bx * FX, j0 = 1 + by * kFY, k0 = 1 + bz * kFZ;
+  for (int e = tid; e < NX * NY * NZ; e += kFieldThreads<FX>) {
     const int ex = e / (NY * NZ), ey = (e / NZ) % NY, ez = e % NZ;
     const int i = i0 + ex, j = j0 + ey, k = k0 + ez;
     if (i > d.nxn - 2 || j > d.nyn - 2 || k > d.nzn - 2) continue;
@@ -509,7 +512,7 @@ __global__ __launch_bounds__(kFieldThreads) void k_image_d(Dims d, ImageArgs a, 
     s_d[2][e] = dz;
     // a node belongs to the tile of the cell it starts; the last plane's
     // nodes start no interior cell and belong to the last tile
-    if ((ex < kFX || i == d.nxn - 2) && (ey < kFY || j == d.nyn - 2) &&
+    if ((ex < FX || i == d.nxn - 2) && (ey < kFY || j == d.nyn - 2) &&
         (ez < kFZ || k == d.nzn - 2)) {
       gmem(a.D[0])[n] = dx;
       gmem(a.D[1])[n] = dy;
@@ -517,7 +520,7 @@ __global__ __launch_bounds__(kFieldThreads) void k_image_d(Dims d, ImageArgs a, 
     }
   }
   __syncthreads();
-  if (tid >= kFX * kFY * kFZ) return;
+  if (tid >= FX * kFY * kFZ) return;
   const int lx = tid / (kFY * kFZ), ly = (tid / kFZ) % kFY, lz = tid % kFZ;
   const int i = i0 + lx, j = j0 + ly, k = k0 + lz;
   if (i > d.nxc - 2 || j > d.nyc - 2 || k > d.nzc - 2) return;
@@ -543,7 +546,7 @@ __device__ __forceinline__ void load3(const SPIC_GLOBAL double *p, double v[3]) 
 // (src/MaxwellSolver.cpp:168-231, src/Grid.cpp:187-225 and 668-717).  The
 // ghosts of v (applyBCscalarFieldNzero) and of divC (applyBCscalarFieldC)
 // are read at their sources: no unpacked copy of v and no ghost update runs.
-// The operator takes two launches instead of eight: 31 us per application on
+// The operator takes two launches instead of eight: 28 us per application on
 // 128x64x64 cells against 53.
 __global__ void k_image(Dims d, ImageArgs a, GhostMap gn, GhostMap gc, const double *divc,
                         double *im, double invdx, double invdy, double invdz, double dd) {
@@ -794,7 +797,13 @@ int spic_maxwell_image(const spic_grid *grd, const spic_field *field,
   a.ns = ns;
   const spic::GhostMap gn = spic::ghost_map(d.nxn, d.nyn, d.nzn, true, p),
                        gc = spic::ghost_map(d.nxc, d.nyc, d.nzc, false, p);
-  const spic::Tiles tiles = spic::tiles_of(d.nxc - 2, d.nyc - 2, d.nzc - 2);
+  // Larger tiles compute fewer nodes twice but leave a small grid with fewer
+  // workgroups: the operator takes 28.3 us with FX 8 on 128x64x64 cells (1024
+  // workgroups of it) and 29.6 with FX 4, but a cycle with eight of them on
+  // 33x17x19 cells (32) 300 and 293; on 64x32x32 (128) they do not differ.
+  spic::Tiles tiles = spic::tiles_of(8, d.nxc - 2, d.nyc - 2, d.nzc - 2);
+  const bool wide = tiles.total >= 256;
+  if (!wide) tiles = spic::tiles_of(4, d.nxc - 2, d.nyc - 2, d.nzc - 2);
   // the image's nodes read their neighbours' unknowns: an image in the
   // vector's own memory is formed from a copy
   hipError_t e = hipSuccess;
@@ -804,8 +813,13 @@ int spic_maxwell_image(const spic_grid *grd, const spic_field *field,
                        hipMemcpyDeviceToDevice, s);
     if (e != hipSuccess) return spic::hip_fail(e, "MaxwellImage");
   }
-  hipLaunchKernelGGL(spic::k_image_d, dim3(spic::xcd_grid(tiles.total)), dim3(spic::kFieldThreads), 0, s, d, a,
-                     tiles, divc, .25 * grd->invdx, .25 * grd->invdy, .25 * grd->invdz);
+  const dim3 grid(spic::xcd_grid(tiles.total));
+  if (wide)
+    hipLaunchKernelGGL(spic::k_image_d<8>, grid, dim3(spic::kFieldThreads<8>), 0, s, d, a, tiles,
+                       divc, .25 * grd->invdx, .25 * grd->invdy, .25 * grd->invdz);
+  else
+    hipLaunchKernelGGL(spic::k_image_d<4>, grid, dim3(spic::kFieldThreads<4>), 0, s, d, a, tiles,
+                       divc, .25 * grd->invdx, .25 * grd->invdy, .25 * grd->invdz);
   e = hipGetLastError();
   if (e == hipSuccess) {
     hipLaunchKernelGGL(spic::k_image, dim3(spic::xcd_grid(spic::grid1(d.in_nodes))), dim3(256), 0, s, d, a, gn,
