@@ -11,9 +11,9 @@
 // 4 * cells-per-tile consecutive particles holds about four per cell: the
 // phase kernel sums one such run per batch cell by cell, and
 // particles that stay in their tile keep this order from phase to phase.
-// A load from the caller's arrays gets there by tiles (counts, places and one
-// workgroup per tile); its largest tiles, and a binned source, by a stable LSD
-// radix sort (rocPRIM) of (key, source slot) pairs, whose result is the
+// A load of an FP64 engine gets there by tiles (counts, places and one workgroup
+// per tile); other loads, and a binned source, by a stable LSD radix sort
+// (rocPRIM) of (key, source slot) pairs, whose result is the
 // permutation; the seven arrays and the particle id are gathered to sorted
 // position i + tile * slack, so that every segment gets `slack` free slots
 // after its particles.  A binned source is enumerated densely through an
@@ -226,14 +226,14 @@ __global__ void k_bin_gather(Arrays7<TS> src, const uint32_t *__restrict__ src_i
 // 735 us for keys, radix sort and gather.  Most of a line's particles then lie
 // in different tiles: 490 MB are fetched for 232 MB of particles, 3.7 TB/s in
 // all.  Gathering component by component over all tiles instead fetches 797 MB
-// (281 us).  Tiles of more than kLoadHeld particles on average keep the radix
-// sort, whose work does not depend on the number of tiles.
+// (281 us).  Which loads go this way: load_through_tiles.
 constexpr int kLoadThreads = 1024;
 constexpr int kLoadManyTiles = 16384;
 constexpr int kLoadPer = 8;      // particles per thread that a tile's workgroup holds
 constexpr int kLoadHeld = kLoadThreads * kLoadPer;
 constexpr int kLoadStage = 4096;  // values staged in LDS at a time
 constexpr int kLoadRanks = 128;   // ranks in the slot tables
+constexpr int kLoadSorted = 512;  // particles of a cell that are put in caller order
 constexpr int kStoreThreads = 512;
 constexpr int kStorePer = 8;
 constexpr int kStoreHeld = kStoreThreads * kStorePer;
@@ -331,21 +331,35 @@ __device__ __forceinline__ T load_value(TS v, int a, int fixed, const FixedParam
   return (T)v;
 }
 
-// One workgroup per tile, tiles in runs per XCD: counts its cells, turns each
-// particle's rank within its cell into its slot in round-robin order (slot of
-// the k-th particle of cell c: particles of rank < k over all cells, plus the
-// cells before c that hold more than k; tables up to kLoadRanks ranks, a loop
-// over the cells beyond), then takes the components one after another: read in
-// the order of the places, where neighbours of the caller's arrays are mostly
-// neighbours, put at their slots in LDS and written in order.  A tile of more
-// than kLoadHeld particles ranks them in a second sweep and writes each at its
-// slot.
+// One workgroup per tile, tiles in runs per XCD: counts its cells, ranks each
+// particle within its cell, turns the rank into its slot in round-robin order
+// (slot of the k-th particle of cell c: particles of rank < k over all cells,
+// plus the cells before c that hold more than k; tables up to kLoadRanks ranks,
+// a loop over the cells beyond), then takes the components one after another:
+// read in the order of the places, where neighbours of the caller's arrays are
+// mostly neighbours, put at their slots in LDS and written in order.
+//
+// The places come in no particular order (atomics, workgroup by workgroup), the
+// ranks do: a cell's particles keep the caller's order, so that a load of the
+// same arrays always gives the same storage and its FP32 deposits sum in the same
+// order.  The indices are put in LDS cell by cell and each counts the smaller ones
+// of its cell, whole waves over one run of indices (the LDS reads are broadcast):
+// 4.0M FP64 particles on 1024 tiles 1 to 3% more for the load.
+// Cells of more than kLoadSorted particles keep the order of their places: the
+// count grows with the square.
+// A tile of more than kLoadHeld particles ranks them in a second sweep, in the
+// order of their places, and writes each at its slot.
 template <typename TS, typename T, int NC>
 __global__ __launch_bounds__(kLoadThreads) __attribute__((amdgpu_waves_per_eu(8)))
 void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint32_t *dst_id) {
   __shared__ unsigned int s_count[NC], s_rank[NC], s_A[kLoadRanks];
   __shared__ unsigned char s_T[NC][kLoadRanks];
-  __shared__ T s_stage[kLoadStage];
+  // the indices and their cells, cell by cell; then values by slot
+  __shared__ unsigned char s_cell[kLoadHeld];
+  constexpr int kKeyWords = kLoadHeld * 4, kStageBytes = kLoadStage * (int)sizeof(T);
+  __shared__ __align__(16) unsigned char s_mem[kKeyWords > kStageBytes ? kKeyWords : kStageBytes];
+  uint32_t *const s_key = reinterpret_cast<uint32_t *>(s_mem);
+  T *const s_stage = reinterpret_cast<T *>(s_mem);
   const int t = (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
   if (t >= L.ntiles) return;
   const int tid = threadIdx.x;
@@ -385,6 +399,12 @@ void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint3
       before += m > (unsigned)tid ? 1u : 0u;
     }
     s_A[tid] = a;
+  } else if (held && tid < kLoadRanks + NC) {
+    // first place of each cell's indices
+    unsigned int before = 0;
+#pragma unroll 8
+    for (int c = 0; c < NC; ++c) before += c < tid - kLoadRanks ? s_count[c] : 0u;
+    s_rank[tid - kLoadRanks] = before;
   }
   __syncthreads();
   auto slot = [&](unsigned int c, unsigned int k) -> unsigned int {
@@ -411,7 +431,36 @@ void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint3
   }
 #pragma unroll
   for (int e = 0; e < kLoadPer; ++e)
-    if (e * kLoadThreads + tid < n) pos[e] = slot(pos[e] & 0xffu, pos[e] >> 8);
+    if (e * kLoadThreads + tid < n) {
+      const unsigned int c = pos[e] & 0xffu, at = s_rank[c] + (pos[e] >> 8);
+      s_key[at] = j[e];
+      s_cell[at] = (unsigned char)c;
+      pos[e] = at;
+    }
+  __syncthreads();
+  uint32_t rank[kLoadPer];  // of the index at place e * kLoadThreads + tid
+#pragma unroll
+  for (int e = 0; e < kLoadPer; ++e) {
+    const int at = e * kLoadThreads + tid;
+    if (at >= n) break;
+    const unsigned int c = s_cell[at], first = s_rank[c], m = s_count[c];
+    rank[e] = (unsigned)at - first;
+    if (m <= (unsigned)kLoadSorted) {
+      const uint32_t key = s_key[at];
+      rank[e] = 0u;
+#pragma unroll 4
+      for (unsigned int i = 0; i < m; ++i) rank[e] += s_key[first + i] < key ? 1u : 0u;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < kLoadPer; ++e)
+    if (e * kLoadThreads + tid < n) s_key[e * kLoadThreads + tid] = rank[e];
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < kLoadPer; ++e)
+    if (e * kLoadThreads + tid < n) pos[e] = slot(s_cell[pos[e]], s_key[pos[e]]);
+  __syncthreads();
 #pragma unroll
   for (int a = 0; a < 7; ++a) {
     T val[kLoadPer];
@@ -1317,7 +1366,13 @@ hipError_t phase_start(const CountArrays &c, hipStream_t s) {
 // average, and workgroups can count them in LDS (beyond kLdsTiles those of 1024
 // threads, for enough particles).  28.8M FP32 particles on 16640 tiles, counted
 // with global atomics: 5.75 ms, 5.0 by the radix sort; 2.1M 505 / 390 us.
+// FP32 engines keep the radix sort, though tiles take half its time (4.0M
+// particles 519 / 969 us): their deposits sum in the load's order, with few
+// particles per cell the same to the last bit each time, and another order gives
+// other roundings.
+template <typename T>
 inline bool load_through_tiles(int64_t n, int ntiles) {
+  if (sizeof(T) == 4) return false;
   return n <= (int64_t)kLoadHeld * ntiles &&
          (ntiles <= kLdsTiles || (ntiles <= kLoadManyTiles && n >= 256 * 1024 * 16));
 }
@@ -1416,7 +1471,7 @@ hipError_t bin_sort(const KGrid<T> &g, const BinLayout &L, int64_t n,
   const size_t a_c = align_up(sizeof(uint32_t) * (size_t)ncell);
   const int shift = L.rank_bits + L.cell_bits;
   const int key_bits = L.tile_bits + shift;
-  if (!binned && load_through_tiles(n, L.ntiles)) {
+  if (!binned && load_through_tiles<T>(n, L.ntiles)) {
     const size_t a_w = align_up(2 * sizeof(uint32_t) * nt1);
     const size_t total = a_w + 2 * a_n;
     if (needed) *needed = total;
