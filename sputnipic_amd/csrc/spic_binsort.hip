@@ -1370,9 +1370,14 @@ hipError_t phase_start(const CountArrays &c, hipStream_t s) {
 // particles 519 / 969 us): their deposits sum in the load's order, with few
 // particles per cell the same to the last bit each time, and another order gives
 // other roundings.
+// Many tiles of a few particles each, whose workgroups are mostly tables, keep
+// the radix sort too (FP64, tiles / radix, us): 2048 tiles of 1 / 8 / 32
+// particles 61 / 71, 69 / 83, 73 / 99; 3072 75 / 70, 89 / 92, 98 / 113; 4096
+// 89 / 71, 109 / 95, 121 / 120; 5120 105 / 83, 129 / 101, 145 / 128.  From 64 on
+// tiles win (4096: 144 / 167, 5120: 171 / 192).
 template <typename T>
 inline bool load_through_tiles(int64_t n, int ntiles) {
-  if (sizeof(T) == 4) return false;
+  if (sizeof(T) == 4 || (ntiles > 2048 && n < 64 * (int64_t)ntiles)) return false;
   return n <= (int64_t)kLoadHeld * ntiles &&
          (ntiles <= kLdsTiles || (ntiles <= kLoadManyTiles && n >= 256 * 1024 * 16));
 }

@@ -48,6 +48,8 @@ CASES = [
     # as many per cell, cell by cell (a cell's particles in one wave)
     ((13, 9, 6), 2, "cells"), ((13, 9, 6), 8, "cells"), ((5, 4, 4), 64, "cells"),
     ((16, 16, 16), 32, "cells"), ((40, 32, 30), 1, "cells"),
+    # 2197 tiles of 64 particles, and of fewer
+    ((52, 52, 52), 1, "cells"), ((52, 52, 51), 1, "cells"),
 ]
 
 
