@@ -345,6 +345,8 @@ struct TileSortJob {
   unsigned int *dst_cnt;
   unsigned int ovf_cap;
   unsigned int *count, *own, *fill;
+  unsigned int *big;  // of a load (spic_binsort.hip, LoadBins); else null
+  uint4 *pieces;
 };
 
 // Workgroups of the count and sort launches per job: one per tile, plus

@@ -251,16 +251,21 @@ struct LoadBins {
   const int64_t *seg;      // the segments: tile t's places begin at seg[t] - t * slack
   uint32_t *where;         // [n] tile | cell in the tile (cell_bits)
   uint32_t *perm;          // [n] by place: index of the particle
+  // tiles of more than kLoadHeld particles, in pieces of that many
+  unsigned int *big;       // [0] pieces, [1] such tiles
+  uint4 *pieces;           // tile, number among those tiles, first place, 0
+  unsigned int *cells;     // [2 NC] of each such tile: particles per cell, ranks taken
+  int tile_blocks;         // workgroups of whole tiles, before those of pieces
 };
 
 // Counts the particles into tiles, NT threads per workgroup, which counts up to
 // LT tiles in LDS and adds each tile it met once; LT = 0: one atomic per wave and
 // tile in global memory.
-template <typename TS, typename T, int NT, int LT>
-__global__ __launch_bounds__(NT) void k_load_count(KGrid<T> g, BinLayout L, LoadBins b,
-                                                   const TS *__restrict__ x,
-                                                   const TS *__restrict__ y,
-                                                   const TS *__restrict__ z) {
+template <int NT, int LT>
+__global__ __launch_bounds__(NT) void k_load_count(KGrid<double> g, BinLayout L, LoadBins b,
+                                                   const double *__restrict__ x,
+                                                   const double *__restrict__ y,
+                                                   const double *__restrict__ z) {
   __shared__ unsigned int s_cnt[LT > 0 ? LT : 1];
   const int tid = threadIdx.x;
   if constexpr (LT > 0) {
@@ -321,16 +326,6 @@ __global__ __launch_bounds__(NT) void k_load_place(BinLayout L, LoadBins b) {
   }
 }
 
-// A caller's value into binned storage: with fixed-point storage positions
-// are converted, everything else is rounded to T.
-template <typename TS, typename T>
-__device__ __forceinline__ T load_value(TS v, int a, int fixed, const FixedParams &fx) {
-  if constexpr (sizeof(T) == 4) {
-    if (a < 3 && fixed) return __int_as_float(to_fixed_pos((double)v, fx, a));
-  }
-  return (T)v;
-}
-
 // One workgroup per tile, tiles in runs per XCD: counts its cells, ranks each
 // particle within its cell, turns the rank into its slot in round-robin order
 // (slot of the k-th particle of cell c: particles of rank < k over all cells,
@@ -341,54 +336,87 @@ __device__ __forceinline__ T load_value(TS v, int a, int fixed, const FixedParam
 //
 // The places come in no particular order (atomics, workgroup by workgroup), the
 // ranks do: a cell's particles keep the caller's order, so that a load of the
-// same arrays always gives the same storage and its FP32 deposits sum in the same
-// order.  The indices are put in LDS cell by cell and each counts the smaller ones
+// same arrays always gives the same storage.  The indices are put in LDS cell by cell and each counts the smaller ones
 // of its cell, whole waves over one run of indices (the LDS reads are broadcast):
 // 4.0M FP64 particles on 1024 tiles 1 to 3% more for the load.
 // Cells of more than kLoadSorted particles keep the order of their places: the
 // count grows with the square.
-// A tile of more than kLoadHeld particles ranks them in a second sweep, in the
-// order of their places, and writes each at its slot.
-template <typename TS, typename T, int NC>
+// A tile of more than kLoadHeld particles is taken in pieces, a workgroup each:
+// the cells are counted over all of them first (k_load_pieces), a piece takes its
+// ranks of each cell at once, in the order of the places, and writes every
+// particle at its slot.  3.6M of 4.0M FP64 particles in one of 512 tiles:
+// 0.94 ms (one workgroup for the tile 50, the radix sort 2.4), in one cell of it
+// 0.32 (25, 1.08).  Where no tile is that full the two additions cost 3 us.
+template <int NC>
+__global__ __launch_bounds__(kLoadThreads) void k_load_pieces(BinLayout L, LoadBins b) {
+  __shared__ unsigned int s_count[NC];
+  if (blockIdx.x >= b.big[0]) return;
+  const int tid = threadIdx.x;
+  const uint4 piece = b.pieces[blockIdx.x];
+  const int t = (int)piece.x;
+  const int n = min(b.count[t] - piece.z, (unsigned)kLoadHeld);
+  const uint32_t *perm = b.perm + (b.seg[t] - (int64_t)t * L.slack) + piece.z;
+  const uint32_t mask = (1u << L.cell_bits) - 1u;
+  if (tid < NC) s_count[tid] = 0u;
+  __syncthreads();
+  for (int r = tid; r < (n + 63) / 64 * 64; r += kLoadThreads)
+    key_rank(s_count, r < n ? b.where[perm[r]] & mask : 0u, r < n);
+  __syncthreads();
+  if (tid < NC && s_count[tid]) atomicAdd(b.cells + (size_t)piece.y * 2 * NC + tid, s_count[tid]);
+}
+
+template <int NC>
 __global__ __launch_bounds__(kLoadThreads) __attribute__((amdgpu_waves_per_eu(8)))
-void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint32_t *dst_id) {
-  __shared__ unsigned int s_count[NC], s_rank[NC], s_A[kLoadRanks];
+void k_load_tile(BinLayout L, LoadBins b, Arrays7<double> src, Arrays7<double> dst,
+                 uint32_t *dst_id) {
+  // particles per cell; a whole tile's first place of each cell's indices, or
+  // the first rank of a piece's in each cell
+  __shared__ unsigned int s_count[NC], s_first[NC], s_A[kLoadRanks];
   __shared__ unsigned char s_T[NC][kLoadRanks];
   // the indices and their cells, cell by cell; then values by slot
   __shared__ unsigned char s_cell[kLoadHeld];
-  constexpr int kKeyWords = kLoadHeld * 4, kStageBytes = kLoadStage * (int)sizeof(T);
-  __shared__ __align__(16) unsigned char s_mem[kKeyWords > kStageBytes ? kKeyWords : kStageBytes];
-  uint32_t *const s_key = reinterpret_cast<uint32_t *>(s_mem);
-  T *const s_stage = reinterpret_cast<T *>(s_mem);
-  const int t = (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
-  if (t >= L.ntiles) return;
+  __shared__ double s_stage[kLoadStage];
+  uint32_t *const s_key = reinterpret_cast<uint32_t *>(s_stage);
+  static_assert(2 * kLoadStage >= kLoadHeld, "room for the indices");
   const int tid = threadIdx.x;
-  const int64_t n64 = b.count[t], out0 = b.seg[t];
-  if (n64 == 0) return;
-  const uint32_t *perm = b.perm + (out0 - (int64_t)t * L.slack);
+  const bool whole = (int)blockIdx.x < b.tile_blocks;
+  int t;
+  uint4 piece = make_uint4(0u, 0u, 0u, 0u);
+  if (whole) {
+    t = (int)((blockIdx.x % 8) * (b.tile_blocks / 8) + blockIdx.x / 8);
+    if (t >= L.ntiles || b.count[t] == 0u || b.count[t] > (unsigned)kLoadHeld) return;
+  } else {
+    if (blockIdx.x - b.tile_blocks >= b.big[0]) return;
+    piece = b.pieces[blockIdx.x - b.tile_blocks];
+    t = (int)piece.x;
+  }
+  const int64_t out0 = b.seg[t];
+  const int n = min(b.count[t] - piece.z, (unsigned)kLoadHeld);
+  const uint32_t *perm = b.perm + (out0 - (int64_t)t * L.slack) + piece.z;
   const uint32_t mask = (1u << L.cell_bits) - 1u;
-  const bool held = n64 <= kLoadHeld;
-  const int n = held ? (int)n64 : 0;
-  for (int c = tid; c < NC; c += kLoadThreads) s_count[c] = s_rank[c] = 0u;
+  if (tid < NC) s_count[tid] = 0u;
   __syncthreads();
   uint32_t j[kLoadPer], pos[kLoadPer];  // index; rank and cell, then slot
-  if (held) {
 #pragma unroll
-    for (int e = 0; e < kLoadPer; ++e) {
-      const int r = e * kLoadThreads + tid;
-      if (r < n) j[e] = perm[r];
-    }
-#pragma unroll
-    for (int e = 0; e < kLoadPer; ++e)
-      if (e * kLoadThreads + tid < n) pos[e] = b.where[j[e]] & mask;
-#pragma unroll
-    for (int e = 0; e < kLoadPer; ++e)
-      if (e * kLoadThreads + tid < n) pos[e] |= atomicAdd(&s_count[pos[e]], 1u) << 8;
-  } else {
-    for (int64_t r = tid; r < n64; r += kLoadThreads)
-      atomicAdd(&s_count[b.where[perm[r]] & mask], 1u);
+  for (int e = 0; e < kLoadPer; ++e) {
+    const int r = e * kLoadThreads + tid;
+    if (r < n) j[e] = perm[r];
   }
+#pragma unroll
+  for (int e = 0; e < kLoadPer; ++e)
+    if (e * kLoadThreads + tid < n) pos[e] = b.where[j[e]] & mask;
+#pragma unroll
+  for (int e = 0; e < kLoadPer; ++e)
+    if (e * kLoadThreads + tid < n) pos[e] |= atomicAdd(&s_count[pos[e]], 1u) << 8;
   __syncthreads();
+  if (!whole) {
+    if (tid < NC) {
+      unsigned int *cells = b.cells + (size_t)piece.y * 2 * NC;
+      s_first[tid] = s_count[tid] ? atomicAdd(cells + NC + tid, s_count[tid]) : 0u;
+      s_count[tid] = cells[tid];
+    }
+    __syncthreads();
+  }
   if (tid < kLoadRanks) {
     unsigned int a = 0, before = 0;
 #pragma unroll 8
@@ -399,12 +427,11 @@ void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint3
       before += m > (unsigned)tid ? 1u : 0u;
     }
     s_A[tid] = a;
-  } else if (held && tid < kLoadRanks + NC) {
-    // first place of each cell's indices
+  } else if (whole && tid < kLoadRanks + NC) {
     unsigned int before = 0;
 #pragma unroll 8
     for (int c = 0; c < NC; ++c) before += c < tid - kLoadRanks ? s_count[c] : 0u;
-    s_rank[tid - kLoadRanks] = before;
+    s_first[tid - kLoadRanks] = before;
   }
   __syncthreads();
   auto slot = [&](unsigned int c, unsigned int k) -> unsigned int {
@@ -418,21 +445,22 @@ void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint3
     }
     return p;
   };
-  if (!held) {
-    for (int64_t r = tid; r < n64; r += kLoadThreads) {
-      const uint32_t i = perm[r], c = b.where[i] & mask;
-      const int64_t o = out0 + slot(c, atomicAdd(&s_rank[c], 1u));
+  if (!whole) {
 #pragma unroll
-      for (int a = 0; a < 7; ++a)
-        dst.p[a][o] = load_value<TS, T>(src.p[a][i], a, L.fixed, L.fx);
-      if (dst_id) dst_id[o] = i;
-    }
+    for (int e = 0; e < kLoadPer; ++e)
+      if (e * kLoadThreads + tid < n) {
+        const unsigned int c = pos[e] & 0xffu;
+        const int64_t o = out0 + slot(c, s_first[c] + (pos[e] >> 8));
+#pragma unroll
+        for (int a = 0; a < 7; ++a) dst.p[a][o] = src.p[a][j[e]];
+        if (dst_id) dst_id[o] = j[e];
+      }
     return;
   }
 #pragma unroll
   for (int e = 0; e < kLoadPer; ++e)
     if (e * kLoadThreads + tid < n) {
-      const unsigned int c = pos[e] & 0xffu, at = s_rank[c] + (pos[e] >> 8);
+      const unsigned int c = pos[e] & 0xffu, at = s_first[c] + (pos[e] >> 8);
       s_key[at] = j[e];
       s_cell[at] = (unsigned char)c;
       pos[e] = at;
@@ -443,7 +471,7 @@ void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint3
   for (int e = 0; e < kLoadPer; ++e) {
     const int at = e * kLoadThreads + tid;
     if (at >= n) break;
-    const unsigned int c = s_cell[at], first = s_rank[c], m = s_count[c];
+    const unsigned int c = s_cell[at], first = s_first[c], m = s_count[c];
     rank[e] = (unsigned)at - first;
     if (m <= (unsigned)kLoadSorted) {
       const uint32_t key = s_key[at];
@@ -463,12 +491,11 @@ void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint3
   __syncthreads();
 #pragma unroll
   for (int a = 0; a < 7; ++a) {
-    T val[kLoadPer];
+    double val[kLoadPer];
 #pragma unroll
     for (int e = 0; e < kLoadPer; ++e)
-      if (e * kLoadThreads + tid < n)
-        val[e] = load_value<TS, T>(src.p[a][j[e]], a, L.fixed, L.fx);
-    T *__restrict__ to = dst.p[a] + out0;
+      if (e * kLoadThreads + tid < n) val[e] = src.p[a][j[e]];
+    double *__restrict__ to = dst.p[a] + out0;
     for (int c0 = 0; c0 < n; c0 += kLoadStage) {
 #pragma unroll
       for (int e = 0; e < kLoadPer; ++e)
@@ -1033,6 +1060,12 @@ __device__ __forceinline__ void tile_bounds_body(const TileSortJob<T> &J) {
       gmem(J.dst_cnt)[2 * (nt + 1) + t] = 0u;
       gmem(J.dst_cnt)[3 * (nt + 1) + t] = 0u;
     }
+    if (J.big && c > (unsigned)kLoadHeld) {
+      const unsigned int pieces = (c + kLoadHeld - 1) / kLoadHeld;
+      const unsigned int number = atomicAdd(J.big + 1, 1u), at = atomicAdd(J.big, pieces);
+      for (unsigned int k = 0; k < pieces; ++k)
+        J.pieces[at + k] = make_uint4((unsigned)t, number, k * kLoadHeld, 0u);
+    }
     __syncthreads();
     if (tid == 0) s_carry = carry + s_wsum[NW - 1];
     __syncthreads();
@@ -1375,22 +1408,40 @@ hipError_t phase_start(const CountArrays &c, hipStream_t s) {
 // particles 61 / 71, 69 / 83, 73 / 99; 3072 75 / 70, 89 / 92, 98 / 113; 4096
 // 89 / 71, 109 / 95, 121 / 120; 5120 105 / 83, 129 / 101, 145 / 128.  From 64 on
 // tiles win (4096: 144 / 167, 5120: 171 / 192).
-template <typename T>
 inline bool load_through_tiles(int64_t n, int ntiles) {
-  if (sizeof(T) == 4 || (ntiles > 2048 && n < 64 * (int64_t)ntiles)) return false;
+  if (ntiles > 2048 && n < 64 * (int64_t)ntiles) return false;
   return n <= (int64_t)kLoadHeld * ntiles &&
          (ntiles <= kLdsTiles || (ntiles <= kLoadManyTiles && n >= 256 * 1024 * 16));
 }
 
-// The load of a dense source through tiles.  Workspace: two words per tile,
-// two per particle.
-template <typename TS, typename T>
-hipError_t load_tiles(const KGrid<T> &g, const BinLayout &L, int64_t n, const void *const src[7],
-                      T *const dst[7], uint32_t *dst_id, int64_t *dst_seg,
-                      unsigned int *dst_cnt, char *w, size_t a_t, size_t a_n, hipStream_t s) {
+// The workspace of such a load: two words per tile, the counters of the tiles
+// taken in pieces (all of these zeroed first), the pieces, two words per particle.
+struct LoadSpace {
+  int64_t zeroed;       // words
+  unsigned int pieces;  // at most
+  size_t a_zeroed, a_pieces, a_n, total;
+};
+
+inline LoadSpace load_space(const BinLayout &L, int64_t n) {
+  const int64_t big = n / kLoadHeld < L.ntiles ? n / kLoadHeld : L.ntiles;
+  LoadSpace sp;
+  sp.zeroed = 2 * ((int64_t)L.ntiles + 1) + 2 + big * 2 * (L.tx * L.ty * L.tz);
+  sp.pieces = (unsigned)(n > kLoadHeld ? n / kLoadHeld + big : 0);
+  sp.a_zeroed = align_up(sizeof(unsigned int) * (size_t)sp.zeroed);
+  sp.a_pieces = align_up(sizeof(uint4) * (size_t)sp.pieces);
+  sp.a_n = align_up(sizeof(uint32_t) * (size_t)(n > 0 ? n : 1));
+  sp.total = sp.a_zeroed + sp.a_pieces + 2 * sp.a_n;
+  return sp;
+}
+
+// The load of a dense source through tiles.
+inline hipError_t load_tiles(const KGrid<double> &g, const BinLayout &L, int64_t n,
+                             const void *const src[7], double *const dst[7],
+                             uint32_t *dst_id, int64_t *dst_seg, unsigned int *dst_cnt, char *w,
+                             const LoadSpace &sp, hipStream_t s) {
   const int nc = L.tx * L.ty * L.tz;
   if (nc != 64 && nc != 128) return hipErrorInvalidValue;
-  TileSortJob<T> J;
+  TileSortJob<double> J;
   std::memset(&J, 0, sizeof(J));
   J.L = L;
   J.dst_seg = dst_seg;
@@ -1401,38 +1452,43 @@ hipError_t load_tiles(const KGrid<T> &g, const BinLayout &L, int64_t n, const vo
   b.count = J.count;
   b.next = J.count + L.ntiles + 1;
   b.seg = dst_seg;
-  b.where = (uint32_t *)(w + a_t);
-  b.perm = (uint32_t *)(w + a_t + a_n);
+  b.big = b.next + L.ntiles + 1;
+  b.cells = b.big + 2;
+  b.pieces = (uint4 *)(w + sp.a_zeroed);
+  b.where = (uint32_t *)(w + sp.a_zeroed + sp.a_pieces);
+  b.perm = (uint32_t *)(w + sp.a_zeroed + sp.a_pieces + sp.a_n);
+  b.tile_blocks = (L.ntiles + 7) / 8 * 8;
+  J.big = sp.pieces ? b.big : nullptr;
+  J.pieces = b.pieces;
   // many tiles: workgroups of 1024 threads and 64 KB of counters, 16384
   // particles each, where that leaves one per CU
   const bool many = L.ntiles > kLdsTiles;
   const int64_t per = n / (256 * 2048);
   b.per = many || per > 16 ? 16 : per < 1 ? 1 : (int)per;
-  Arrays7<TS> as;
-  Arrays7<T> ad;
+  Arrays7<double> as, ad;
   for (int a = 0; a < 7; ++a) {
-    as.p[a] = (TS *)src[a];
+    as.p[a] = (double *)src[a];
     ad.p[a] = dst[a];
   }
-  const int64_t nzero = 2 * ((int64_t)L.ntiles + 1);
-  hipLaunchKernelGGL(k_zero_u32, dim3(nblocks(nzero)), dim3(256), 0, s, J.count, nzero);
+  hipLaunchKernelGGL(k_zero_u32, dim3(nblocks((long)sp.zeroed)), dim3(256), 0, s, J.count,
+                     sp.zeroed);
   hipError_t e;
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (n > 0) {
     const int nt = many ? 1024 : 256;
     const dim3 grid((unsigned)((n + nt * b.per - 1) / (nt * b.per)));
     if (many)
-      hipLaunchKernelGGL((k_load_count<TS, T, 1024, kLoadManyTiles>), grid, dim3(1024), 0, s, g,
+      hipLaunchKernelGGL((k_load_count<1024, kLoadManyTiles>), grid, dim3(1024), 0, s, g,
                          L, b, as.p[0], as.p[1], as.p[2]);
     else if (L.ntiles <= kLdsTiles && L.ntiles <= 8 * 256 * b.per)
-      hipLaunchKernelGGL((k_load_count<TS, T, 256, kLdsTiles>), grid, dim3(256), 0, s, g, L, b,
+      hipLaunchKernelGGL((k_load_count<256, kLdsTiles>), grid, dim3(256), 0, s, g, L, b,
                          as.p[0], as.p[1], as.p[2]);
     else
-      hipLaunchKernelGGL((k_load_count<TS, T, 256, 0>), grid, dim3(256), 0, s, g, L, b, as.p[0],
+      hipLaunchKernelGGL((k_load_count<256, 0>), grid, dim3(256), 0, s, g, L, b, as.p[0],
                          as.p[1], as.p[2]);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k_tile_bounds<T>, dim3(1), dim3(kScanThreads), 0, s, J);
+  hipLaunchKernelGGL(k_tile_bounds<double>, dim3(1), dim3(kScanThreads), 0, s, J);
   if ((e = hipGetLastError()) != hipSuccess || n == 0) return e;
   // places by workgroup or by wave, as the deposit through tiles takes them
   auto blocks = [n](int per) { return dim3((unsigned)((n + 256 * per - 1) / (256 * per))); };
@@ -1446,13 +1502,14 @@ hipError_t load_tiles(const KGrid<T> &g, const BinLayout &L, int64_t n, const vo
   else
     hipLaunchKernelGGL((k_load_place<1, 256, 0>), blocks(1), dim3(256), 0, s, L, b);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  const dim3 tiles((unsigned)((L.ntiles + 7) / 8 * 8));
-  if (nc == 64)
-    hipLaunchKernelGGL((k_load_tile<TS, T, 64>), tiles, dim3(kLoadThreads), 0, s, L, b, as, ad,
-                       dst_id);
-  else
-    hipLaunchKernelGGL((k_load_tile<TS, T, 128>), tiles, dim3(kLoadThreads), 0, s, L, b, as, ad,
-                       dst_id);
+  const dim3 threads(kLoadThreads), grid(b.tile_blocks + sp.pieces);
+  if (nc == 64) {
+    if (sp.pieces) hipLaunchKernelGGL((k_load_pieces<64>), dim3(sp.pieces), threads, 0, s, L, b);
+    hipLaunchKernelGGL((k_load_tile<64>), grid, threads, 0, s, L, b, as, ad, dst_id);
+  } else {
+    if (sp.pieces) hipLaunchKernelGGL((k_load_pieces<128>), dim3(sp.pieces), threads, 0, s, L, b);
+    hipLaunchKernelGGL((k_load_tile<128>), grid, threads, 0, s, L, b, as, ad, dst_id);
+  }
   return hipGetLastError();
 }
 
@@ -1476,17 +1533,14 @@ hipError_t bin_sort(const KGrid<T> &g, const BinLayout &L, int64_t n,
   const size_t a_c = align_up(sizeof(uint32_t) * (size_t)ncell);
   const int shift = L.rank_bits + L.cell_bits;
   const int key_bits = L.tile_bits + shift;
-  if (!binned && load_through_tiles<T>(n, L.ntiles)) {
-    const size_t a_w = align_up(2 * sizeof(uint32_t) * nt1);
-    const size_t total = a_w + 2 * a_n;
-    if (needed) *needed = total;
-    if (!workspace) return hipSuccess;
-    if (workspace_bytes < total) return hipErrorInvalidValue;
-    return widened ? load_tiles<double, T>(g, L, n, src, dst, dst_id, dst_seg, dst_cnt,
-                                           (char *)workspace, a_w, a_n, s)
-                   : load_tiles<T, T>(g, L, n, src, dst, dst_id, dst_seg, dst_cnt,
-                                      (char *)workspace, a_w, a_n, s);
-  }
+  if constexpr (sizeof(T) == 8)
+    if (!binned && load_through_tiles(n, L.ntiles)) {
+      const LoadSpace sp = load_space(L, n);
+      if (needed) *needed = sp.total;
+      if (!workspace) return hipSuccess;
+      if (workspace_bytes < sp.total) return hipErrorInvalidValue;
+      return load_tiles(g, L, n, src, dst, dst_id, dst_seg, dst_cnt, (char *)workspace, sp, s);
+    }
   size_t sort_bytes = 0, scan_bytes = 0;
   hipError_t e = rocprim::radix_sort_pairs(
       nullptr, sort_bytes, (uint32_t *)nullptr, (uint32_t *)nullptr,
