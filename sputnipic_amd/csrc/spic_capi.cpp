@@ -64,11 +64,32 @@ struct StatusBuf {
   // others may write the words too: a captured graph's replays, a batch run by
   // another thread
   bool shared = false;
-  bool maybe_set = false;  // a call since the last read may have set a word
+  bool set = false;  // maybe set by work that has ended
+  // streams with asynchronous calls whose end has not been waited for (a
+  // destroyed stream's work has ended: hipStreamDestroy waits, 76 ms for as much)
+  hipStream_t writers[4];
+  int nwriters = 0;
+
+  bool clean() const { return !shared && !set && nwriters == 0; }
+  void will_write(hipStream_t s) {
+    for (int i = 0; i < nwriters; ++i)
+      if (writers[i] == s) return;
+    if (nwriters == 4) shared = true;  // too many to follow
+    else writers[nwriters++] = s;
+  }
+  bool waited_for(hipStream_t s) {
+    for (int i = 0; i < nwriters; ++i)
+      if (writers[i] == s) {
+        writers[i] = writers[--nwriters];
+        return true;
+      }
+    return false;
+  }
 };
 // Words of threads that have ended, for the next ones: those that nothing can
-// write any more and that were last read as zeros.  Never destroyed, since
-// threads may end after static objects have.
+// write any more (every stream with asynchronous calls has been waited for) and
+// that were last read as zeros.  Never destroyed, since threads may end after
+// static objects have.
 struct StatusFree {
   std::mutex mutex;
   std::vector<StatusBuf> bufs;
@@ -82,8 +103,11 @@ struct ThreadStatus {
   ~ThreadStatus() {
     StatusFree &f = status_free();
     std::lock_guard<std::mutex> lock(f.mutex);
-    for (const auto &sb : bufs)
-      if (!sb.shared && !sb.maybe_set) f.bufs.push_back(sb);
+    try {
+      for (const auto &sb : bufs)
+        if (sb.clean()) f.bufs.push_back(sb);
+    } catch (const std::bad_alloc &) {  // the rest is not handed on
+    }
   }
 };
 thread_local ThreadStatus t_thread_status;
@@ -95,6 +119,12 @@ StatusBuf *status_words(hipError_t *err) {
   std::vector<StatusBuf> &t_status = t_thread_status.bufs;
   for (auto &sb : t_status)
     if (sb.device == dev) return &sb;
+  try {
+    t_status.reserve(t_status.size() + 1);
+  } catch (const std::bad_alloc &) {
+    *err = hipErrorOutOfMemory;
+    return nullptr;
+  }
   {
     StatusFree &f = status_free();
     std::lock_guard<std::mutex> lock(f.mutex);
@@ -119,6 +149,18 @@ StatusBuf *status_words(hipError_t *err) {
   }
   t_status.push_back(sb);
   return &t_status.back();
+}
+
+// The thread has waited for stream s, or for all of the device's.
+static void status_waited(bool all, hipStream_t s) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return;
+  for (auto &sb : t_thread_status.bufs)
+    if (sb.device == dev) {
+      if (all && sb.nwriters) sb.set = true;
+      if (all) sb.nwriters = 0;
+      else if (sb.waited_for(s)) sb.set = true;
+    }
 }
 
 unsigned int *status_buffer(hipError_t *err) {
@@ -296,19 +338,23 @@ bool strict_mode() { return g_strict.load() != 0; }
 int subcycle_mode() { return g_subcycle.load(); }
 
 // Prepare the status words for one call; returns the device pointer.  A
-// synchronous call starts from zero words: they are zero unless something may
-// have set one since they were last read as zeros.
+// synchronous call starts from zero words: they are zero unless a read left them
+// set or something else may write them.
 int begin_call(hipStream_t s, unsigned int **st) {
   hipError_t e;
   StatusBuf *sb = status_words(&e);
   if (!sb) return hip_fail(e, "status buffer");
   *st = sb->d;
-  if (!g_async.load() && (sb->shared || sb->maybe_set)) {
+  if (g_async.load()) {
+    sb->will_write(s);
+    if (!stream_may_alloc(s)) sb->shared = true;  // being captured
+    return SPIC_OK;
+  }
+  if (!sb->clean()) {
     e = spic::zero_u32(sb->d, 3, s);
     if (e != hipSuccess) return hip_fail(e, "status reset");
   }
-  sb->maybe_set = true;
-  if (g_async.load() && !stream_may_alloc(s)) sb->shared = true;  // being captured
+  sb->set = true;  // until it has been read
   return SPIC_OK;
 }
 
@@ -321,13 +367,16 @@ static int read_status(hipStream_t s, StatusBuf *sb, bool clear) {
   if (e != hipSuccess) return hip_fail(e, "status readback");
   e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hip_fail(e, "kernel execution");
+  (void)sb->waited_for(s);
   const unsigned int h[3] = {sb->h[0], sb->h[1], sb->h[2]};
-  const bool set = h[0] || h[1] || h[2];
-  if (clear && set) {
-    e = hipMemset(sb->d, 0, sizeof(h));
-    if (e != hipSuccess) return hip_fail(e, "status reset");
+  sb->set = h[0] || h[1] || h[2];
+  if (clear && sb->set) {
+    // waited for, since the next call may run on another stream and not reset
+    if ((e = spic::zero_u32(sb->d, 3, s)) != hipSuccess ||
+        (e = hipStreamSynchronize(s)) != hipSuccess)
+      return hip_fail(e, "status reset");
+    sb->set = false;
   }
-  sb->maybe_set = set && !clear;
   if (h[2])
     return fail(SPIC_ENOMEM,
                 "engine particle storage full: %u workgroups could not place "
@@ -558,6 +607,7 @@ int spic_memset(void *dptr, int value, size_t bytes) {
 
 int spic_synchronize(void) {
   hipError_t e = hipDeviceSynchronize();
+  if (e == hipSuccess) spic::status_waited(true, nullptr);
   return e == hipSuccess ? SPIC_OK : hip_fail(e, "hipDeviceSynchronize");
 }
 
@@ -600,6 +650,7 @@ int spic_stream_destroy(void *stream) {
 
 int spic_stream_synchronize(void *stream) {
   hipError_t e = hipStreamSynchronize((hipStream_t)stream);
+  if (e == hipSuccess) spic::status_waited(false, (hipStream_t)stream);
   return e == hipSuccess ? SPIC_OK : hip_fail(e, "hipStreamSynchronize");
 }
 
