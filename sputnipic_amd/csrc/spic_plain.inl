@@ -259,7 +259,8 @@ __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 4)))
 void k_mover(KGrid<T> g, FV f, KPart<T> p, KPush<T> k, unsigned int *status) {
   bool bad = false;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < p.n;
+  // unsigned: the last index plus the grid does not fit an int near 2^31
+  for (unsigned int i = blockIdx.x * kBlock + threadIdx.x; i < (unsigned)p.n;
        i += gridDim.x * kBlock) {
     T x = p.x[i], y = p.y[i], z = p.z[i], u = p.u[i], v = p.v[i], w = p.w[i];
     bad |= push_particle(g, f, k, x, y, z, u, v, w);
@@ -345,6 +346,34 @@ __global__ __launch_bounds__(64) void k_deposit(KGrid<T> g, KPart<T> p, KMom m,
   flush();
 }
 
+// Calls f(first, count) for n items in runs of at most `slice`, until it returns
+// false.  In 64 bits: the run after the last one of a species of 2^31 - 1
+// particles starts beyond an int.
+template <typename F>
+constexpr void for_slices(int64_t n, int64_t slice, F f) {
+  for (int64_t first = 0; first < n; first += slice)
+    if (!f(first, n - first < slice ? n - first : slice)) return;
+}
+constexpr int64_t slices_sum(int64_t n, int64_t slice) {
+  int64_t sum = 0;
+  for_slices(n, slice, [&sum, slice](int64_t first, int64_t count) {
+    const bool next = first == sum && count > 0 && count <= slice;
+    sum += count;
+    return next;
+  });
+  return sum;
+}
+
+template <typename T>
+KPart<T> part_slice(const KPart<T> &p, int64_t first, int64_t count) {
+  KPart<T> q = p;
+  q.x += first; q.y += first; q.z += first;
+  q.u += first; q.v += first; q.w += first;
+  q.q += first;
+  q.n = (int)count;
+  return q;
+}
+
 static inline unsigned grid_for(int n) {
   long blocks = ((long)n + kBlock - 1) / kBlock;
   if (blocks < 1) blocks = 1;
@@ -372,6 +401,12 @@ constexpr int kDepBatch = 512;         // particles staged in LDS at a time
 constexpr int kDepMaxRun = 4096;       // particles per workgroup at most
 constexpr int kDepSlice = 1 << 24;     // particles binned at a time (24-bit indices)
 constexpr uint32_t kDepIndexMask = (1u << 24) - 1u;
+static_assert(slices_sum(2147483647, kDepSlice) == 2147483647 &&
+                  slices_sum(kDepSlice, kDepSlice) == kDepSlice &&
+                  slices_sum(kDepSlice + 1, kDepSlice) == kDepSlice + 1 &&
+                  slices_sum(127 * (int64_t)kDepSlice + 1, kDepSlice) ==
+                      127 * (int64_t)kDepSlice + 1,
+              "every particle in one slice");
 
 struct DepBins {
   int nty, ntz, ntiles;
@@ -712,13 +747,9 @@ hipError_t tile_deposit(const KGrid<T> &g, const KField<T> *f, const KPart<T> &p
   b.perm = (unsigned int *)(w + a_cnt + a_next + a_items + a_n);
   const PackedField<T> packed{(const T *)(w + a_cnt + a_next + a_items + 2 * a_n)};
   if (pack) pack_fields(*f, packed, nn, s);
-  for (int first = 0; first < p.n && e == hipSuccess; first += slice) {
-    KPart<T> q = p;
-    q.x += first; q.y += first; q.z += first;
-    q.u += first; q.v += first; q.w += first;
-    q.q += first;
-    q.n = p.n - first < slice ? p.n - first : slice;
-    if ((e = zero_u32(b.cnt, (size_t)ntiles + 2, s)) != hipSuccess) break;
+  for_slices(p.n, slice, [&](int64_t first, int64_t count) {
+    const KPart<T> q = part_slice(p, first, count);
+    if ((e = zero_u32(b.cnt, (size_t)ntiles + 2, s)) != hipSuccess) return false;
     const unsigned counts = (unsigned)((q.n + kBlock * b.per - 1) / (kBlock * b.per));
     if (pack)
       hipLaunchKernelGGL((k_dep_count<T, true, PackedField<T>>), dim3(counts), dim3(kBlock), 0,
@@ -747,7 +778,8 @@ hipError_t tile_deposit(const KGrid<T> &g, const KField<T> *f, const KPart<T> &p
     hipLaunchKernelGGL(k_tile_deposit<T>, dim3((unsigned)items), dim3(4 * kDepCells), 0, s, g,
                        q, m, b);
     e = hipGetLastError();
-  }
+    return e == hipSuccess;
+  });
   const hipError_t ef = stream_free(w, s);
   return e != hipSuccess ? e : ef;
 }
@@ -778,6 +810,20 @@ hipError_t launch_mover(const KGrid<T> &g, const KField<T> &f,
   return e != hipSuccess ? e : ef;
 }
 
+// k_deposit in launches of fewer than 2^32 threads.
+template <typename T>
+hipError_t direct_deposit(const KGrid<T> &g, const KPart<T> &p, const KMom &m,
+                          unsigned int *status, hipStream_t s) {
+  hipError_t e = hipSuccess;
+  for_slices(p.n, 1 << 30, [&](int64_t first, int64_t count) {
+    const KPart<T> q = part_slice(p, first, count);
+    hipLaunchKernelGGL(k_deposit<T>, dim3((q.n - 1) / kRun + 1), dim3(64), 0, s, g, q, m, status);
+    e = hipGetLastError();
+    return e == hipSuccess;
+  });
+  return e;
+}
+
 template <typename T>
 hipError_t launch_deposit(const KGrid<T> &g, const KPart<T> &p, const KMom &m,
                           unsigned int *status, hipStream_t s) {
@@ -785,8 +831,7 @@ hipError_t launch_deposit(const KGrid<T> &g, const KPart<T> &p, const KMom &m,
   bool taken;
   const hipError_t e = tile_deposit<T>(g, nullptr, p, nullptr, m, status, s, taken);
   if (taken) return e;
-  hipLaunchKernelGGL(k_deposit<T>, dim3((p.n - 1) / kRun + 1), dim3(64), 0, s, g, p, m, status);
-  return hipGetLastError();
+  return direct_deposit<T>(g, p, m, status, s);
 }
 
 template <typename T>
@@ -800,8 +845,7 @@ hipError_t launch_mover_deposit(const KGrid<T> &g, const KField<T> &f,
   if (taken) return e;
   const hipError_t em = launch_mover<T>(g, f, p, k, status, s);
   if (em != hipSuccess) return em;
-  hipLaunchKernelGGL(k_deposit<T>, dim3((p.n - 1) / kRun + 1), dim3(64), 0, s, g, p, m, status);
-  return hipGetLastError();
+  return direct_deposit<T>(g, p, m, status, s);
 }
 
 #define SPIC_INSTANTIATE(T)                                                   \

@@ -25,7 +25,8 @@ __global__ void k_bin_keys(const T *__restrict__ x, const T *__restrict__ y,
                            unsigned int *__restrict__ key,
                            unsigned int *__restrict__ idx) {
   const long lost = nbx * nby * nbz;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n;
+  // unsigned: the last index plus the grid does not fit an int near 2^31
+  for (unsigned int i = blockIdx.x * blockDim.x + threadIdx.x; i < (unsigned)n;
        i += gridDim.x * blockDim.x) {
     // floor of the FPpart quotient, then to long (Particles.cpp:180-182);
     // the quotient is clamped so the conversion is defined for any input.
@@ -41,7 +42,7 @@ __global__ void k_bin_keys(const T *__restrict__ x, const T *__restrict__ y,
     else
       b = pz + py * nbz + px * nbz * nby;
     key[i] = (unsigned int)b;
-    idx[i] = (unsigned int)i;
+    idx[i] = i;
   }
 }
 
@@ -56,7 +57,7 @@ struct Several {
 template <typename T, int N>
 __global__ __launch_bounds__(256) void k_gather(Several<T> src, Several<T> dst,
                                                 const unsigned int *__restrict__ perm, int n) {
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+  for (unsigned int i = blockIdx.x * 256 + threadIdx.x; i < (unsigned)n; i += gridDim.x * 256) {
     const unsigned int j = perm[i];
     T v[N];
 #pragma unroll
@@ -68,7 +69,7 @@ __global__ __launch_bounds__(256) void k_gather(Several<T> src, Several<T> dst,
 
 template <typename T, int N>
 __global__ __launch_bounds__(256) void k_copy(Several<T> src, Several<T> dst, int n) {
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+  for (unsigned int i = blockIdx.x * 256 + threadIdx.x; i < (unsigned)n; i += gridDim.x * 256) {
     T v[N];
 #pragma unroll
     for (int a = 0; a < N; ++a) v[a] = src.p[a][i];
