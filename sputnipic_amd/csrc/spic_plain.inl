@@ -400,6 +400,10 @@ constexpr int kDepCells = kDepTile * kDepTile * kDepTile;
 constexpr int kDepBatch = 512;         // particles staged in LDS at a time
 constexpr int kDepMaxRun = 4096;       // particles per workgroup at most
 constexpr int kDepSlice = 1 << 24;     // particles binned at a time (24-bit indices)
+// Tiles at most: each may be a work item of its own, of 4 * kDepCells threads, and a
+// launch has fewer than 2^32.
+constexpr long kDepMaxTiles = 1 << 23;
+static_assert((kDepMaxTiles + kDepSlice / kDepBatch) * 4 * kDepCells < (1ll << 32), "one launch");
 constexpr uint32_t kDepIndexMask = (1u << 24) - 1u;
 static_assert(slices_sum(2147483647, kDepSlice) == 2147483647 &&
                   slices_sum(kDepSlice, kDepSlice) == kDepSlice &&
@@ -686,8 +690,8 @@ void k_tile_deposit(KGrid<T> g, KPart<T> p, KMom m,
 // workgroups' batches, and a stream that may allocate (a capture keeps the
 // direct kernels).
 inline bool dep_through_tiles(long ntiles, int n, hipStream_t s) {
-  return n >= kDepMinParticles && (long)n >= ntiles * kDepMinPerTile && ntiles <= (1 << 26) &&
-         stream_may_alloc(s);
+  return n >= kDepMinParticles && (long)n >= ntiles * kDepMinPerTile &&
+         ntiles <= kDepMaxTiles && stream_may_alloc(s);
 }
 
 // Whether the push packs the fields first.  Packing costs a launch and the
