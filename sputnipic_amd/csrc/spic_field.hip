@@ -272,7 +272,7 @@ __global__ void k_rhoc(Dims d, GhostMap g, double *rhon, double *__restrict__ rh
 // .25 * (a - b) * inv, one term of the reference's divergence stencils, with
 // inv4 = .25 * inv: a factor of a power of two commutes with the rounding, so
 // the value is the same as long as nothing underflows.  Multiplying by .25
-// here becomes a v_ldexp_f64 per term (75 in k_hat).
+// here becomes a v_ldexp_f64 per term (36 per cell and species in k_divsymm).
 __device__ __forceinline__ double q4(double a, double b, double inv4) {
   return (a - b) * inv4;
 }
@@ -323,7 +323,11 @@ constexpr int kFieldThreads = ((FX + 1) * (kFY + 1) * (kFZ + 1) + 63) / 64 * 64;
 struct Tiles {
   int ny, nz;  // tiles per axis
   unsigned total;
+  unsigned first = 0, end = 0;  // of one launch
 };
+// Tiles per launch: a thin grid has tiles that are mostly empty, and a launch fewer
+// than 2^32 threads.
+constexpr unsigned kMaxTiles = 1u << 16;
 
 inline Tiles tiles_of(int fx, int n0, int n1, int n2) {
   Tiles t;
@@ -477,8 +481,8 @@ __global__ __launch_bounds__(kFieldThreads<FX>) void k_image_d(Dims d, ImageArgs
   constexpr int NX = FX + 1, NY = kFY + 1, NZ = kFZ + 1;
   __shared__ double s_d[3][NX * NY * NZ];
   const int tid = threadIdx.x;
-  const unsigned tile = xcd_block();
-  if (tile >= tiles.total) return;
+  const unsigned tile = tiles.first + xcd_block();
+  if (tile >= tiles.end) return;
   const int bz = tile % tiles.nz, by = (tile / tiles.nz) % tiles.ny,
             bx = tile / (tiles.nz * tiles.ny);
   const int i0 = 1 + bx * FX, j0 = 1 + by * kFY, k0 = 1 + bz * kFZ;
@@ -813,13 +817,17 @@ int spic_maxwell_image(const spic_grid *grd, const spic_field *field,
                        hipMemcpyDeviceToDevice, s);
     if (e != hipSuccess) return spic::hip_fail(e, "MaxwellImage");
   }
-  const dim3 grid(spic::xcd_grid(tiles.total));
-  if (wide)
-    hipLaunchKernelGGL(spic::k_image_d<8>, grid, dim3(spic::kFieldThreads<8>), 0, s, d, a, tiles,
-                       divc, .25 * grd->invdx, .25 * grd->invdy, .25 * grd->invdz);
-  else
-    hipLaunchKernelGGL(spic::k_image_d<4>, grid, dim3(spic::kFieldThreads<4>), 0, s, d, a, tiles,
-                       divc, .25 * grd->invdx, .25 * grd->invdy, .25 * grd->invdz);
+  for (tiles.first = 0; tiles.first < tiles.total; tiles.first = tiles.end) {
+    tiles.end = tiles.total - tiles.first > spic::kMaxTiles ? tiles.first + spic::kMaxTiles
+                                                            : tiles.total;
+    const dim3 grid(spic::xcd_grid(tiles.end - tiles.first));
+    if (wide)
+      hipLaunchKernelGGL(spic::k_image_d<8>, grid, dim3(spic::kFieldThreads<8>), 0, s, d, a, tiles,
+                         divc, .25 * grd->invdx, .25 * grd->invdy, .25 * grd->invdz);
+    else
+      hipLaunchKernelGGL(spic::k_image_d<4>, grid, dim3(spic::kFieldThreads<4>), 0, s, d, a, tiles,
+                         divc, .25 * grd->invdx, .25 * grd->invdy, .25 * grd->invdz);
+  }
   e = hipGetLastError();
   if (e == hipSuccess) {
     hipLaunchKernelGGL(spic::k_image, dim3(spic::xcd_grid(spic::grid1(d.in_nodes))), dim3(256), 0, s, d, a, gn,
