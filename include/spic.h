@@ -118,6 +118,13 @@ typedef struct spic_push {
 /* (the default, spic_set_async(0)) each call waits for its stream and     */
 /* reports out-of-domain particles as SPIC_EDOMAIN; in asynchronous mode   */
 /* calls only enqueue work and spic_check_domain() reports later.          */
+/* For larger species spic_mover_pc (from 262144 particles),               */
+/* spic_interp_p2g and spic_mover_interp (from 16384) take scratch memory  */
+/* in the order of their stream, in either mode: at most 8 bytes per       */
+/* particle (128 MiB), 32 per tile of 4x4x4 cells and 48 (FP32: 32) per    */
+/* node, from a pool of the device that keeps up to 512 MiB between calls  */
+/* (spic_release_scratch).  Under stream capture, and where the device has */
+/* none left, they run kernels that need none.                             */
 /* ---------------------------------------------------------------------- */
 
 /* mover_PC: NiterMover predictor-corrector iterations per particle, final
@@ -519,6 +526,9 @@ int spic_set_subcycling(int mode);
 /* In asynchronous mode: wait for `stream`, return SPIC_EDOMAIN if any
  * out-of-domain particle was seen since the last check, and clear it. */
 int spic_check_domain(void *stream);
+/* Give back what the scratch pool of the current device keeps and no call in
+ * flight uses (see the reference-path entry points). */
+int spic_release_scratch(void);
 
 /* Testing hook (no counterpart in the reference): the engine device
  * allocation `after` allocations from now (0: the next one) fails as an
@@ -549,7 +559,7 @@ int spic_stream_synchronize(void *stream);
  * spic_set_async(1)) once and replay it with one launch.  Every entry point
  * above that takes a stream can be captured once its buffers exist (an
  * engine after spic_engine_load, the moment arrays after allocation); none
- * allocates or synchronizes in async mode.  A replay repeats the captured
+ * allocates or synchronizes while it is captured.  A replay repeats the captured
  * work on the same device buffers: an engine phase captures which of its
  * two particle buffers it reads, so capture an even number of phases and
  * sorts to replay a run more than once.  Replays do not advance the host

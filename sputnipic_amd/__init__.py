@@ -16,7 +16,7 @@ from .core import (Batch, DeviceArray, DeviceParticles, EMField, Engine, Event, 
                    GemSpecies, Grid, InterpDensNet, InterpDensSpecies, Parameters,
                    Particles, Stream, FIELD_NAMES, MOMENT_NAMES, PARTICLE_NAMES, applyBCids,
                    applyBCids_all, beam_species, check_domain, device_count, gem_fields, gem_particles, get_async, harris_species,
-                   interpP2G, mover_interp, mover_PC, particle_sort, set_async,
+                   interpP2G, mover_interp, mover_PC, particle_sort, release_scratch, set_async,
                    set_strict_fp, set_subcycling, setZeroSpeciesDensities, sumOverSpecies)
 
 __all__ = [

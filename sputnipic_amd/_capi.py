@@ -197,6 +197,7 @@ SIGNATURES = {
     "spic_set_strict_fp": (C.c_int, [C.c_int]),
     "spic_set_subcycling": (C.c_int, [C.c_int]),
     "spic_check_domain": (C.c_int, [_P]),
+    "spic_release_scratch": (C.c_int, []),
     "spic_test_fail_engine_alloc": (C.c_int, [C.c_int]),
     "spic_device_count": (C.c_int, [C.POINTER(C.c_int)]),
     "spic_malloc": (C.c_int, [C.POINTER(_P), C.c_size_t]),

@@ -380,6 +380,12 @@ def check_domain(stream: Optional["Stream"] = None) -> None:
     check(lib().spic_check_domain(stream.ptr if stream else None), "spic_check_domain")
 
 
+def release_scratch() -> None:
+    """Give back the scratch memory that calls on large species have left in the
+    device's pool (up to 512 MiB)."""
+    check(lib().spic_release_scratch(), "spic_release_scratch")
+
+
 def mover_PC(part: Particles, field: EMField, grd: Grid, param: Parameters) -> int:
     """mover_PC (src/Mover.cpp:4-162); returns 0 like the reference."""
     _check_prec(part, grd)

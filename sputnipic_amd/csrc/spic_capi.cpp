@@ -252,6 +252,16 @@ hipError_t stream_alloc(void **p, size_t bytes, hipStream_t s) {
 
 hipError_t stream_free(void *p, hipStream_t s) { return hipFreeAsync(p, s); }
 
+hipError_t release_scratch() {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(g_pool_mutex);
+  for (const auto &sp : g_pools)
+    if (sp.device == dev) return hipMemPoolTrimTo(sp.pool, 0);
+  return hipSuccess;
+}
+
 bool stream_may_alloc(hipStream_t s) {
   if (s == nullptr) return true;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -433,6 +443,11 @@ int spic_check_domain(void *stream) {
   spic::StatusBuf *sb = spic::status_words(&e);
   if (!sb) return hip_fail(e, "status buffer");
   return spic::read_status((hipStream_t)stream, sb, true);
+}
+
+int spic_release_scratch(void) {
+  const hipError_t e = spic::release_scratch();
+  return e == hipSuccess ? SPIC_OK : hip_fail(e, "scratch release");
 }
 
 int spic_mover_pc(const spic_grid *grd, const spic_field *field,
