@@ -146,6 +146,7 @@ struct BinnedArgs {
   int ns;
   int lds_fp64;            // FP32 particles: LDS moment block in FP64
   int n_ovf_blocks;        // workgroups for the overflow regions
+  int split;               // 1: a workgroup per tile and species (single engines)
   int push_off;            // 1: deposit only (interpP2G); no push, no field read
   int fixed;               // 1: positions in fixed point (FP32 engines), see above
   int ppt;                 // particles per thread and batch of the phase kernel: 1, or

@@ -1550,21 +1550,13 @@ template hipError_t launch_binned_phase_queue<float>(const BinnedArgs<float> *,
                                                      unsigned int *, int, int, int, int, int,
                                                      hipStream_t);
 
-// Below one workgroup per CU the species of a tile run side by side, one
-// workgroup each; from there on one workgroup takes them in turn and stages its
-// tile once.  Measured, in turn / side by side, four species: 225 tiles of 27
-// particles per cell 231 / 194 us in FP64 and 206 / 191 in FP32, of 125 per
-// cell 740 / 460 and 657 / 350; 432 tiles of 27 per cell 303 / 354 and
-// 268 / 334; 3456 tiles of 27 per cell 1608 / 1969 in FP64.
-constexpr int kSplitTiles = 256;
-
 template <typename T, typename A, bool PUSH, bool FX>
 hipError_t launch_binned_shape(const BinnedArgs<T> &a, hipStream_t s) {
   // two particles per thread and batch: the FP32 fixed-point phase only
   constexpr bool kPpt2 = sizeof(T) == 4 && FX && PUSH;
   const bool ppt2 = PUSH && a.ppt == 2;  // the deposit alone keeps one
   if (ppt2 && !kPpt2) return hipErrorInvalidValue;
-  const dim3 grid(a.ntiles, a.ntiles < kSplitTiles ? a.ns : 1);
+  const dim3 grid(a.ntiles, a.split ? a.ns : 1);
   if (a.tx == 4 && a.ty == 4 && a.tz == 4) {
     if constexpr (kPpt2) {
       if (ppt2)

@@ -31,6 +31,7 @@ struct spic_engine {
   int keep_ids = 1;                // a load index per particle (store in load order)
   int ovf_pct = 100;               // overflow slots per buffer, percent of n
   int ppt = 1;                     // particles per thread and batch of the phase
+  int cus = 256;                   // compute units of the device
   int64_t phases = 0, sorts = 0;
   uint64_t gen = 0;                // bumped by every load (storage may move)
   size_t bytes = 0;
@@ -211,6 +212,26 @@ hipError_t sort_any(spic_engine *e, int is, void *const *src, hipStream_t s,
                                  : sort_species<float>(e, is, src, src_f64, s);
 }
 
+// Whether the species of a tile run side by side, one workgroup each, or in turn
+// in one that stages its tile once.  Side by side pays where there are few tiles
+// for the compute units, and the longer the more particles a (full) tile and
+// species has: up to a tile for four units and one more per 2400 / cus particles,
+// at most two per unit.  Time in turn over side by side, 256 units, 2 to 8 species
+// of 128 / 512 / 1728 / 4096 particles per tile, FP64: 64 tiles 1.08 to 1.15, 1.14 to
+// 1.34, 1.5 to 2.3, 1.6 to 3.4; 128 tiles 1.01 to 1.04, 0.99 to 1.02, 1.3 to 1.6, 1.6
+// to 2.2; 225 tiles 0.89 to 0.96, 0.79 to 0.93, 1.06 to 1.14, 1.2 to 1.5; 288 tiles
+// 0.83 to 0.88, 0.75 to 0.82, 0.91 to 1.14, 1.1 to 1.5; 384 tiles 0.73 to 0.9, 0.65 to
+// 0.8, 0.88 to 0.96, 0.98 to 1.28; 512 tiles 0.66 to 0.87, 0.59 to 0.77, 0.79 to 0.86,
+// 0.95 to 1.0; beyond (640 tiles 0.63 to 1.36) neither side wins throughout.  FP32
+// within 0.1 of that.
+bool species_side_by_side(const spic_engine *e, int64_t particles, int species) {
+  const auto &L = e->L;
+  const double cells = (double)L.ncx * L.ncy * L.ncz * species;
+  const double per = (double)particles * (L.tx * L.ty * L.tz) / cells;
+  const double line = e->cus * (0.25 + per / 2400.0), most = 2.0 * e->cus;
+  return L.ntiles <= (line < most ? line : most);
+}
+
 // The phase kernel's argument block for the loaded species of `e`, read
 // from buffer `cur` (the species' own when negative).
 // idx[k] is the engine species of argument species k; returns the count.
@@ -263,6 +284,9 @@ int fill_args(const spic_engine *e, const spic_field *field, const spic_moments 
     ++k;
   }
   a.ns = k;
+  int64_t particles = 0;
+  for (int j = 0; j < k; ++j) particles += a.sp[j].n;
+  a.split = k > 1 && species_side_by_side(e, particles, k) ? 1 : 0;
   return k;
 }
 
@@ -437,6 +461,13 @@ int spic_engine_create(spic_engine **out, const spic_grid *grd, int ns,
   e->keep_ids = keep_ids;
   e->ovf_pct = ovf_pct;
   e->ppt = ppt;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) == hipSuccess &&
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+      cus > 0)
+    e->cus = cus;
+  else
+    (void)hipGetLastError();
   auto &L = e->L;
   L.ncx = grd->nxc - 2; L.ncy = grd->nyc - 2; L.ncz = grd->nzc - 2;
   L.tx = tx; L.ty = ty; L.tz = tz;
