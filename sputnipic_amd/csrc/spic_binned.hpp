@@ -179,6 +179,11 @@ struct BinnedReduceArgs {
   KMom mom[kMaxSpecies];
 };
 
+// Workgroups that write the segments of ntiles tiles: 1024 tiles each, at most 256.
+__host__ __device__ constexpr int layout_blocks(int ntiles) {
+  return ntiles <= 1024 ? 1 : ntiles >= 256 * 1024 ? 256 : (ntiles + 1023) / 1024;
+}
+
 // The segments of the buffer a phase writes, from those and the counters of
 // the buffer it reads.
 struct LayoutArgs {
@@ -274,8 +279,8 @@ hipError_t phase_start(const CountArrays &c, hipStream_t s);
 // The reduce and the count reset of a batch, from the device-resident
 // argument blocks tab[i] of its instances: per instance, the node blocks
 // nodes.start[i].. of 256 nodes each (reduce) and the blocks
-// counts.start[i].. of 256 threads each: the first writes the segments of
-// every species' output buffer, thread j of the others resets counter j of its
+// counts.start[i].. of 256 threads each: the first layout_blocks write the segments
+// of every species' output buffer, thread j of the others resets counter j of its
 // cnt_out (kCntArrays * (ntiles + 1) entries) and, with `moments`, node j of
 // its ten moment arrays; max_ns species per launch row.
 template <typename T>

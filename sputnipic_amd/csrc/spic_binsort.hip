@@ -685,21 +685,26 @@ void k_store_tile(Arrays7<T> src, const uint32_t *__restrict__ id,
   }
 }
 
-// One workgroup of 256 threads writes the output buffer's segments of a
-// species: the input buffer's, or, when its overflow region holds more than
-// kRelayoutOverflow particles, segments of each tile's particles plus its
-// share of the slack, half of it even and half in proportion to the particles
-// (arrivals grow with them).  Both halves are rounded down, so the segments
-// take at most n + ntiles * slack slots and the overflow region after them
-// stays inside the buffer.
-__device__ __forceinline__ void phase_layout(const LayoutArgs &l, int ntiles) {
+// Workgroup b of nb (layout_blocks), 256 threads each, writes its part of the
+// output buffer's segments of a species: the input buffer's, or, when its
+// overflow region holds more than kRelayoutOverflow particles, segments of each
+// tile's particles plus its share of the slack, half of it even and half in
+// proportion to the particles (arrivals grow with them).  Both halves are rounded
+// down, so the segments take at most n + ntiles * slack slots and the overflow
+// region after them stays inside the buffer.  A workgroup adds up the tiles before
+// its own by itself: half a million tiles by one workgroup took 1.7 of 25.7 ms of a
+// phase of 33.5M particles.
+__device__ __forceinline__ void phase_layout(const LayoutArgs &l, int ntiles, int b, int nb) {
   __shared__ unsigned long long s_sum[4];
   const SPIC_GLOBAL int64_t *in = gmem(l.seg_in);
   SPIC_GLOBAL int64_t *out = gmem(l.seg_out);
   const SPIC_GLOBAL unsigned int *cnt = gmem(l.cnt_in);
   const int tid = threadIdx.x, lane = tid & 63;
+  const int chunk = (ntiles + nb - 1) / nb;
+  const int t0 = min(b * chunk, ntiles), t1 = min(t0 + chunk, ntiles);
   if (cnt[ntiles] <= kRelayoutOverflow) {
-    for (int t = tid; t <= ntiles; t += 256) out[t] = in[t];
+    for (int t = t0 + tid; t < t1; t += 256) out[t] = in[t];
+    if (b == nb - 1 && tid == 0) out[ntiles] = in[ntiles];
     return;
   }
   const int64_t even = l.slack / 2;
@@ -709,41 +714,50 @@ __device__ __forceinline__ void phase_layout(const LayoutArgs &l, int ntiles) {
     return (unsigned long long)held + (unsigned long long)even +
            (unsigned long long)((double)held * share);
   };
-  // thread t sums a run of tiles, the workgroup scans the sums
-  const int per = (ntiles + 255) / 256;
-  const int t0 = min(tid * per, ntiles), t1 = min(t0 + per, ntiles);
-  unsigned long long sum = 0;
-  for (int t = t0; t < t1; ++t) sum += slots(t);
-  unsigned long long at = sum;
+  // inclusive sum over the workgroup's threads; total: of all of them
+  auto scan = [&](unsigned long long v, unsigned long long &total) -> unsigned long long {
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const unsigned long long v = __shfl_up(at, d);
-    if (lane >= d) at += v;
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned long long u = __shfl_up(v, d);
+      if (lane >= d) v += u;
+    }
+    __syncthreads();  // the last scan's sums have been read
+    if (lane == 63) s_sum[tid >> 6] = v;
+    __syncthreads();
+    total = 0;
+    for (int w = 0; w < 4; ++w) {
+      if (w == (tid >> 6)) v += total;
+      total += s_sum[w];
+    }
+    return v;
+  };
+  unsigned long long before = 0, first, total;
+#pragma unroll 4
+  for (int t = tid; t < t0; t += 256) before += slots(t);
+  (void)scan(before, first);
+  for (int base = t0; base < t1; base += 256) {
+    const int t = base + tid;
+    const unsigned long long v = t < t1 ? slots(t) : 0;
+    const unsigned long long at = first + scan(v, total) - v;
+    if (t < t1) out[t] = (int64_t)at;
+    first += total;
   }
-  if (lane == 63) s_sum[tid >> 6] = at;
-  __syncthreads();
-  at -= sum;
-  for (int w = 0; w < (tid >> 6); ++w) at += s_sum[w];
-  for (int t = t0; t < t1; ++t) {
-    out[t] = (int64_t)at;
-    at += slots(t);
-  }
-  if (tid == 255) out[ntiles] = (int64_t)at;
+  if (b == nb - 1 && tid == 0) out[ntiles] = (int64_t)first;
 }
 
-// Per species (blockIdx.y): the first workgroup writes the output segments;
-// thread i of the others zeroes counter i (i < n) and, with c.nn > 0, node i
-// of the ten moment arrays (i < nn).
+// Per species (blockIdx.y): the first layout_blocks workgroups write the output
+// segments; thread i of the others zeroes counter i (i < n) and, with c.nn > 0,
+// node i of the ten moment arrays (i < nn).
 __global__ __launch_bounds__(256) void k_phase_start(CountArrays c) {
-  const int s = blockIdx.y;
+  const int s = blockIdx.y, nb = layout_blocks(c.ntiles);
   if (s >= c.ns) return;
-  if (blockIdx.x == 0) {
-    if (c.lay[s].seg_out) phase_layout(c.lay[s], c.ntiles);
+  if ((int)blockIdx.x < nb) {
+    if (c.lay[s].seg_out) phase_layout(c.lay[s], c.ntiles, blockIdx.x, nb);
     return;
   }
   const int64_t total = c.n > c.nn ? c.n : c.nn;
-  for (int64_t i = (blockIdx.x - 1) * (int64_t)blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)(gridDim.x - 1) * blockDim.x) {
+  for (int64_t i = (blockIdx.x - nb) * (int64_t)blockDim.x + threadIdx.x; i < total;
+       i += (int64_t)(gridDim.x - nb) * blockDim.x) {
     if (i < c.n) gmem(c.p[s])[i] = 0u;
     if (i < c.nn) {
 #pragma unroll
@@ -831,12 +845,14 @@ __global__ __launch_bounds__(256) void k_phase_start_batch(
   const int s = blockIdx.y;
   if (s >= a.ns) return;
   const int block = blockIdx.x - map.start[i];
-  if (block == 0) {
+  const int nb = layout_blocks(a.ntiles);
+  if (block < nb) {
     const BinnedSpecies<T> &sp = a.sp[s];
-    phase_layout(LayoutArgs{sp.seg_in, sp.seg_out, sp.cnt_in, sp.slack, sp.n}, a.ntiles);
+    phase_layout(LayoutArgs{sp.seg_in, sp.seg_out, sp.cnt_in, sp.slack, sp.n}, a.ntiles, block,
+                 nb);
     return;
   }
-  const int64_t j = (int64_t)(block - 1) * 256 + threadIdx.x;
+  const int64_t j = (int64_t)(block - nb) * 256 + threadIdx.x;
   if (j < kCntArrays * (int64_t)(a.ntiles + 1)) gmem(a.sp[s].cnt_out)[j] = 0u;
   if (moments && j < (int64_t)a.g.nxn * a.g.nyn * a.g.nzn) {
 #pragma unroll
@@ -1390,7 +1406,7 @@ template hipError_t tile_sort_batch<float>(const TileSortJob<float> *, const Til
 
 hipError_t phase_start(const CountArrays &c, hipStream_t s) {
   if (c.ns <= 0 || c.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_phase_start, dim3(1 + nblocks(c.n > c.nn ? c.n : c.nn), c.ns), dim3(256),
+  hipLaunchKernelGGL(k_phase_start, dim3(layout_blocks(c.ntiles) + nblocks(c.n > c.nn ? c.n : c.nn), c.ns), dim3(256),
                      0, s, c);
   return hipGetLastError();
 }

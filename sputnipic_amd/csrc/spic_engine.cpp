@@ -934,7 +934,7 @@ hipError_t build_tables(spic_batch *b, unsigned int *status) {
     const int64_t ncnt = spic::kCntArrays * (int64_t)(e->L.ntiles + 1);
     const int64_t zeroed =
         (b->flags & SPIC_BATCH_SET_MOMENTS) && nn > ncnt ? nn : ncnt;
-    b->counts.start[i + 1] = b->counts.start[i] + (any ? 1 + blocks(zeroed, 256) : 0);
+    b->counts.start[i + 1] = b->counts.start[i] + (any ? spic::layout_blocks(e->L.ntiles) + blocks(zeroed, 256) : 0);
     b->gen[i] = e->gen;
   }
   b->status = status;
