@@ -21,7 +21,8 @@
 //        cells are placed in LDS sorted by cell (a count per cell, a scan, a
 //        place per particle), and the four threads of each cell take the
 //        cell's run, each thread two of the cell's eight nodes, and accumulate
-//        their ten moments in registers; a particle in a halo cell adds its
+//        their ten moments in registers; a particle in a halo cell (and in FP32
+//        one of more than a dozen of its cell in the batch) adds its
 //        80 contributions to the LDS moment block; one outside the block adds
 //        them to global memory;
 //      the register sums are added to the LDS moment block after the last
@@ -839,15 +840,16 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
   // step
   constexpr int NP = NT * PPT;
   constexpr int NL = kListCap;  // list ring entries
-  // FP32 sums go on in FP64, in the LDS block, before they are long: twice per
-  // species, or four times where it has many batches, and after kRun particles
-  // of one cell in a batch.  Relative L2 errors of the ten moments against a
-  // 64-bit deposit of the same particles: all of a tile's in one cell, 0.5 to
-  // 2.0e-7 (1.6 to 3.5e-6 in one run over the species); 125 per cell evenly
-  // spread, 0.6 to 1.4e-7 (0.8 to 2.2e-7); 8 per cell, 0.6 to 1.0e-7 (0.6 to
-  // 1.1e-7).  The folds cost 1 to 3% of a phase: 8.64 ms instead of 8.46 on the
-  // 262M-particle sheet, 11.1 instead of 10.8 with eight species, 0.795 instead
-  // of 0.772 for 12 instances.
+  // FP32 sums are kept short: a cell takes kRun particles of a batch at most, the
+  // others go through the list, whose deposits are added to the LDS block in FP64,
+  // and the sums go on there twice per species (every 64 batches at least).
+  // Relative L2 errors of the ten moments against a 64-bit deposit of the same
+  // particles: all of a tile's in one cell, 0.5 to 2.1e-7 (1.6 to 3.5e-6 in one run
+  // over the species); 125 per cell evenly spread, 0.6 to 1.7e-7 (0.8 to 2.2e-7);
+  // 8 per cell, 0.6 to 1.0e-7 (0.6 to 1.1e-7).  It costs 1 to 2% of a phase: 8.61 ms
+  // instead of 8.51 on the 262M-particle sheet, 11.04 instead of 10.88 with eight
+  // species, 0.797 instead of 0.780 for 12 instances (with runs of 12 cut within the
+  // cell step instead of at the list, 8.89, 11.28 and 0.804).
   constexpr bool kShort = sizeof(T) == 4;
   constexpr unsigned int kRun = 12 * PPT;
   __shared__ T s_fld[NB * 6];
@@ -979,8 +981,7 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
 
     const uint32_t nbatches = (nin + NP - 1) / NP;
     // batches from one fold to the next; the last batch's is the last
-    const uint32_t fold_every = !kShort ? nbatches : nbatches <= 8 ? (nbatches + 1) / 2
-                                                                   : min((nbatches + 3) / 4, 32u);
+    const uint32_t fold_every = kShort ? min((nbatches + 1) / 2, 64u) : nbatches;
     uint32_t fold_at = fold_every - 1;
     // this thread's particle of batch j (x y z u v w q and its id), loaded
     // one batch ahead.  PREFETCH: batch j + 1 is loaded while batch j is
@@ -1081,13 +1082,17 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
       if (active) {
         bool done = false;
         if (in_tile) {
-          CELL[pp] =
+          const int cell =
               ((ix - 2 - blk.c0x) * TY + (iy - 2 - blk.c0y)) * TZ + (iz - 2 - blk.c0z);
-          RANK[pp] = atomicAdd(&s_cnt[buf][CELL[pp]], 1u);
-          done = true;
-          ++n_ld;
-        } else {
-          // halo cell or outside the block: to the list
+          RANK[pp] = atomicAdd(&s_cnt[buf][cell], 1u);
+          done = !kShort || RANK[pp] < kRun;
+          if (done) {
+            CELL[pp] = cell;
+            ++n_ld;
+          }
+        }
+        if (!done) {
+          // halo cell, outside the block, or a clump: to the list
           const unsigned int k = atomicAdd(&s_nl, 1u);
           if (k - lst_free < (unsigned int)NL) {
             const unsigned int e = k % NL;
@@ -1137,6 +1142,7 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
 #pragma unroll
         for (int i = 0; i < CPL; ++i) {
           c[i] = s_cnt[buf][lane * CPL + i];
+          if (kShort) c[i] = min(c[i], kRun);
           sum += c[i];
         }
         unsigned int at = wave_scan(sum);
@@ -1233,13 +1239,8 @@ __device__ __forceinline__ void binned_phase_tile(const BinnedArgs<T> &a, const 
         };
         const bool due = j == fold_at;
         if (due) fold_at = min(j + fold_every, nbatches - 1);
-        for (unsigned int e = s_off[my_cell];;) {
-          const unsigned int stop = kShort ? min(end, e + kRun) : end;
-          for (; e < stop; ++e) add(acc, e);
-          const bool more = kShort && e < end;
-          if (more || due) fold();
-          if (!more) break;
-        }
+        for (unsigned int e = s_off[my_cell]; e < end; ++e) add(acc, e);
+        if (due) fold();
       }
       // list step: once the ring is half full, all threads deposit its pending
       // entries, eight threads per entry, one node each, in whole rounds of

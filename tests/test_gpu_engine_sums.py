@@ -2,11 +2,11 @@
 of a tile that the grid's end leaves one cell wide, and of every cell alike,
 against the FP64 oracle's deposit of the very particles that the engine holds.
 
-Here a sum in FP32 runs over at most 64 terms (a quarter of 64 batches at four
-per cell; in a clump, 24) before it goes on in FP64, and the tile's sum is
-rounded to FP32 once.  With rounding errors of 0.41 * 2^-24 (rms) of the running
-value that is 0.41 sqrt(64 / 3) + 0.41 = 2.3 * 2^-24 of the sum of the terms'
-magnitudes; a term's own ten roundings average out over the many terms of a
+Here a sum in FP32 runs over at most 128 terms (half of 64 batches at four per
+cell; of a clump at most 24 per batch) before it goes on in FP64, and the tile's sum
+is rounded to FP32 once.  With rounding errors of 0.41 * 2^-24 (rms) of the running
+value that is 0.41 sqrt(128 / 3) / sqrt(2) + 0.41 = 2.3 * 2^-24 of the sum of the
+terms' magnitudes; a term's own ten roundings average out over the many terms of a
 node.  Bound: 8 * 2^-24 of the largest sum of magnitudes.  One FP32 chain over
 all 32768 particles of a cell is off by 0.41 sqrt(32768 / 3) = 43 * 2^-24.
 """
