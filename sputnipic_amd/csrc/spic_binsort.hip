@@ -11,8 +11,8 @@
 // 4 * cells-per-tile consecutive particles holds about four per cell: the
 // phase kernel sums one such run per batch cell by cell, and
 // particles that stay in their tile keep this order from phase to phase.
-// A load of an FP64 engine gets there by tiles (counts, places and one workgroup
-// per tile); other loads, and a binned source, by a stable LSD radix sort
+// Most loads get there by tiles (counts, places and one workgroup per tile;
+// load_through_tiles); the others, and a binned source, by a stable LSD radix sort
 // (rocPRIM) of (key, source slot) pairs, whose result is the
 // permutation; the seven arrays and the particle id are gathered to sorted
 // position i + tile * slack, so that every segment gets `slack` free slots
@@ -231,7 +231,6 @@ constexpr int kLoadThreads = 1024;
 constexpr int kLoadManyTiles = 16384;
 constexpr int kLoadPer = 8;      // particles per thread that a tile's workgroup holds
 constexpr int kLoadHeld = kLoadThreads * kLoadPer;
-constexpr int kLoadStage = 4096;  // values staged in LDS at a time
 constexpr int kLoadRanks = 128;   // ranks in the slot tables
 constexpr int kLoadSorted = 512;  // particles of a cell that are put in caller order
 constexpr int kStoreThreads = 512;
@@ -261,11 +260,11 @@ struct LoadBins {
 // Counts the particles into tiles, NT threads per workgroup, which counts up to
 // LT tiles in LDS and adds each tile it met once; LT = 0: one atomic per wave and
 // tile in global memory.
-template <int NT, int LT>
-__global__ __launch_bounds__(NT) void k_load_count(KGrid<double> g, BinLayout L, LoadBins b,
-                                                   const double *__restrict__ x,
-                                                   const double *__restrict__ y,
-                                                   const double *__restrict__ z) {
+template <typename TS, typename T, int NT, int LT>
+__global__ __launch_bounds__(NT) void k_load_count(KGrid<T> g, BinLayout L, LoadBins b,
+                                                   const TS *__restrict__ x,
+                                                   const TS *__restrict__ y,
+                                                   const TS *__restrict__ z) {
   __shared__ unsigned int s_cnt[LT > 0 ? LT : 1];
   const int tid = threadIdx.x;
   if constexpr (LT > 0) {
@@ -326,6 +325,16 @@ __global__ __launch_bounds__(NT) void k_load_place(BinLayout L, LoadBins b) {
   }
 }
 
+// A caller's value into binned storage: with fixed-point storage positions
+// are converted, everything else is rounded to T.
+template <typename TS, typename T>
+__device__ __forceinline__ T load_value(TS v, int a, int fixed, const FixedParams &fx) {
+  if constexpr (sizeof(T) == 4) {
+    if (a < 3 && fixed) return __int_as_float(to_fixed_pos((double)v, fx, a));
+  }
+  return (T)v;
+}
+
 // One workgroup per tile, tiles in runs per XCD: counts its cells, ranks each
 // particle within its cell, turns the rank into its slot in round-robin order
 // (slot of the k-th particle of cell c: particles of rank < k over all cells,
@@ -365,19 +374,18 @@ __global__ __launch_bounds__(kLoadThreads) void k_load_pieces(BinLayout L, LoadB
   if (tid < NC && s_count[tid]) atomicAdd(b.cells + (size_t)piece.y * 2 * NC + tid, s_count[tid]);
 }
 
-template <int NC>
+template <typename TS, typename T, int NC>
 __global__ __launch_bounds__(kLoadThreads) __attribute__((amdgpu_waves_per_eu(8)))
-void k_load_tile(BinLayout L, LoadBins b, Arrays7<double> src, Arrays7<double> dst,
-                 uint32_t *dst_id) {
+void k_load_tile(BinLayout L, LoadBins b, Arrays7<TS> src, Arrays7<T> dst, uint32_t *dst_id) {
   // particles per cell; a whole tile's first place of each cell's indices, or
   // the first rank of a piece's in each cell
   __shared__ unsigned int s_count[NC], s_first[NC], s_A[kLoadRanks];
   __shared__ unsigned char s_T[NC][kLoadRanks];
   // the indices and their cells, cell by cell; then values by slot
   __shared__ unsigned char s_cell[kLoadHeld];
-  __shared__ double s_stage[kLoadStage];
+  constexpr int kStage = kLoadHeld * 4 / (int)sizeof(T);  // values: 32 KB
+  __shared__ T s_stage[kStage];
   uint32_t *const s_key = reinterpret_cast<uint32_t *>(s_stage);
-  static_assert(2 * kLoadStage >= kLoadHeld, "room for the indices");
   const int tid = threadIdx.x;
   const bool whole = (int)blockIdx.x < b.tile_blocks;
   int t;
@@ -452,7 +460,7 @@ void k_load_tile(BinLayout L, LoadBins b, Arrays7<double> src, Arrays7<double> d
         const unsigned int c = pos[e] & 0xffu;
         const int64_t o = out0 + slot(c, s_first[c] + (pos[e] >> 8));
 #pragma unroll
-        for (int a = 0; a < 7; ++a) dst.p[a][o] = src.p[a][j[e]];
+        for (int a = 0; a < 7; ++a) dst.p[a][o] = load_value<TS, T>(src.p[a][j[e]], a, L.fixed, L.fx);
         if (dst_id) dst_id[o] = j[e];
       }
     return;
@@ -491,31 +499,32 @@ void k_load_tile(BinLayout L, LoadBins b, Arrays7<double> src, Arrays7<double> d
   __syncthreads();
 #pragma unroll
   for (int a = 0; a < 7; ++a) {
-    double val[kLoadPer];
+    T val[kLoadPer];
 #pragma unroll
     for (int e = 0; e < kLoadPer; ++e)
-      if (e * kLoadThreads + tid < n) val[e] = src.p[a][j[e]];
-    double *__restrict__ to = dst.p[a] + out0;
-    for (int c0 = 0; c0 < n; c0 += kLoadStage) {
+      if (e * kLoadThreads + tid < n)
+        val[e] = load_value<TS, T>(src.p[a][j[e]], a, L.fixed, L.fx);
+    T *__restrict__ to = dst.p[a] + out0;
+    for (int c0 = 0; c0 < n; c0 += kStage) {
 #pragma unroll
       for (int e = 0; e < kLoadPer; ++e)
-        if (e * kLoadThreads + tid < n && pos[e] - c0 < (unsigned)kLoadStage)
+        if (e * kLoadThreads + tid < n && pos[e] - c0 < (unsigned)kStage)
           s_stage[pos[e] - c0] = val[e];
       __syncthreads();
-      const int m = min(n - c0, kLoadStage);
+      const int m = min(n - c0, kStage);
       for (int p = tid; p < m; p += kLoadThreads) to[c0 + p] = s_stage[p];
       __syncthreads();
     }
   }
   if (!dst_id) return;
   uint32_t *s_id = reinterpret_cast<uint32_t *>(s_stage);
-  for (int c0 = 0; c0 < n; c0 += kLoadStage) {
+  for (int c0 = 0; c0 < n; c0 += kStage) {
 #pragma unroll
     for (int e = 0; e < kLoadPer; ++e)
-      if (e * kLoadThreads + tid < n && pos[e] - c0 < (unsigned)kLoadStage)
+      if (e * kLoadThreads + tid < n && pos[e] - c0 < (unsigned)kStage)
         s_id[pos[e] - c0] = j[e];
     __syncthreads();
-    const int m = min(n - c0, kLoadStage);
+    const int m = min(n - c0, kStage);
     for (int p = tid; p < m; p += kLoadThreads) dst_id[out0 + c0 + p] = s_id[p];
     __syncthreads();
   }
@@ -1415,19 +1424,21 @@ hipError_t phase_start(const CountArrays &c, hipStream_t s) {
 // average, and workgroups can count them in LDS (beyond kLdsTiles those of 1024
 // threads, for enough particles).  28.8M FP32 particles on 16640 tiles, counted
 // with global atomics: 5.75 ms, 5.0 by the radix sort; 2.1M 505 / 390 us.
-// FP32 engines keep the radix sort, though tiles take half its time (4.0M
-// particles 519 / 969 us): their deposits sum in the load's order, with few
-// particles per cell the same to the last bit each time, and another order gives
-// other roundings.
 // Many tiles of a few particles each, whose workgroups are mostly tables, keep
 // the radix sort too (FP64, tiles / radix, us): 2048 tiles of 1 / 8 / 32
 // particles 61 / 71, 69 / 83, 73 / 99; 3072 75 / 70, 89 / 92, 98 / 113; 4096
 // 89 / 71, 109 / 95, 121 / 120; 5120 105 / 83, 129 / 101, 145 / 128.  From 64 on
 // tiles win (4096: 144 / 167, 5120: 171 / 192).
-inline bool load_through_tiles(int64_t n, int ntiles) {
-  if (ntiles > 2048 && n < 64 * (int64_t)ntiles) return false;
-  return n <= (int64_t)kLoadHeld * ntiles &&
-         (ntiles <= kLdsTiles || (ntiles <= kLoadManyTiles && n >= 256 * 1024 * 16));
+// FP32 engines take tiles from four particles per cell on (4.0M particles on 512
+// tiles 519 / 969 us).  With fewer, a tile's deposit is one batch of a few
+// waves, whose sums follow the load's order and repeat to the last bit; the radix
+// sort's order there gives the roundings it always gave.
+inline bool load_through_tiles(const BinLayout &L, int64_t n, bool fp32) {
+  const int64_t nt = L.ntiles;
+  if (fp32 && n < 4 * nt * (L.tx * L.ty * L.tz)) return false;
+  if (nt > 2048 && n < 64 * nt) return false;
+  return n <= kLoadHeld * nt &&
+         (nt <= kLdsTiles || (nt <= kLoadManyTiles && n >= 256 * 1024 * 16));
 }
 
 // The workspace of such a load: two words per tile, the counters of the tiles
@@ -1451,13 +1462,13 @@ inline LoadSpace load_space(const BinLayout &L, int64_t n) {
 }
 
 // The load of a dense source through tiles.
-inline hipError_t load_tiles(const KGrid<double> &g, const BinLayout &L, int64_t n,
-                             const void *const src[7], double *const dst[7],
-                             uint32_t *dst_id, int64_t *dst_seg, unsigned int *dst_cnt, char *w,
-                             const LoadSpace &sp, hipStream_t s) {
+template <typename TS, typename T>
+hipError_t load_tiles(const KGrid<T> &g, const BinLayout &L, int64_t n, const void *const src[7],
+                      T *const dst[7], uint32_t *dst_id, int64_t *dst_seg,
+                      unsigned int *dst_cnt, char *w, const LoadSpace &sp, hipStream_t s) {
   const int nc = L.tx * L.ty * L.tz;
   if (nc != 64 && nc != 128) return hipErrorInvalidValue;
-  TileSortJob<double> J;
+  TileSortJob<T> J;
   std::memset(&J, 0, sizeof(J));
   J.L = L;
   J.dst_seg = dst_seg;
@@ -1481,9 +1492,10 @@ inline hipError_t load_tiles(const KGrid<double> &g, const BinLayout &L, int64_t
   const bool many = L.ntiles > kLdsTiles;
   const int64_t per = n / (256 * 2048);
   b.per = many || per > 16 ? 16 : per < 1 ? 1 : (int)per;
-  Arrays7<double> as, ad;
+  Arrays7<TS> as;
+  Arrays7<T> ad;
   for (int a = 0; a < 7; ++a) {
-    as.p[a] = (double *)src[a];
+    as.p[a] = (TS *)src[a];
     ad.p[a] = dst[a];
   }
   hipLaunchKernelGGL(k_zero_u32, dim3(nblocks((long)sp.zeroed)), dim3(256), 0, s, J.count,
@@ -1494,17 +1506,17 @@ inline hipError_t load_tiles(const KGrid<double> &g, const BinLayout &L, int64_t
     const int nt = many ? 1024 : 256;
     const dim3 grid((unsigned)((n + nt * b.per - 1) / (nt * b.per)));
     if (many)
-      hipLaunchKernelGGL((k_load_count<1024, kLoadManyTiles>), grid, dim3(1024), 0, s, g,
+      hipLaunchKernelGGL((k_load_count<TS, T, 1024, kLoadManyTiles>), grid, dim3(1024), 0, s, g,
                          L, b, as.p[0], as.p[1], as.p[2]);
     else if (L.ntiles <= kLdsTiles && L.ntiles <= 8 * 256 * b.per)
-      hipLaunchKernelGGL((k_load_count<256, kLdsTiles>), grid, dim3(256), 0, s, g, L, b,
+      hipLaunchKernelGGL((k_load_count<TS, T, 256, kLdsTiles>), grid, dim3(256), 0, s, g, L, b,
                          as.p[0], as.p[1], as.p[2]);
     else
-      hipLaunchKernelGGL((k_load_count<256, 0>), grid, dim3(256), 0, s, g, L, b, as.p[0],
+      hipLaunchKernelGGL((k_load_count<TS, T, 256, 0>), grid, dim3(256), 0, s, g, L, b, as.p[0],
                          as.p[1], as.p[2]);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k_tile_bounds<double>, dim3(1), dim3(kScanThreads), 0, s, J);
+  hipLaunchKernelGGL(k_tile_bounds<T>, dim3(1), dim3(kScanThreads), 0, s, J);
   if ((e = hipGetLastError()) != hipSuccess || n == 0) return e;
   // places by workgroup or by wave, as the deposit through tiles takes them
   auto blocks = [n](int per) { return dim3((unsigned)((n + 256 * per - 1) / (256 * per))); };
@@ -1521,10 +1533,10 @@ inline hipError_t load_tiles(const KGrid<double> &g, const BinLayout &L, int64_t
   const dim3 threads(kLoadThreads), grid(b.tile_blocks + sp.pieces);
   if (nc == 64) {
     if (sp.pieces) hipLaunchKernelGGL((k_load_pieces<64>), dim3(sp.pieces), threads, 0, s, L, b);
-    hipLaunchKernelGGL((k_load_tile<64>), grid, threads, 0, s, L, b, as, ad, dst_id);
+    hipLaunchKernelGGL((k_load_tile<TS, T, 64>), grid, threads, 0, s, L, b, as, ad, dst_id);
   } else {
     if (sp.pieces) hipLaunchKernelGGL((k_load_pieces<128>), dim3(sp.pieces), threads, 0, s, L, b);
-    hipLaunchKernelGGL((k_load_tile<128>), grid, threads, 0, s, L, b, as, ad, dst_id);
+    hipLaunchKernelGGL((k_load_tile<TS, T, 128>), grid, threads, 0, s, L, b, as, ad, dst_id);
   }
   return hipGetLastError();
 }
@@ -1549,14 +1561,16 @@ hipError_t bin_sort(const KGrid<T> &g, const BinLayout &L, int64_t n,
   const size_t a_c = align_up(sizeof(uint32_t) * (size_t)ncell);
   const int shift = L.rank_bits + L.cell_bits;
   const int key_bits = L.tile_bits + shift;
-  if constexpr (sizeof(T) == 8)
-    if (!binned && load_through_tiles(n, L.ntiles)) {
-      const LoadSpace sp = load_space(L, n);
-      if (needed) *needed = sp.total;
-      if (!workspace) return hipSuccess;
-      if (workspace_bytes < sp.total) return hipErrorInvalidValue;
-      return load_tiles(g, L, n, src, dst, dst_id, dst_seg, dst_cnt, (char *)workspace, sp, s);
-    }
+  if (!binned && load_through_tiles(L, n, sizeof(T) == 4)) {
+    const LoadSpace sp = load_space(L, n);
+    if (needed) *needed = sp.total;
+    if (!workspace) return hipSuccess;
+    if (workspace_bytes < sp.total) return hipErrorInvalidValue;
+    return widened ? load_tiles<double, T>(g, L, n, src, dst, dst_id, dst_seg, dst_cnt,
+                                           (char *)workspace, sp, s)
+                   : load_tiles<T, T>(g, L, n, src, dst, dst_id, dst_seg, dst_cnt,
+                                      (char *)workspace, sp, s);
+  }
   size_t sort_bytes = 0, scan_bytes = 0;
   hipError_t e = rocprim::radix_sort_pairs(
       nullptr, sort_bytes, (uint32_t *)nullptr, (uint32_t *)nullptr,

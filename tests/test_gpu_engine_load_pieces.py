@@ -1,4 +1,4 @@
-"""Loads of FP64 engines with tiles of more particles than one workgroup holds
+"""Loads of engines with tiles of more particles than one workgroup holds
 (8192), which are taken in pieces (GPU): every particle comes back whole, and
 every slot of the storage holds one of the cell that the order by rank and cell
 gives it (which one of a cell is open).  No arithmetic, no tolerance.
@@ -25,20 +25,22 @@ def _modes():
 @pytest.mark.parametrize("counts", [
     [8193, 3], [16384, 0, 8192], [5, 16385, 8193, 0, 9000], [100003, 1],
 ])
-def test_pieces(counts, spread, tile, order):
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_pieces(counts, spread, tile, order, prec):
     r = np.random.default_rng(sum(counts))
     nx = 3 * tile[0] * len(counts)
     t = np.repeat(np.arange(len(counts)), counts)
     n = len(t)
     cit = [r.integers(0, m, n) if spread == "tile" else np.full(n, m - 1) for m in tile]
-    p = {k: (c + (3 * t * tile[0] if k == "x" else 0) + r.uniform(0.1, 0.9, n)) * 0.5
+    # positions and charges that FP32 engines hold exactly
+    p = {k: (c + (3 * t * tile[0] if k == "x" else 0) + r.integers(1, 256, n) / 256.0) * 0.5
          for k, c in zip("xyz", cit)}
     by = r.permutation(n)
     t, cit, p = t[by], [c[by] for c in cit], {k: v[by] for k, v in p.items()}
     for k in "uvw":
-        p[k] = r.normal(0, 1, n)
+        p[k] = r.integers(-1000, 1000, n) / 256.0
     p["q"] = np.arange(n) + 1.0
-    grd = S.Grid(nx, tile[1], tile[2], 0.5 * nx, 0.5 * tile[1], 0.5 * tile[2], "f64")
+    grd = S.Grid(nx, tile[1], tile[2], 0.5 * nx, 0.5 * tile[1], 0.5 * tile[2], prec)
     part = S.Particles(p, 1.0, "f64")
     eng = S.Engine(grd, 1, tile=tile,
                    order=S.SPIC_ORDER_ENGINE if order == "engine" else S.SPIC_ORDER_LOAD)
